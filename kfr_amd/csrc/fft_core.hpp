@@ -256,7 +256,8 @@ enum twiddle_mode : int
     tw_linear = 0, // a = (i*mult + add) mod M
     tw_radix  = 1, // radix-pass table: i = k*(R-1) + (r-1), a = r*k; M = Ns*R
     tw_square = 2, // a = i^2 mod M (Bluestein chirp, M = 2N)
-    tw_radix_full = 3 // radix-pass table with r = 0 included: i = k*R + r, a = r*k; M = Ns*R
+    tw_radix_full = 3, // radix-pass table with r = 0 included: i = k*R + r, a = r*k; M = Ns*R
+    tw_powers = 4 // power-of-two pass table: i = b*Ns + k, a = k << b (b < log2 R); M = Ns*R
 };
 
 template <typename T>
@@ -267,7 +268,13 @@ __global__ void k_twiddles(cx<T>* out, long long count, long long M, long long m
     if (i >= count)
         return;
     unsigned long long a;
-    if (mode == tw_radix_full)
+    if (mode == tw_powers)
+    {
+        const long long ns = M / R;
+        const long long b  = i / ns;
+        a                  = (unsigned long long)(((i - b * ns) << b) % M);
+    }
+    else if (mode == tw_radix_full)
     {
         const long long k = i / R;
         const long long r = i - k * R;

@@ -70,13 +70,14 @@ __host__ __device__ constexpr int pass_lns(int L, int le, int p) // log2 of the 
         s += pass_lr(L, le, q);
     return s;
 }
-// pass p's table holds W_{Ns*R}^(r*k) at k*R + r (k < Ns, r < R); passes with Ns = 1 have none
+// pass p's table holds W_{Ns*R}^(k*2^b) at b*Ns + k (k < Ns, 2^b < R), so that consecutive lanes
+// (consecutive k) read consecutive values; passes with Ns = 1 have none
 __host__ __device__ constexpr int pass_twoff(int L, int le, int p)
 {
     int o = 0;
     for (int q = 0; q < p; ++q)
         if (pass_lns(L, le, q) > 0)
-            o += 1 << (pass_lns(L, le, q) + pass_lr(L, le, q));
+            o += pass_lr(L, le, q) << pass_lns(L, le, q);
     return o;
 }
 
@@ -179,28 +180,6 @@ __device__ __forceinline__ int laddr(int tb, int i)
 {
     const int x = (ROLE == role_col || ROLE == role_pass) ? i * W + tb : tb * LD + i;
     return x + (x >> 4);
-}
-
-template <typename T, int R>
-__device__ __forceinline__ void load_table(const cx<T>* p, cx<T> (&w)[R])
-{
-    if constexpr (sizeof(T) == 4 && R >= 2)
-    {
-        const float4* q = reinterpret_cast<const float4*>(p);
-#pragma unroll
-        for (int i = 0; i < R / 2; ++i)
-        {
-            const float4 f = q[i];
-            w[2 * i]       = { f.x, f.y };
-            w[2 * i + 1]   = { f.z, f.w };
-        }
-    }
-    else
-    {
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-            w[i] = p[i];
-    }
 }
 
 template <typename T>
@@ -462,26 +441,18 @@ __device__ __forceinline__ void run_pass(regs<T, L, ROLE, PREC>& v, cx<T>* lds, 
                                ? mirror_lane<MIRRORL, TP>(t) + m * TP
                                : t + m * TP;
             const int kt = j & (NS - 1);
+            // W^(kt*r) from the table's values at r = 2^b, one complex product per value: fewer loads
+            // than all R - 1 (measured faster everywhere once the one-workgroup and row kernels are
+            // compiled for the waves their LDS allows)
+            const cx<T>* col = tw + S::twoff(P) + kt;
             cx<T> w[R];
-            if constexpr (R >= 8)
-            {
-                // W^(kt*r) from the row's entries at r = 2^b, one complex product per value: fewer
-                // loads than the whole row (measured faster everywhere once the one-workgroup and row
-                // kernels are compiled for the waves their LDS allows: the f32 2^14 and 2^15
-                // one-workgroup kernels and the f64 2^10 row kernel had taken a wave per SIMD more
-                // registers and kept whole-row loads, 5-14% slower)
-                const cx<T>* row = tw + S::twoff(P) + kt * R;
-                w[0]             = { T(1), T(0) };
 #pragma unroll
-                for (int b = 0; (1 << b) < R; ++b)
-                    w[1 << b] = row[1 << b];
+            for (int b = 0; (1 << b) < R; ++b)
+                w[1 << b] = col[b * NS];
 #pragma unroll
-                for (int r = 3; r < R; ++r)
-                    if ((r & (r - 1)) != 0)
-                        w[r] = cmul(w[r - (1 << (ilog2c(r + 1) - 1))], w[1 << (ilog2c(r + 1) - 1)]);
-            }
-            else
-                load_table<T, R>(tw + S::twoff(P) + kt * R, w);
+            for (int r = 3; r < R; ++r)
+                if ((r & (r - 1)) != 0)
+                    w[r] = cmul(w[r - (1 << (ilog2c(r + 1) - 1))], w[1 << (ilog2c(r + 1) - 1)]);
 #pragma unroll
             for (int r = 1; r < R; ++r)
                 v[m + r * M] = ctw<INV>(v[m + r * M], w[r]);
@@ -1046,7 +1017,7 @@ void gen_pass_tables(int L, cx<T>* tw, hipStream_t s)
         const long long ns = 1ll << pass_lns(L, le, p);
         const int r        = 1 << pass_lr(L, le, p);
         if (ns > 1)
-            gen_twiddles(tw + pass_twoff(L, le, p), ns * r, ns * r, 0, 0, tw_radix_full, r, s);
+            gen_twiddles(tw + pass_twoff(L, le, p), ns * pass_lr(L, le, p), ns * r, 0, 0, tw_powers, r, s);
     }
 }
 
