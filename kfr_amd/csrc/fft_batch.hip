@@ -59,6 +59,75 @@ __global__ void k_queue_reset(unsigned* counter)
         counter[0] = 0u;
 }
 
+// the passes of one item whose transform c runs in LDS: pass 0 straight from `in`, the last one straight
+// to `out`, inverse transforms as conj(DFT(conj x)); Bluestein lengths premultiply by the chirp and pad
+template <typename T, bool PAD>
+__device__ __forceinline__ void run_item(const len_desc& D, const cx<T>* __restrict__ tab, const fft_ctx<T, PAD>& c,
+                                         const cx<T>* in, cx<T>* out, bool inv)
+{
+    const lds_geom& G = D.G;
+    const cx<T>* tw   = tab + D.tw;
+    if (!D.bluestein && G.np >= 2 && G.pass[0].kind == pass_radix && G.pass[G.np - 1].kind == pass_radix)
+    {
+        first_pass<T, false, true>(G, tw, c, from_global<T, true>{ in, 1, c.valid, inv });
+        fft_passes<T, false, true>(G, tw, c, 1, G.np - 1);
+        // nontemporal: the outputs are not read again by this launch (measured 4% faster)
+        last_pass<T, false, true>(G, tw, c, to_global<T, true, true>{ out, 1, c.valid, inv });
+        return;
+    }
+    const int n     = D.n;
+    const cx<T>* ch = tab + D.chirp;
+    for (int i0 = c.t; i0 < G.n; i0 += stage_values<T> * G.tpt)
+    {
+        cx<T> v[stage_values<T>];
+#pragma unroll
+        for (int k = 0; k < stage_values<T>; ++k)
+        {
+            const int i = i0 + k * G.tpt;
+            v[k]        = { T(0), T(0) };
+            if (i < n)
+                v[k] = in[i];
+        }
+#pragma unroll
+        for (int k = 0; k < stage_values<T>; ++k)
+        {
+            const int i = i0 + k * G.tpt;
+            if (i < G.n)
+            {
+                cx<T> x = v[k];
+                if (i < n)
+                {
+                    if (inv)
+                        x = cconj(x);
+                    if (D.bluestein)
+                        x = cmul(x, ch[i]);
+                }
+                c.at(i) = x;
+            }
+        }
+    }
+    __syncthreads();
+    fft_passes<T, false, true>(G, tw, c);
+    if (D.bluestein)
+    {
+        // IFFT_M(A conj(H)) = conj(FFT_M(conj(A) H)); H carries the 1/M
+        const cx<T>* H = tab + D.H;
+        for (int i = c.t; i < G.n; i += G.tpt)
+            c.at(i) = cmul(cconj(c.at(i)), H[i]);
+        __syncthreads();
+        fft_passes<T, false, true>(G, tw, c);
+    }
+    for (int i = c.t; i < n; i += G.tpt)
+    {
+        cx<T> v = c.at(i);
+        if (D.bluestein)
+            v = cmul(cconj(v), ch[i]);
+        v = inv ? cconj(v) : v;
+        using V2 = T __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store(V2{ v.re, v.im }, reinterpret_cast<V2*>(out + i));
+    }
+}
+
 // at most 128 VGPRs (4 waves per SIMD), so two workgroups share a CU: measured faster than the
 // unconstrained build (185 VGPRs, one workgroup per CU) despite a little spilling
 template <typename T>
@@ -88,91 +157,27 @@ __global__ void __launch_bounds__(block) __attribute__((amdgpu_waves_per_eu(4)))
         const len_desc& D = lens[I.len];
         const lds_geom& G = D.G;
         const int tid     = threadIdx.x;
-        const int tb      = tid / G.tpt;
+        const int tb      = (int)fdiv((uint32_t)tid, G.tpt_div);
         const bool active = tb < I.count;
-        fft_ctx<T> c;
-        c.lds   = lds;
-        c.tb    = tb;
-        c.base  = active ? tb * G.ld : 0;
-        c.ls    = 1;
-        c.ps    = G.padshift;
-        c.t     = active ? tid - tb * G.tpt : G.n; // idle threads skip every element loop
-        c.valid = active;
-        c.g     = 0;
         const int mbr       = active ? members[I.first + tb] : 0;
         const long long off = active ? offs[mbr >> 1] : 0;
-        const bool inv      = (mbr & 1) != 0;
-        const int n         = D.n;
-        const cx<T>* ch     = tab + D.chirp;
-
-        // load; the inverse runs as conj(DFT(conj x)); Bluestein premultiplies by the chirp and pads.
-        // A thread holds at most EM values of one transform (every pass gives it at most
-        // ceil(pm/R)*R <= pm + 6 of them): the loads of all of them are issued before the first is
-        // used, so their latencies overlap instead of adding up; any value beyond EM (none for the
-        // schedules the planner makes) takes the plain loop.
-        constexpr int EM = pmax_of<T> + 7;
+        auto run            = [&](auto pad)
         {
-            cx<T> v[EM];
-#pragma unroll
-            for (int k = 0; k < EM; ++k)
-            {
-                const int i = c.t + k * G.tpt;
-                v[k]        = { T(0), T(0) };
-                if (i < n)
-                    v[k] = in[off + i];
-            }
-#pragma unroll
-            for (int k = 0; k < EM; ++k)
-            {
-                const int i = c.t + k * G.tpt;
-                if (i < G.n)
-                {
-                    cx<T> x = v[k];
-                    if (i < n)
-                    {
-                        if (inv)
-                            x = cconj(x);
-                        if (D.bluestein)
-                            x = cmul(x, ch[i]);
-                    }
-                    c.at(i) = x;
-                }
-            }
-        }
-        for (int i = c.t + EM * G.tpt; i < G.n; i += G.tpt)
-        {
-            cx<T> v = { T(0), T(0) };
-            if (i < n)
-            {
-                v = in[off + i];
-                if (inv)
-                    v = cconj(v);
-                if (D.bluestein)
-                    v = cmul(v, ch[i]);
-            }
-            c.at(i) = v;
-        }
-        __syncthreads();
-        fft_passes<T, false, true, true>(G, tab + D.tw, c);
-        if (D.bluestein)
-        {
-            // IFFT_M(A conj(H)) = conj(FFT_M(conj(A) H)); H carries the 1/M
-            const cx<T>* H = tab + D.H;
-            for (int i = c.t; i < G.n; i += G.tpt)
-                c.at(i) = cmul(cconj(c.at(i)), H[i]);
-            __syncthreads();
-            fft_passes<T, false, true, true>(G, tab + D.tw, c);
-        }
-        for (int i = c.t; i < n; i += G.tpt)
-        {
-            cx<T> v = c.at(i);
-            if (D.bluestein)
-                v = cmul(cconj(v), ch[i]);
-            v = inv ? cconj(v) : v;
-            // nontemporal: the outputs are not read again by this launch (measured 4% faster)
-            using V2 = T __attribute__((ext_vector_type(2)));
-            __builtin_nontemporal_store(V2{ v.re, v.im }, reinterpret_cast<V2*>(out + off + i));
-        }
+            fft_ctx<T, decltype(pad)::value> c;
+            c.lds   = lds;
+            c.tb    = tb;
+            c.base  = active ? tb * G.ld : 0;
+            c.ls    = 1;
+            c.ps    = G.padshift;
+            c.t     = active ? tid - tb * G.tpt : G.n; // idle threads skip every element loop
+            c.valid = active;
+            c.g     = 0;
+            run_item<T, decltype(pad)::value>(D, tab, c, in + off, out + off, (mbr & 1) != 0);
+        };
+        if (G.padshift >= 30)
+            run(std::false_type{});
+        else
+            run(std::true_type{});
         if (threadIdx.x == 0)
             s_item = (int)next;
         __syncthreads(); // LDS is rewritten by the next item, whose index is now in s_item
@@ -189,13 +194,15 @@ struct host_len
     stockham S;                            // schedule of the chosen pass order
     std::vector<std::vector<int>> orders;  // candidate pass orders (the planner's first)
     int order    = 0;                      // chosen pass order
-    int padshift = 4;                      // chosen LDS padding: one slot per 2^padshift values
+    int padshift = 4;                      // chosen LDS padding: one slot per 2^padshift values (30: none)
     int tpb_max  = 1;
     int tpb      = 1;
     long long tw = 0, chirp = 0, H = 0;
 };
 
-// LDS paddings tried: one slot per 16 or per 32 values, or none (the tile is sized for one per 16)
+// LDS paddings: one slot per 16 or per 32 values, or none (the tile is sized for one per 16). Untuned
+// lengths with odd factors run without (an odd first radix spreads its writes), powers of two with one
+// per 16
 constexpr int padshifts[] = { 4, 5, 30 };
 
 // Pass orders tried for one length: the planner's (powers of two, largest first, then 7, 5, 3 and the
@@ -223,7 +230,7 @@ template <typename T>
 void set_order(host_len<T>& h, int k)
 {
     h.order = k;
-    if (!stockham_from_radices((long long)h.m, h.orders[k], h.S, pmax_of<T>, true))
+    if (!stockham_from_radices((long long)h.m, h.orders[k], h.S, pmax_of<T>))
         throw std::logic_error("batch: pass order does not factor its length");
 }
 
@@ -503,10 +510,13 @@ gpu_batch<T>::gpu_batch(size_t count, const size_t* sizes, const int* inverse, b
         h.n  = n;
         h.bs = describe_dft(dt, n, false).arblen;
         h.m  = h.bs ? next_pow2(2 * n - 1) : n;
-        if (!make_stockham((long long)h.m, h.S, pmax_of<T>, true) || h.S.tpt > block || lds_of<T>(h.m, 1) > lds_cap)
+        if (workgroup_threads((long long)h.m, pmax_of<T>, true) > block || !make_stockham((long long)h.m, h.S, pmax_of<T>) ||
+            h.S.tpt > block || lds_of<T>(h.m, 1) > lds_cap)
             throw std::invalid_argument("transform length " + std::to_string(n) +
                                         " does not fit one workgroup of the batch kernel");
         h.orders = radix_orders(h.S.radix);
+        if (is_mixed(h.S))
+            h.padshift = 30; // an odd first radix: its LDS writes spread over the banks by themselves
         h.tpb_max = std::max(1, block / h.S.tpt);
         while (h.tpb_max > 1 && lds_of<T>(h.m, h.tpb_max) > lds_cap)
             --h.tpb_max;

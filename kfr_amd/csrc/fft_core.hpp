@@ -329,11 +329,8 @@ struct stockham
     int tpt            = 0;
 };
 
-inline bool lds_radix(int r) { return r == 2 || r == 3 || r == 4 || r == 5 || r == 7 || r == 8 || r == 16; }
-
 // Pass geometry of an explicit radix list (product n): strides, twiddle offsets, threads per transform
-// (wide: the ceil(pm/R) butterflies per thread of radix_pass<..., WIDE>)
-inline bool stockham_from_radices(long long nn, const std::vector<int>& radices, stockham& S, int pm, bool wide = false)
+inline bool stockham_from_radices(long long nn, const std::vector<int>& radices, stockham& S, int pm)
 {
     S = stockham{};
     if (nn < 1 || nn > (1 << 28) || (int)radices.size() > max_passes)
@@ -358,7 +355,7 @@ inline bool stockham_from_radices(long long nn, const std::vector<int>& radices,
         {
             if (ns > 1)
                 off += ns * (r - 1);
-            const int M  = wide ? (pm + r - 1) / r : std::max(1, pm / r); // bflies_of
+            const int M  = bflies(r, pm);
             const int nb = n / r;
             tpt          = std::max(tpt, (nb + M - 1) / M);
         }
@@ -389,12 +386,13 @@ inline bool odd_factors(long long& m, std::vector<int>& odd)
     return m == 1;
 }
 
-// Factor n into GPU passes (wide: the ceil(pm/R) butterflies per thread of radix_pass<..., WIDE>).
-// Power-of-2 part: the largest butterfly that fits a thread's pm values (16 for f32, 8 for f64) first,
-// remainder 8/4/2; then 7, 5, 3; any other prime factor up to 127 becomes a direct DFT pass, placed last.
-inline bool make_stockham(long long nn, stockham& S, int pm, bool wide = false)
+// Factors of n: its power-of-two part in the largest butterflies that fit a thread's pm values (16 for
+// f32, 8 for f64) and the remainder 8/4/2; then 7, 5, 3; then any other prime factor up to 127 (a direct
+// DFT pass). False if another prime remains. This is the schedule of the power-of-two lengths, and its
+// thread count is the capacity rule of one workgroup for every length (workgroup_threads).
+inline bool factor_radices(long long nn, std::vector<int>& radix, int pm)
 {
-    S = stockham{};
+    radix.clear();
     if (nn < 1 || nn > (1 << 28))
         return false;
     long long m = nn;
@@ -404,7 +402,6 @@ inline bool make_stockham(long long nn, stockham& S, int pm, bool wide = false)
         m /= 2;
         ++a;
     }
-    std::vector<int> radix;
     const int rbits = pm >= 16 ? 4 : 3;
     while (a >= rbits)
     {
@@ -413,9 +410,109 @@ inline bool make_stockham(long long nn, stockham& S, int pm, bool wide = false)
     }
     if (a > 0)
         radix.push_back(1 << a);
-    if (!odd_factors(m, radix))
+    return odd_factors(m, radix);
+}
+
+// Threads that one transform counts for in the capacity rule (which lengths one workgroup takes): at
+// most pm values per thread in every pass of factor_radices, or with `wide` one butterfly more. The
+// planned schedule of a length within the rule never needs more threads than the workgroup limit.
+inline int workgroup_threads(long long nn, int pm, bool wide)
+{
+    std::vector<int> radix;
+    if (!factor_radices(nn, radix, pm))
+        return INT_MAX;
+    long long t = 1;
+    for (int r : radix)
+    {
+        const bool g      = !(r <= 5 || r == 7 || r == 8 || r == 16);
+        const long long M = g ? 1 : wide ? (pm + r - 1) / r : std::max(1, pm / r);
+        t                 = std::max(t, g ? (nn + pm - 1) / pm : (nn / r + M - 1) / M);
+    }
+    return (int)std::min<long long>(t, INT_MAX);
+}
+
+// Schedule of a length with odd factors: the product of butterfly radices (2..10, 12, 14, 15, 16) with
+// the least modelled work per point. A pass costs its butterfly's arithmetic, its twiddles and one
+// exchange through LDS, times the lanes that its butterflies leave idle at the schedule's thread count,
+// so few passes of large radices with equal thread counts win: 960 points run as 15 x 16 x 4 on 64
+// threads. The largest odd radix goes first (its strided LDS writes meet no bank twice), direct passes
+// of larger primes last.
+inline bool plan_mixed(long long nn, stockham& S, int pm, int max_threads)
+{
+    std::vector<int> base;
+    if (!factor_radices(nn, base, pm))
         return false;
-    return stockham_from_radices(nn, radix, S, pm, wide);
+    std::vector<int> direct;
+    long long m = nn;
+    for (int r : base)
+        if (r > 7 && r % 2 != 0)
+        {
+            direct.push_back(r);
+            m /= r;
+        }
+    struct choice
+    {
+        int r;
+        double cost; // vector instructions per point of the butterfly
+    };
+    static constexpr choice menu[] = { { 16, 10.5 }, { 15, 13 }, { 14, 16 }, { 12, 9 }, { 10, 10 }, { 9, 11 }, { 8, 7 },
+                                       { 7, 14 },    { 6, 7 },   { 5, 8 },   { 4, 4 },  { 3, 5 },   { 2, 2 } };
+    constexpr int choices = (int)(sizeof(menu) / sizeof(menu[0]));
+    std::vector<int> cur, best;
+    double best_cost = 1e300;
+    auto search = [&](auto&& self, long long rest, int from) -> void
+    {
+        if (rest == 1)
+        {
+            std::vector<int> all = cur;
+            all.insert(all.end(), direct.begin(), direct.end());
+            stockham t;
+            if (all.empty() || !stockham_from_radices(nn, all, t, pm) || t.tpt > max_threads)
+                return;
+            double cost = 0;
+            for (int r : cur)
+                for (const choice& c : menu)
+                    if (c.r == r)
+                        cost += (c.cost + 4 + 13) * ((double)t.tpt * bflies(r, pm) * r / (double)nn);
+            if (cost < best_cost)
+            {
+                best_cost = cost;
+                best      = cur;
+            }
+            return;
+        }
+        if ((int)cur.size() + (int)direct.size() >= max_passes)
+            return;
+        for (int i = from; i < choices; ++i)
+        {
+            const int r = menu[i].r;
+            // f64 butterflies above radix 10 hold more values than the kernels have registers for
+            if (rest % r != 0 || (pm < 16 && r > 10))
+                continue;
+            cur.push_back(r);
+            self(self, rest / r, i);
+            cur.pop_back();
+        }
+    };
+    search(search, m, 0);
+    if (best_cost == 1e300)
+        return false;
+    auto odd = std::find_if(best.begin(), best.end(), [](int r) { return r % 2 != 0; }); // the largest
+    if (odd != best.end())
+        std::rotate(best.begin(), odd, odd + 1);
+    best.insert(best.end(), direct.begin(), direct.end());
+    return stockham_from_radices(nn, best, S, pm);
+}
+
+// Factor n into GPU passes: the fixed schedule for powers of two, the planned one for the others
+inline bool make_stockham(long long nn, stockham& S, int pm)
+{
+    std::vector<int> radix;
+    if (!factor_radices(nn, radix, pm))
+        return false;
+    if ((nn & (nn - 1)) == 0 || !plan_mixed(nn, S, pm, max_block_mixed))
+        return stockham_from_radices(nn, radix, S, pm);
+    return true;
 }
 
 // A finer schedule of the same transform for progressive execution, about `want` passes: every odd
@@ -467,6 +564,7 @@ inline lds_geom make_geom(const stockham& S, int tpb, int mapping, int ls, int l
     G.n       = S.n;
     G.np      = (int)S.radix.size();
     G.tpt     = S.tpt;
+    G.tpt_div = make_fastdiv((uint32_t)S.tpt);
     G.tpb     = tpb;
     G.mapping = mapping;
     G.ls      = ls;
@@ -482,6 +580,7 @@ inline lds_geom make_geom(const stockham& S, int tpb, int mapping, int ls, int l
     {
         G.pass[p].radix  = S.radix[p];
         G.pass[p].ns     = S.ns[p];
+        G.pass[p].nb     = S.n / S.radix[p];
         G.pass[p].tw     = (int)S.tw_off[p];
         G.pass[p].kind   = S.kind[p];
         G.pass[p].ns_div = make_fastdiv((uint32_t)S.ns[p]);
@@ -514,202 +613,220 @@ struct fourstep_args
     long long n = 1;
 };
 
-// Load and store phases. Each thread stages its (at most pmax) elements in registers, so that all of
-// its global loads (or stores) are in flight together; the host guarantees tpb*n <= pmax*blockDim.
+// Load and store phases. A thread stages up to stage_values elements at a time in registers, so that
+// all of their global loads (or stores) are in flight together. In the power-of-two builds (PAD) one
+// round holds them all.
+template <typename T>
+inline constexpr int stage_values = pmax_of<T>;
 
 template <typename T>
-__device__ __forceinline__ bool plain_contiguous(const xload<T>& ld, long long n)
+__host__ __device__ __forceinline__ bool plain(const xload<T>& ld)
 {
-    return ld.mode == ld_plain && ld.pdist == n && ld.mtab == nullptr && ld.lim == LLONG_MAX;
+    return ld.mode == ld_plain && ld.mtab == nullptr && ld.lim == LLONG_MAX;
 }
 template <typename T>
-__device__ __forceinline__ bool plain_contiguous(const xstore<T>& st, long long n)
+__host__ __device__ __forceinline__ bool plain(const xstore<T>& st)
 {
-    return st.mode == st_plain && st.pdist == n && st.mtab == nullptr && st.lim == LLONG_MAX;
+    return st.mode == st_plain && st.mtab == nullptr && st.lim == LLONG_MAX;
 }
 
 // the block's transforms, element index fastest (e = tb*n + i); LDS layout lds[e] (ld = n, ls = 1)
-template <typename T>
+template <bool PAD, typename T>
 __device__ __forceinline__ void block_load(const lds_geom& G, cx<T>* lds, long long first, long long batch,
                                            const xload<T>& ld, const fastdiv& ndiv)
 {
     const int total     = G.tpb * G.n;
     const int bs        = blockDim.x;
-    const int tid       = threadIdx.x;
     const long long rem = (batch - first) * (long long)G.n;
     const int lim       = rem < total ? (int)rem : total;
-    cx<T> v[pmax_of<T>];
-    if (plain_contiguous(ld, G.n))
+    int e0 = threadIdx.x;
+    do
     {
-        const cx<T>* src = static_cast<const cx<T>*>(ld.p) + (first + ld.b0) * (long long)G.n;
-#pragma unroll
-        for (int k = 0; k < pmax_of<T>; ++k)
+        cx<T> v[stage_values<T>];
+        if (plain(ld) && ld.pdist == G.n)
         {
-            const int e = tid + k * bs;
-            v[k]        = e < lim ? src[e] : cx<T>{ T(0), T(0) };
-        }
-    }
-    else
-    {
+            const cx<T>* src = static_cast<const cx<T>*>(ld.p) + (first + ld.b0) * (long long)G.n;
 #pragma unroll
-        for (int k = 0; k < pmax_of<T>; ++k)
-        {
-            const int e = tid + k * bs;
-            v[k]        = { T(0), T(0) };
-            if (e < lim)
+            for (int k = 0; k < stage_values<T>; ++k)
             {
-                const int tb = (int)fdiv((uint32_t)e, ndiv);
-                v[k]         = ld.load(first + tb, e - tb * G.n);
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < pmax_of<T>; ++k)
-    {
-        const int e = tid + k * bs;
-        if (e < total)
-            lds[lds_pad(e, G.padshift)] = v[k];
-    }
-}
-template <typename T>
-__device__ __forceinline__ void block_store(const lds_geom& G, const cx<T>* lds, long long first, long long batch,
-                                            const xstore<T>& st, const fastdiv& ndiv)
-{
-    const int total     = G.tpb * G.n;
-    const int bs        = blockDim.x;
-    const int tid       = threadIdx.x;
-    const long long rem = (batch - first) * (long long)G.n;
-    const int lim       = rem < total ? (int)rem : total;
-    cx<T> v[pmax_of<T>];
-#pragma unroll
-    for (int k = 0; k < pmax_of<T>; ++k)
-    {
-        const int e = tid + k * bs;
-        if (e < total)
-            v[k] = lds[lds_pad(e, G.padshift)];
-    }
-    if (plain_contiguous(st, G.n))
-    {
-        cx<T>* dst = static_cast<cx<T>*>(st.p) + (first + st.b0) * (long long)G.n;
-#pragma unroll
-        for (int k = 0; k < pmax_of<T>; ++k)
-        {
-            const int e = tid + k * bs;
-            if (e < lim)
-                dst[e] = v[k];
-        }
-    }
-    else
-    {
-#pragma unroll
-        for (int k = 0; k < pmax_of<T>; ++k)
-        {
-            const int e = tid + k * bs;
-            if (e < lim)
-            {
-                const int tb = (int)fdiv((uint32_t)e, ndiv);
-                st.store(first + tb, e - tb * G.n, v[k]);
-            }
-        }
-    }
-}
-
-template <typename T, bool INV, int ROLE, bool MIXED>
-__global__ void __launch_bounds__(max_block_of(MIXED)) k_fft(lds_geom G, const cx<T>* __restrict__ tw, long long batch,
-                                              xload<T> ld, xstore<T> st, fourstep_args<T> fs)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T>* lds            = reinterpret_cast<cx<T>*>(smem_raw);
-    const long long first = (long long)blockIdx.x * G.tpb;
-    const fft_ctx<T> c    = make_ctx<T>(G, lds, first, batch);
-    cx<T> v[pmax_of<T>];
-    if constexpr (ROLE == role_direct)
-    {
-        block_load(G, lds, first, batch, ld, fs.ndiv);
-    }
-    else if constexpr (ROLE == role_col)
-    {
-        // column col of batch item bl: elements col + n1*i; consecutive lanes take consecutive columns
-        const uint32_t bl = fdiv((uint32_t)c.g, fs.n1div);
-        const int col     = (int)((uint32_t)c.g - bl * (uint32_t)fs.n1);
-        if (ld.mode == ld_plain && ld.mtab == nullptr && ld.lim == LLONG_MAX)
-        {
-            const cx<T>* src = static_cast<const cx<T>*>(ld.p) + ((long long)bl + ld.b0) * ld.pdist + col;
-#pragma unroll
-            for (int k = 0; k < pmax_of<T>; ++k)
-            {
-                const int i = c.t + k * G.tpt;
-                v[k]        = (i < G.n && c.valid) ? src[(long long)fs.n1 * i] : cx<T>{ T(0), T(0) };
+                const int e = e0 + k * bs;
+                v[k]        = e < lim ? src[e] : cx<T>{ T(0), T(0) };
             }
         }
         else
         {
 #pragma unroll
-            for (int k = 0; k < pmax_of<T>; ++k)
+            for (int k = 0; k < stage_values<T>; ++k)
             {
-                const int i = c.t + k * G.tpt;
-                v[k] = (i < G.n && c.valid) ? ld.load(bl, (long long)col + (long long)fs.n1 * i) : cx<T>{ T(0), T(0) };
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < pmax_of<T>; ++k)
-        {
-            const int i = c.t + k * G.tpt;
-            if (i < G.n)
-                c.at(i) = v[k];
-        }
-    }
-    else
-    {
-        // row g of the intermediate, contiguous
-        const cx<T>* src = fs.scratch + c.g * (long long)G.n;
-#pragma unroll
-        for (int k = 0; k < pmax_of<T>; ++k)
-        {
-            const int i = c.t + k * G.tpt;
-            v[k]        = (i < G.n && c.valid) ? src[i] : cx<T>{ T(0), T(0) };
-        }
-#pragma unroll
-        for (int k = 0; k < pmax_of<T>; ++k)
-        {
-            const int i = c.t + k * G.tpt;
-            if (i < G.n)
-                c.at(i) = v[k];
-        }
-    }
-    __syncthreads();
-    fft_passes<T, INV, MIXED>(G, tw, c);
-    if constexpr (ROLE == role_direct)
-    {
-        block_store(G, lds, first, batch, st, fs.ndiv);
-    }
-    else if constexpr (ROLE == role_col)
-    {
-        if (c.valid)
-        {
-            const uint32_t bl = fdiv((uint32_t)c.g, fs.n1div);
-            const int col     = (int)((uint32_t)c.g - bl * (uint32_t)fs.n1);
-            cx<T>* dst        = fs.scratch + (long long)bl * fs.n + col;
-            const unsigned long long mask = (1ull << fs.lbits) - 1;
-#pragma unroll
-            for (int k = 0; k < pmax_of<T>; ++k)
-            {
-                const int i = c.t + k * G.tpt;
-                if (i < G.n)
-                    v[k] = c.at(i);
-            }
-#pragma unroll
-            for (int k = 0; k < pmax_of<T>; ++k)
-            {
-                const int i = c.t + k * G.tpt;
-                if (i < G.n)
+                const int e = e0 + k * bs;
+                v[k]        = { T(0), T(0) };
+                if (e < lim)
                 {
-                    const unsigned long long m = (unsigned long long)col * (unsigned long long)i; // < n
-                    const cx<T> w              = cmul(fs.ta[m >> fs.lbits], fs.tb[m & mask]);
-                    dst[(long long)fs.n1 * i]  = ctw<INV>(v[k], w);
+                    const int tb = (int)fdiv((uint32_t)e, ndiv);
+                    v[k]         = ld.load(first + tb, e - tb * G.n);
                 }
             }
         }
+#pragma unroll
+        for (int k = 0; k < stage_values<T>; ++k)
+        {
+            const int e = e0 + k * bs;
+            if (e < total)
+                lds[lds_pad<PAD>(e, G.padshift)] = v[k];
+        }
+        e0 += stage_values<T> * bs;
+    } while (!PAD && e0 < total);
+}
+template <bool PAD, typename T>
+__device__ __forceinline__ void block_store(const lds_geom& G, const cx<T>* lds, long long first, long long batch,
+                                            const xstore<T>& st, const fastdiv& ndiv)
+{
+    const int total     = G.tpb * G.n;
+    const int bs        = blockDim.x;
+    const long long rem = (batch - first) * (long long)G.n;
+    const int lim       = rem < total ? (int)rem : total;
+    int e0 = threadIdx.x;
+    do
+    {
+        cx<T> v[stage_values<T>];
+#pragma unroll
+        for (int k = 0; k < stage_values<T>; ++k)
+        {
+            const int e = e0 + k * bs;
+            if (e < total)
+                v[k] = lds[lds_pad<PAD>(e, G.padshift)];
+        }
+        if (plain(st) && st.pdist == G.n)
+        {
+            cx<T>* dst = static_cast<cx<T>*>(st.p) + (first + st.b0) * (long long)G.n;
+#pragma unroll
+            for (int k = 0; k < stage_values<T>; ++k)
+            {
+                const int e = e0 + k * bs;
+                if (e < lim)
+                    dst[e] = v[k];
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (int k = 0; k < stage_values<T>; ++k)
+            {
+                const int e = e0 + k * bs;
+                if (e < lim)
+                {
+                    const int tb = (int)fdiv((uint32_t)e, ndiv);
+                    st.store(first + tb, e - tb * G.n, v[k]);
+                }
+            }
+        }
+        e0 += stage_values<T> * bs;
+    } while (!PAD && e0 < total);
+}
+
+// Waves per SIMD that the mixed-radix kernels are compiled for: f32 in 128 VGPRs without spills (155
+// unbounded, a wave fewer); f64 as many as it comes to
+template <typename T, bool MIXED>
+inline constexpr int mixed_waves = MIXED && sizeof(T) == 4 ? 4 : 1;
+
+// FL: the first pass reads HBM itself (plain loads; row kernels, whose input is the intermediate); FS: the
+// last of two or more passes writes HBM itself (plain stores; column kernels). Mixed-radix builds only:
+// powers of two with plain data have kernels of their own.
+template <typename T, bool INV, int ROLE, bool MIXED, bool FL, bool FS>
+__global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) k_fft(lds_geom G, const cx<T>* __restrict__ tw, long long batch,
+                                              xload<T> ld, xstore<T> st, fourstep_args<T> fs)
+{
+    constexpr bool PAD = !MIXED;
+    constexpr int SV   = stage_values<T>;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    cx<T>* lds               = reinterpret_cast<cx<T>*>(smem_raw);
+    const long long first    = (long long)blockIdx.x * G.tpb;
+    const fft_ctx<T, PAD> c  = make_ctx<PAD, T>(G, lds, first, batch);
+    [[maybe_unused]] uint32_t bl = 0;
+    [[maybe_unused]] int col     = 0;
+    if constexpr (ROLE == role_col)
+    {
+        // column col of batch item bl: elements col + n1*i; consecutive lanes take consecutive columns
+        bl  = c.valid ? fdiv((uint32_t)c.g, fs.n1div) : 0u;
+        col = c.valid ? (int)((uint32_t)c.g - bl * (uint32_t)fs.n1) : 0;
+    }
+    if constexpr (FL)
+    {
+        const cx<T>* src = static_cast<const cx<T>*>(ld.p);
+        from_global<T> in{ nullptr, 1, c.valid };
+        if constexpr (ROLE == role_direct)
+            in.p = src + (c.valid ? c.g + ld.b0 : 0) * ld.pdist;
+        else if constexpr (ROLE == role_col)
+        {
+            in.p      = src + ((long long)bl + ld.b0) * ld.pdist + col;
+            in.stride = fs.n1;
+        }
+        else
+            in.p = fs.scratch + (c.valid ? c.g : 0) * (long long)G.n; // row g of the intermediate, contiguous
+        first_pass<T, INV, MIXED>(G, tw, c, in);
+    }
+    else
+    {
+        if constexpr (ROLE == role_direct)
+            block_load<PAD>(G, lds, first, batch, ld, fs.ndiv);
+        else
+        {
+            for (int i0 = c.t; i0 < G.n; i0 += SV * G.tpt)
+            {
+                cx<T> v[SV];
+#pragma unroll
+                for (int k = 0; k < SV; ++k)
+                {
+                    const int i = i0 + k * G.tpt;
+                    v[k]        = { T(0), T(0) };
+                    if (i < G.n && c.valid)
+                    {
+                        if constexpr (ROLE == role_col)
+                            v[k] = ld.load(bl, (long long)col + (long long)fs.n1 * i);
+                        else
+                            v[k] = fs.scratch[c.g * (long long)G.n + i];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < SV; ++k)
+                {
+                    const int i = i0 + k * G.tpt;
+                    if (i < G.n)
+                        c.at(i) = v[k];
+                }
+            }
+        }
+        __syncthreads();
+    }
+    fft_passes<T, INV, MIXED>(G, tw, c, FL ? 1 : 0, FS ? G.np - 1 : G.np);
+    if constexpr (ROLE == role_direct)
+    {
+        if constexpr (FS)
+            last_pass<T, INV, MIXED>(G, tw, c,
+                                     to_global<T>{ static_cast<cx<T>*>(st.p) + (c.valid ? c.g + st.b0 : 0) * st.pdist, 1,
+                                                   c.valid });
+        else
+            block_store<PAD>(G, lds, first, batch, st, fs.ndiv);
+    }
+    else if constexpr (ROLE == role_col)
+    {
+        to_column<T> out;
+        out.p      = fs.scratch + (long long)bl * fs.n + col;
+        out.stride = fs.n1;
+        out.valid  = c.valid;
+        out.ta     = fs.ta;
+        out.tb     = fs.tb;
+        out.lbits  = fs.lbits;
+        out.col    = (unsigned)col;
+        if constexpr (FS)
+            last_pass<T, INV, MIXED>(G, tw, c, out);
+        else if (c.valid)
+            for (int i = c.t; i < G.n; i += G.tpt)
+            {
+                const cx<T> v = c.at(i);
+                out.p[(long long)fs.n1 * i] =
+                    out.ta ? ctw<INV>(v, out.table((unsigned long long)col * (unsigned)i)) : v;
+            }
     }
     else
     {
@@ -717,38 +834,42 @@ __global__ void __launch_bounds__(max_block_of(MIXED)) k_fft(lds_geom G, const c
         // blockDim = tpt*tpb, so a thread keeps one transform and steps i by tpt.
         const int tid    = threadIdx.x;
         const int tb     = tid % G.tpb;
-        const int i0     = tid / G.tpb;
+        const int t2     = tid / G.tpb;
         const long long g = first + tb;
         if (g < batch)
         {
-            const uint32_t bl = fdiv((uint32_t)g, fs.n2div);
-            const int k2      = (int)((uint32_t)g - bl * (uint32_t)fs.n2);
-#pragma unroll
-            for (int k = 0; k < pmax_of<T>; ++k)
+            const uint32_t b2 = fdiv((uint32_t)g, fs.n2div);
+            const int k2      = (int)((uint32_t)g - b2 * (uint32_t)fs.n2);
+            cx<T>* dst        = static_cast<cx<T>*>(st.p) + ((long long)b2 + st.b0) * st.pdist + k2;
+            for (int i0 = t2; i0 < G.n; i0 += SV * G.tpt)
             {
-                const int i = i0 + k * G.tpt;
-                if (i < G.n)
-                    v[k] = lds[lds_pad(tb * G.ld + i, G.padshift)];
-            }
-            if (st.mode == st_plain && st.mtab == nullptr && st.lim == LLONG_MAX)
-            {
-                cx<T>* dst = static_cast<cx<T>*>(st.p) + ((long long)bl + st.b0) * st.pdist + k2;
+                cx<T> v[SV];
 #pragma unroll
-                for (int k = 0; k < pmax_of<T>; ++k)
+                for (int k = 0; k < SV; ++k)
                 {
                     const int i = i0 + k * G.tpt;
                     if (i < G.n)
-                        dst[(long long)fs.n2 * i] = v[k];
+                        v[k] = c.slot(tb * G.ld + i);
                 }
-            }
-            else
-            {
-#pragma unroll
-                for (int k = 0; k < pmax_of<T>; ++k)
+                if (plain(st))
                 {
-                    const int i = i0 + k * G.tpt;
-                    if (i < G.n)
-                        st.store(bl, (long long)k2 + (long long)fs.n2 * i, v[k]);
+#pragma unroll
+                    for (int k = 0; k < SV; ++k)
+                    {
+                        const int i = i0 + k * G.tpt;
+                        if (i < G.n)
+                            dst[(long long)fs.n2 * i] = v[k];
+                    }
+                }
+                else
+                {
+#pragma unroll
+                    for (int k = 0; k < SV; ++k)
+                    {
+                        const int i = i0 + k * G.tpt;
+                        if (i < G.n)
+                            st.store(b2, (long long)k2 + (long long)fs.n2 * i, v[k]);
+                    }
                 }
             }
         }
@@ -782,14 +903,24 @@ inline void check_pass_radices(const stockham& s, bool mixed_build)
 {
     for (int r : s.radix)
     {
-        const bool ok = r == 2 || r == 4 || r == 8 || (r == 16 && pmax_of<T> >= 16) ||
-                        (mixed_build && (r & (r - 1)) != 0 && r > 2);
+        const bool pow2 = (r & (r - 1)) == 0;
+        const bool ok   = pow2 ? r == 2 || r == 4 || r == 8 || (r == 16 && pmax_of<T> >= 16) : mixed_build;
         if (!ok)
             throw std::logic_error("no butterfly for a radix-" + std::to_string(r) + " pass in this kernel build");
     }
 }
 
-// launches the power-of-two or the mixed-radix build of a kernel role
+template <typename T, bool INV, int ROLE, bool MIXED, bool FL, bool FS>
+void launch_fft_as(const lds_geom& G, const cx<T>* tw, long long batch, const xload<T>& ld, const xstore<T>& st,
+                   const fourstep_args<T>& fs, unsigned grid, unsigned block, size_t sh, hipStream_t s)
+{
+    allow_lds(k_fft<T, INV, ROLE, MIXED, FL, FS>, sh);
+    hipLaunchKernelGGL((k_fft<T, INV, ROLE, MIXED, FL, FS>), dim3(grid), dim3(block), sh, s, G, tw, batch, ld, st, fs);
+}
+
+// launches the power-of-two or the mixed-radix build of a kernel role; mixed radices with the first
+// and last pass on HBM directly where the data are plain. Transforms of fewer than 16 threads load and
+// store through LDS in whole-workgroup runs instead (their lanes would touch a line each).
 template <typename T, bool INV, int ROLE>
 void launch_fft(bool mixed, const lds_geom& G, const cx<T>* tw, long long batch, const xload<T>& ld,
                 const xstore<T>& st, const fourstep_args<T>& fs, unsigned grid, unsigned block, size_t sh,
@@ -798,15 +929,27 @@ void launch_fft(bool mixed, const lds_geom& G, const cx<T>* tw, long long batch,
     // complex values in and out: batch items (columns or rows in the four-step roles) of G.n points
     timing::span ts([mixed] { return timing::kernel_name("k_fft", timing::type_name<T>(), INV, ROLE, mixed); },
                     2 * (long long)sizeof(cx<T>) * batch * G.n, s);
-    if (mixed)
+    const bool wide = ROLE != role_direct || G.tpt >= 16;
+    const bool fl   = wide && G.pass[0].kind == pass_radix && (ROLE == role_row || plain(ld));
+    const bool fl2  = fl && G.np >= 2;
+    const bool fst  = wide && G.np >= 2 && G.pass[G.np - 1].kind == pass_radix && (ROLE == role_col || plain(st));
+    if (!mixed)
+        launch_fft_as<T, INV, ROLE, false, false, false>(G, tw, batch, ld, st, fs, grid, block, sh, s);
+    else if constexpr (ROLE == role_row)
     {
-        allow_lds(k_fft<T, INV, ROLE, true>, sh);
-        hipLaunchKernelGGL((k_fft<T, INV, ROLE, true>), dim3(grid), dim3(block), sh, s, G, tw, batch, ld, st, fs);
+        if (fl)
+            launch_fft_as<T, INV, ROLE, true, true, false>(G, tw, batch, ld, st, fs, grid, block, sh, s);
+        else
+            launch_fft_as<T, INV, ROLE, true, false, false>(G, tw, batch, ld, st, fs, grid, block, sh, s);
     }
     else
     {
-        allow_lds(k_fft<T, INV, ROLE, false>, sh);
-        hipLaunchKernelGGL((k_fft<T, INV, ROLE, false>), dim3(grid), dim3(block), sh, s, G, tw, batch, ld, st, fs);
+        if (fl2 && fst)
+            launch_fft_as<T, INV, ROLE, true, true, true>(G, tw, batch, ld, st, fs, grid, block, sh, s);
+        else if (fst)
+            launch_fft_as<T, INV, ROLE, true, false, true>(G, tw, batch, ld, st, fs, grid, block, sh, s);
+        else
+            launch_fft_as<T, INV, ROLE, true, false, false>(G, tw, batch, ld, st, fs, grid, block, sh, s);
     }
     hip_check(hipGetLastError(), "fft launch");
 }
@@ -835,10 +978,9 @@ struct core_fft
 
     static bool fits_lds(size_t len)
     {
-        stockham s;
-        if (!make_stockham((long long)len, s, pmax_of<T>))
-            return false;
-        return s.tpt <= max_block_of(is_mixed(s)) && len * sizeof(cx<T>) <= lds_budget();
+        const bool mixed = (len & (len - 1)) != 0;
+        return len * sizeof(cx<T>) <= lds_budget() &&
+               workgroup_threads((long long)len, pmax_of<T>, false) <= max_block_of(mixed);
     }
 
     static int pick_tpb(const stockham& s)
@@ -1000,7 +1142,7 @@ struct core_fft
         const long long chunk = round > 0 ? round : this->chunk;
         const cx<T>* t   = tw.as<cx<T>>();
         lds_geom GA      = make_geom(SA, C, 1, C, 1);
-        lds_geom GB      = make_geom(SB, R, 0, 1, (int)n1 + 1);
+        lds_geom GB      = make_geom(SB, R, 0, 1, (int)n1 | 1); // an odd distance: the transposed reads spread
         const size_t shA = lds_padded_elems((size_t)C * n2) * sizeof(cx<T>);
         const size_t shB = lds_padded_elems((size_t)R * (n1 + 1)) * sizeof(cx<T>);
         fourstep_args<T> fs;

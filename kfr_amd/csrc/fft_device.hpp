@@ -288,6 +288,75 @@ __device__ __forceinline__ void bfly_odd(cx<T>* v)
 }
 
 template <int R, bool INV, typename T>
+__device__ __forceinline__ void butterfly(cx<T>* v);
+
+// inverse of a modulo m (coprime)
+constexpr int mod_inverse(int a, int m)
+{
+    for (int x = 1; x < m; ++x)
+        if (a * x % m == 1)
+            return x;
+    return 1;
+}
+
+// N1*N2 points with coprime N1 and N2 (Good and Thomas's prime factor map): input N2*n1 + N1*n2 and
+// output N2*(N2^-1 mod N1)*k1 + N1*(N1^-1 mod N2)*k2, both mod N1*N2, make it an N1 x N2 DFT without
+// twiddles between the two.
+template <int N1, int N2, bool INV, typename T>
+__device__ __forceinline__ void bfly_pfa(cx<T>* v)
+{
+    constexpr int N = N1 * N2;
+    cx<T> a[N1][N2];
+    static_for<N2>([&](auto i2)
+    {
+        constexpr int n2 = decltype(i2)::value;
+        cx<T> u[N1];
+        static_for<N1>([&](auto i1)
+        {
+            constexpr int n1 = decltype(i1)::value;
+            u[n1]            = v[(N2 * n1 + N1 * n2) % N];
+        });
+        butterfly<N1, INV>(u);
+        static_for<N1>([&](auto i1) { a[decltype(i1)::value][n2] = u[decltype(i1)::value]; });
+    });
+    static_for<N1>([&](auto i1)
+    {
+        constexpr int k1 = decltype(i1)::value;
+        butterfly<N2, INV>(a[k1]);
+        static_for<N2>([&](auto i2)
+        {
+            constexpr int k2 = decltype(i2)::value;
+            constexpr int k  = (N2 * mod_inverse(N2 % N1, N1) * k1 + N1 * mod_inverse(N1 % N2, N2) * k2) % N;
+            v[k]             = a[k1][k2];
+        });
+    });
+}
+
+template <bool INV, typename T>
+__device__ __forceinline__ void bfly9(cx<T>* v)
+{
+    // 3 x 3: column DFTs over n = 3*n1 + n2, twiddle W9^(n2*k1), row DFTs; X[k1 + 3*k2]
+    cx<T> a[3][3];
+    static_for<3>([&](auto i2)
+    {
+        constexpr int n2 = decltype(i2)::value;
+        cx<T> u[3]       = { v[n2], v[3 + n2], v[6 + n2] };
+        bfly_odd<3, INV>(u);
+        a[0][n2] = u[0];
+        a[1][n2] = twc<INV, n2, 9>(u[1]);
+        a[2][n2] = twc<INV, 2 * n2, 9>(u[2]);
+    });
+    static_for<3>([&](auto i1)
+    {
+        constexpr int k1 = decltype(i1)::value;
+        bfly_odd<3, INV>(a[k1]);
+        v[k1]     = a[k1][0];
+        v[k1 + 3] = a[k1][1];
+        v[k1 + 6] = a[k1][2];
+    });
+}
+
+template <int R, bool INV, typename T>
 __device__ __forceinline__ void butterfly(cx<T>* v)
 {
     if constexpr (R == 2)
@@ -298,6 +367,18 @@ __device__ __forceinline__ void butterfly(cx<T>* v)
         bfly8<INV>(v);
     else if constexpr (R == 16)
         bfly16<INV>(v);
+    else if constexpr (R == 9)
+        bfly9<INV>(v);
+    else if constexpr (R == 6)
+        bfly_pfa<2, 3, INV>(v);
+    else if constexpr (R == 10)
+        bfly_pfa<2, 5, INV>(v);
+    else if constexpr (R == 12)
+        bfly_pfa<4, 3, INV>(v);
+    else if constexpr (R == 14)
+        bfly_pfa<2, 7, INV>(v);
+    else if constexpr (R == 15)
+        bfly_pfa<3, 5, INV>(v);
     else
         bfly_odd<R, INV>(v);
 }
@@ -334,16 +415,19 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, const fastdiv& f)
 // radices before pass p, butterfly j (0 <= j < n/R) reads x[j + r*n/R] (r = 0..R-1), multiplies
 // element r by W_{Ns*R}^{r*(j mod Ns)}, runs the R-point DFT and writes element r to
 // (j - j mod Ns)*R + j mod Ns + r*Ns. The last pass has Ns*R = n and writes j + r*n/R, so the
-// result is in natural order without a reorder pass. The transform is loaded into LDS with
-// coalesced reads, every pass runs LDS -> registers -> LDS, and the result is stored from LDS, so
-// every HBM element is touched once.
+// result is in natural order without a reorder pass. Where data are plain, the first pass reads
+// its operands straight from HBM (consecutive threads, consecutive addresses) and the last pass
+// writes straight to HBM, so a transform of np passes crosses LDS np - 1 times; a load or store
+// phase with element operations stages through LDS instead. What bounded these kernels was instructions
+// and LDS trips: staging both ends and radices of at most 7 for odd factors, 960 points made five trips
+// and took 172 us for 16384 f32 transforms; as 15 x 16 x 4 with two trips they take 57 us (4.4 TB/s, a
+// copy of the same bytes 49 us). f64 30240 x 256 (four-step, 168 x 180) 229 -> 163 us, the uneven batch of
+// 20,000 transforms 429 -> 338 us.
 
 constexpr int max_passes = 20;
-// Complex values a thread holds per pass and stages per load/store phase: 16 complex f32 (a radix-16
-// butterfly) or 8 complex f64 (radix 8). Kernels come in two register classes: power-of-two radices
-// only, with up to 1024 threads per block (128 VGPRs each), and mixed radices (odd butterflies and
-// direct prime passes need more temporaries), with up to 512 threads (256 VGPRs each). Both fit
-// without spilling to scratch.
+// Complex values a thread holds per pass: about 16 complex f32 or 8 complex f64 (bflies). Kernels come
+// in two register classes: power-of-two radices only, with up to 1024 threads per block (128 VGPRs
+// each), and mixed radices, with up to 512 threads (256 VGPRs each).
 // The f64 value is a build option so that the CPU emulation of these kernels (tests/cpu_emu) can check
 // the 16-points-per-thread geometry for f64 too; the library is built with 8.
 #ifndef KFR_AMD_PMAX_F64
@@ -357,7 +441,7 @@ __host__ __device__ constexpr int max_block_of(bool mixed) { return mixed ? max_
 
 enum pass_kind : int
 {
-    pass_radix   = 0, // specialised butterfly, R in {2,3,4,5,7,8,16}
+    pass_radix   = 0, // specialised butterfly (lds_radix)
     pass_generic = 1  // direct R-point DFT (R prime, 11..127) from a W_{Ns*R} table
 };
 
@@ -365,6 +449,7 @@ struct pass_desc
 {
     int radix;
     int ns;
+    int nb; // butterflies, n / radix
     int tw; // offset of this pass's twiddles in the plan's table (complex elements)
     int kind;
     fastdiv ns_div;
@@ -379,17 +464,38 @@ struct lds_geom
     int mapping; // 0: transform = tid / tpt ; 1: transform = tid % tpb
     int ls;      // LDS element stride
     int ld;      // LDS distance between transforms
-    int padshift; // LDS padding: one slot per 2^padshift elements
+    int padshift; // LDS padding: one slot per 2^padshift elements (padded kernels)
+    fastdiv tpt_div;
     pass_desc pass[max_passes];
 };
 
-// LDS layout: logical element x lives at x + x/16, one padding slot per 16 elements, so that the
-// power-of-two strides of the Stockham passes (stride-R writes of the first pass, one transform per
-// lane for short lengths) spread over the banks instead of hitting one.
-__device__ __forceinline__ int lds_pad(int x, int s) { return x + (x >> s); }
+// Radices with a butterfly, and butterflies per thread of a radix-R pass: as many as a thread's pm
+// values hold, rounded up for the small radices so that every length up to 512*pm runs on at most 512
+// threads; one of radix 12, 14 and 15 (f32), whose tables and temporaries are the largest.
+__host__ __device__ constexpr bool lds_radix(int r)
+{
+    return (r >= 2 && r <= 10) || r == 12 || r == 14 || r == 15 || r == 16;
+}
+__host__ __device__ constexpr int bflies(int r, int pm) { return r >= 12 ? (pm >= r ? pm / r : 1) : (pm + r - 1) / r; }
+template <typename T, int R>
+inline constexpr int bflies_of = bflies(R, pmax_of<T>);
+
+// Padded LDS layout (PAD): logical element x lives at x + (x >> padshift), one padding slot per 16
+// (or 32) elements, so that the power-of-two strides of the Stockham passes spread over the banks
+// instead of hitting one. Schedules with an odd factor start with an odd radix where they can, so the
+// strided writes of their first pass spread by themselves and the layout stays linear: one addition
+// per address instead of three operations.
+template <bool PAD>
+__device__ __forceinline__ int lds_pad(int x, int s)
+{
+    if constexpr (PAD)
+        return x + (x >> s);
+    else
+        return x;
+}
 __host__ __device__ inline size_t lds_padded_elems(size_t logical) { return logical + logical / 16 + 1; }
 
-template <typename T>
+template <typename T, bool PAD>
 struct fft_ctx
 {
     cx<T>* lds;  // the block's LDS
@@ -400,76 +506,202 @@ struct fft_ctx
     int tb;      // transform index within the block
     bool valid;  // transform exists (batch tail)
     long long g; // global transform index
-    // element i of this transform (padded layout, see lds_pad)
-    __device__ __forceinline__ cx<T>& at(int i) const { return lds[lds_pad(base + i * ls, ps)]; }
+    // slot at logical offset x
+    __device__ __forceinline__ cx<T>& slot(int x) const { return lds[lds_pad<PAD>(x, ps)]; }
+    // element i of this transform
+    __device__ __forceinline__ cx<T>& at(int i) const { return slot(base + i * ls); }
 };
 
-// butterflies per thread in a radix-R pass: floor(pmax/R) (at least 1), or with WIDE ceil(pmax/R), so
-// that R*M >= pmax and every length up to 512*pmax runs on at most 512 threads per transform
-template <typename T, int R, bool WIDE>
-inline constexpr int bflies_of = WIDE ? (pmax_of<T> + R - 1) / R : (pmax_of<T> / R > 0 ? pmax_of<T> / R : 1);
-
-// one radix pass, LDS -> LDS
-template <typename T, int R, bool INV, bool WIDE = false>
-__device__ __forceinline__ void radix_pass(const lds_geom& G, const pass_desc& P, const cx<T>* __restrict__ tw,
-                                           const fft_ctx<T>& c)
+// Where a pass reads and writes its values: LDS, or (first and last pass) strided global memory.
+struct via_lds
 {
-    constexpr int M = bflies_of<T, R, WIDE>;
-    const int nb    = G.n / R;
+    static constexpr bool global = false;
+};
+// first pass: element i at p[i * stride]; conj reads conjugates; threads of missing transforms read
+// zeros
+template <typename T, bool CONJ = false>
+struct from_global
+{
+    static constexpr bool global = true;
+    const cx<T>* p;
+    long long stride;
+    bool valid;
+    bool conj = false;
+    __device__ __forceinline__ cx<T> get(const cx<T>* q) const
+    {
+        cx<T> v = valid ? *q : cx<T>{ T(0), T(0) };
+        if constexpr (CONJ)
+            v.im = conj ? -v.im : v.im;
+        return v;
+    }
+};
+// last pass: element i to p[i * stride]; NT: nontemporal stores
+template <typename T, bool CONJ = false, bool NT = false>
+struct to_global
+{
+    static constexpr bool global  = true;
+    static constexpr bool twiddle = false;
+    cx<T>* p;
+    long long stride;
+    bool valid;
+    bool conj = false;
+    __device__ __forceinline__ void put(cx<T>* q, cx<T> v) const
+    {
+        if constexpr (CONJ)
+            v.im = conj ? -v.im : v.im;
+        if constexpr (NT)
+        {
+            using V2 = T __attribute__((ext_vector_type(2)));
+            __builtin_nontemporal_store(V2{ v.re, v.im }, reinterpret_cast<V2*>(q));
+        }
+        else
+            *q = v;
+    }
+};
+// last pass of a four-step column: element i times W_n^(col*i) (ta[h] = W_n^(h*2^lbits), tb[l] = W_n^l;
+// none if ta is null) to p[i * stride]
+template <typename T>
+struct to_column : to_global<T>
+{
+    static constexpr bool twiddle = true;
+    const cx<T>*ta, *tb;
+    int lbits;
+    unsigned col;
+    __device__ __forceinline__ cx<T> table(unsigned long long m) const
+    {
+        return cmul(ta[m >> lbits], tb[m & ((1ull << lbits) - 1)]);
+    }
+};
+
+__host__ __device__ constexpr int ceil_log2(int v)
+{
+    int l = 0;
+    while ((1 << l) < v)
+        ++l;
+    return l;
+}
+
+// workgroup barrier for LDS exchanges: the fences cover the local address space only, so it does not
+// wait for outstanding global memory operations
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// one radix pass from src to dst; FIRST: pass 0 (Ns = 1, no twiddles). When dst is LDS, it ends with a
+// barrier.
+template <typename T, int R, bool INV, bool FIRST, bool PAD, typename Src, typename Dst>
+__device__ __forceinline__ void radix_pass(const lds_geom& G, const pass_desc& P, const cx<T>* __restrict__ tw,
+                                           const fft_ctx<T, PAD>& c, const Src& src, const Dst& dst)
+{
+    constexpr int M = bflies_of<T, R>;
+    const int nb    = P.nb;
     cx<T> v[M][R];
-    int kk[M];
 #pragma unroll
     for (int m = 0; m < M; ++m)
     {
         const int j = c.t + m * G.tpt;
         if (j < nb)
         {
+            if constexpr (Src::global)
+            {
+                const cx<T>* q = src.p + (long long)j * src.stride;
+                const long long step = (long long)nb * src.stride;
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-                v[m][r] = c.at(j + r * nb);
+                for (int r = 0; r < R; ++r)
+                    v[m][r] = src.get(q + r * step);
+            }
+            else
+            {
+                const int x = c.base + j * c.ls, step = nb * c.ls;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    v[m][r] = c.slot(x + r * step);
+            }
         }
     }
+    if constexpr (!Src::global && !Dst::global)
+        lds_barrier(); // every value of the previous pass is read before this pass overwrites it
+    [[maybe_unused]] cx<T> B[R];
+    if constexpr (Dst::global)
+        if constexpr (Dst::twiddle)
+        {
+            // output j + r*Ns of a column takes W^(col*j) times W^(col*Ns*r), the latter built from the
+            // table values at r = 2^b with one product per value
+            if (dst.ta)
+            {
+#pragma unroll
+                for (int b = 0; (1 << b) < R; ++b)
+                    B[1 << b] = dst.table((unsigned long long)dst.col * ((unsigned)P.ns << b));
+#pragma unroll
+                for (int r = 3; r < R; ++r)
+                    if ((r & (r - 1)) != 0)
+                        B[r] = cmul(B[r - (1 << (ceil_log2(r + 1) - 1))], B[1 << (ceil_log2(r + 1) - 1)]);
+            }
+        }
 #pragma unroll
     for (int m = 0; m < M; ++m)
     {
         const int j = c.t + m * G.tpt;
-        kk[m]       = 0;
         if (j < nb)
         {
-            const int k = P.ns == 1 ? 0 : (int)(j - fdiv(j, P.ns_div) * P.ns);
-            kk[m]       = k;
-            if (P.ns > 1)
+            int k = 0;
+            if constexpr (!FIRST)
             {
-                const cx<T>* w = tw + P.tw + k * (R - 1);
+                if (P.ns > 1)
+                {
+                    // the table's row of k: W_{Ns*R}^(r*k) at k*(R-1) + r-1 (one base address, wide loads)
+                    k              = Dst::global ? j : (int)(j - fdiv(j, P.ns_div) * P.ns);
+                    const cx<T>* w = tw + P.tw + k * (R - 1);
 #pragma unroll
-                for (int r = 1; r < R; ++r)
-                    v[m][r] = ctw<INV>(v[m][r], w[r - 1]);
+                    for (int r = 1; r < R; ++r)
+                        v[m][r] = ctw<INV>(v[m][r], w[r - 1]);
+                }
             }
             butterfly<R, INV>(v[m]);
+            if constexpr (Dst::global)
+            {
+                // last pass: j < Ns, output r of butterfly j is element j + r*Ns
+                if constexpr (Dst::twiddle)
+                {
+                    if (dst.ta)
+                    {
+                        const cx<T> A = dst.table((unsigned long long)dst.col * (unsigned)j);
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+                            v[m][r] = ctw<INV>(v[m][r], r == 0 ? A : cmul(A, B[r]));
+                    }
+                }
+                if (dst.valid)
+                {
+                    cx<T>* q             = dst.p + (long long)j * dst.stride;
+                    const long long step = (long long)P.ns * dst.stride;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        dst.put(q + r * step, v[m][r]);
+                }
+            }
+            else
+            {
+                const int x = c.base + ((j - k) * R + k) * c.ls, step = P.ns * c.ls;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    c.slot(x + r * step) = v[m][r];
+            }
         }
     }
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < M; ++m)
-    {
-        const int j = c.t + m * G.tpt;
-        if (j < nb)
-        {
-            const int base = (j - kk[m]) * R + kk[m];
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                c.at(base + r * P.ns) = v[m][r];
-        }
-    }
-    __syncthreads();
+    if constexpr (!Dst::global)
+        lds_barrier();
 }
 
 // direct DFT pass for a prime radix without a specialised butterfly, LDS -> LDS.
 // Output o = q*Ns*R + k2*Ns + k is sum_r x[j + r*n/R] W_{Ns*R}^{r*(k + k2*Ns)} with j = q*Ns + k;
 // the pass's table holds W_{Ns*R}^m for m in [0, Ns*R).
-template <typename T, bool INV>
+template <typename T, bool INV, bool PAD>
 __device__ __forceinline__ void generic_pass(const lds_geom& G, const pass_desc& P, const cx<T>* __restrict__ tw,
-                                             const fft_ctx<T>& c)
+                                             const fft_ctx<T, PAD>& c)
 {
     const int R  = P.radix;
     const int nb = G.n / R;
@@ -501,7 +733,7 @@ __device__ __forceinline__ void generic_pass(const lds_geom& G, const pass_desc&
             out[m] = acc;
         }
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int m = 0; m < pmax_of<T>; ++m)
     {
@@ -509,66 +741,93 @@ __device__ __forceinline__ void generic_pass(const lds_geom& G, const pass_desc&
         if (o < G.n)
             c.at(o) = out[m];
     }
-    __syncthreads();
+    lds_barrier();
 }
 
-// all passes of the transform held in LDS (natural order in, natural order out). MIXED = false
-// compiles only the power-of-two butterflies (radix 16 for f32, 8 for f64, and the remainders). WIDE
-// selects the ceil(pmax/R) butterflies per thread of radix_pass (the geometry must come from
-// make_stockham with wide = true).
-template <typename T, bool INV, bool MIXED, bool WIDE = false>
-__device__ __forceinline__ void fft_passes(const lds_geom& G, const cx<T>* tw, const fft_ctx<T>& c)
+// f(std::integral_constant<int, R>) for the radix r of a pass (MIXED = false: only the power-of-two
+// butterflies; radix 16 only where a thread holds 16 values: check_pass_radices rejects it elsewhere)
+template <typename T, bool MIXED, typename F>
+__device__ __forceinline__ void with_radix(int r, F&& f)
 {
-    for (int p = 0; p < G.np; ++p)
+    auto call = [&](auto R)
     {
-        const pass_desc& P = G.pass[p];
-        switch (P.radix)
-        {
-        case 2:
-            radix_pass<T, 2, INV, WIDE>(G, P, tw, c);
-            break;
-        case 4:
-            radix_pass<T, 4, INV, WIDE>(G, P, tw, c);
-            break;
-        case 8:
-            radix_pass<T, 8, INV, WIDE>(G, P, tw, c);
-            break;
-        case 16: // only where a thread holds 16 values (check_pass_radices rejects it elsewhere)
-            if constexpr (pmax_of<T> >= 16)
-                radix_pass<T, 16, INV, WIDE>(G, P, tw, c);
-            break;
-        default:
-            if constexpr (MIXED)
-            {
-                switch (P.radix)
-                {
-                case 3:
-                    radix_pass<T, 3, INV, WIDE>(G, P, tw, c);
-                    break;
-                case 5:
-                    radix_pass<T, 5, INV, WIDE>(G, P, tw, c);
-                    break;
-                case 7:
-                    radix_pass<T, 7, INV, WIDE>(G, P, tw, c);
-                    break;
-                default:
-                    generic_pass<T, INV>(G, P, tw, c);
-                    break;
-                }
-            }
-            break;
-        }
+        if constexpr ((decltype(R)::value & (decltype(R)::value - 1)) == 0
+                          ? decltype(R)::value <= 8 || pmax_of<T> >= 16
+                          : MIXED)
+            f(R);
+    };
+    switch (r)
+    {
+    case 2: call(std::integral_constant<int, 2>{}); break;
+    case 3: call(std::integral_constant<int, 3>{}); break;
+    case 4: call(std::integral_constant<int, 4>{}); break;
+    case 5: call(std::integral_constant<int, 5>{}); break;
+    case 6: call(std::integral_constant<int, 6>{}); break;
+    case 7: call(std::integral_constant<int, 7>{}); break;
+    case 8: call(std::integral_constant<int, 8>{}); break;
+    case 9: call(std::integral_constant<int, 9>{}); break;
+    case 10: call(std::integral_constant<int, 10>{}); break;
+    case 12: call(std::integral_constant<int, 12>{}); break;
+    case 14: call(std::integral_constant<int, 14>{}); break;
+    case 15: call(std::integral_constant<int, 15>{}); break;
+    case 16: call(std::integral_constant<int, 16>{}); break;
+    default: break;
     }
 }
 
-template <typename T>
-__device__ __forceinline__ fft_ctx<T> make_ctx(const lds_geom& G, cx<T>* lds, long long first_g, long long batch)
+// passes [first, last) of the transform held in LDS
+template <typename T, bool INV, bool MIXED, bool PAD>
+__device__ __forceinline__ void fft_passes(const lds_geom& G, const cx<T>* tw, const fft_ctx<T, PAD>& c, int first,
+                                           int last)
 {
-    fft_ctx<T> c;
+    for (int p = first; p < last; ++p)
+    {
+        const pass_desc& P = G.pass[p];
+        if constexpr (MIXED)
+        {
+            if (P.kind == pass_generic)
+            {
+                generic_pass<T, INV>(G, P, tw, c);
+                continue;
+            }
+        }
+        with_radix<T, MIXED>(P.radix, [&](auto R) {
+            radix_pass<T, decltype(R)::value, INV, false>(G, P, tw, c, via_lds{}, via_lds{});
+        });
+    }
+}
+// all passes (natural order in, natural order out)
+template <typename T, bool INV, bool MIXED, bool PAD>
+__device__ __forceinline__ void fft_passes(const lds_geom& G, const cx<T>* tw, const fft_ctx<T, PAD>& c)
+{
+    fft_passes<T, INV, MIXED>(G, tw, c, 0, G.np);
+}
+// pass 0 from src to LDS
+template <typename T, bool INV, bool MIXED, bool PAD, typename Src>
+__device__ __forceinline__ void first_pass(const lds_geom& G, const cx<T>* tw, const fft_ctx<T, PAD>& c, const Src& src)
+{
+    with_radix<T, MIXED>(G.pass[0].radix, [&](auto R) {
+        radix_pass<T, decltype(R)::value, INV, true>(G, G.pass[0], tw, c, src, via_lds{});
+    });
+}
+// the last of two or more passes from LDS to dst
+template <typename T, bool INV, bool MIXED, bool PAD, typename Dst>
+__device__ __forceinline__ void last_pass(const lds_geom& G, const cx<T>* tw, const fft_ctx<T, PAD>& c, const Dst& dst)
+{
+    const pass_desc& P = G.pass[G.np - 1];
+    with_radix<T, MIXED>(P.radix, [&](auto R) {
+        radix_pass<T, decltype(R)::value, INV, false>(G, P, tw, c, via_lds{}, dst);
+    });
+}
+
+template <bool PAD, typename T>
+__device__ __forceinline__ fft_ctx<T, PAD> make_ctx(const lds_geom& G, cx<T>* lds, long long first_g, long long batch)
+{
+    fft_ctx<T, PAD> c;
     const int tid = threadIdx.x;
     if (G.mapping == 0)
     {
-        c.tb = tid / G.tpt;
+        c.tb = (int)fdiv((uint32_t)tid, G.tpt_div);
         c.t  = tid - c.tb * G.tpt;
     }
     else

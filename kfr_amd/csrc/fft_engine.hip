@@ -93,15 +93,15 @@ __global__ void __launch_bounds__(max_block_pow2) k_bluestein(lds_geom G, const 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds            = reinterpret_cast<cx<T>*>(smem_raw);
     const long long first = (long long)blockIdx.x * G.tpb;
-    const fft_ctx<T> c    = make_ctx<T>(G, lds, first, batch);
-    block_load(G, lds, first, batch, ld, mdiv); // ld carries the chirp and the zero padding
+    const fft_ctx<T, true> c = make_ctx<true, T>(G, lds, first, batch);
+    block_load<true>(G, lds, first, batch, ld, mdiv); // ld carries the chirp and the zero padding
     __syncthreads();
     fft_passes<T, false, false>(G, tw, c); // M is a power of two
     for (int i = c.t; i < G.n; i += G.tpt)
         c.at(i) = INV ? cmul(c.at(i), H[i]) : cmulc(c.at(i), H[i]);
     __syncthreads();
     fft_passes<T, true, false>(G, tw, c);
-    block_store(G, lds, first, batch, st, mdiv); // st carries the chirp and the truncation
+    block_store<true>(G, lds, first, batch, st, mdiv); // st carries the chirp and the truncation
 }
 
 // h: the FP64 chirp mirrored into both ends of M points
@@ -499,9 +499,10 @@ __global__ void k_real_repack(cx<T>* out, long long odist, const cx<T>* Z, long 
         repack_pair<T, true>(o, rtw, csize, k, z[k], z[csize - k]);
 }
 
-// fused forward real transform for LDS-resident half lengths: the FFT result is repacked from LDS
-template <typename T, bool MIXED>
-__global__ void __launch_bounds__(max_block_of(MIXED)) k_real_fwd(lds_geom G, const cx<T>* __restrict__ tw,
+// fused forward real transform for LDS-resident half lengths: the FFT result is repacked from LDS. FL: plain
+// input, read by the first pass itself (mixed radices)
+template <typename T, bool MIXED, bool FL>
+__global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) k_real_fwd(lds_geom G, const cx<T>* __restrict__ tw,
                                                                    long long batch, xload<T> ld, cx<T>* out,
                                                                    long long odist, const cx<T>* __restrict__ rtw,
                                                                    int fmt, fastdiv ndiv)
@@ -509,10 +510,17 @@ __global__ void __launch_bounds__(max_block_of(MIXED)) k_real_fwd(lds_geom G, co
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds            = reinterpret_cast<cx<T>*>(smem_raw);
     const long long first = (long long)blockIdx.x * G.tpb;
-    const fft_ctx<T> c    = make_ctx<T>(G, lds, first, batch);
-    block_load(G, lds, first, batch, ld, ndiv);
-    __syncthreads();
-    fft_passes<T, false, MIXED>(G, tw, c);
+    const fft_ctx<T, !MIXED> c = make_ctx<!MIXED, T>(G, lds, first, batch);
+    if constexpr (FL)
+        first_pass<T, false, MIXED>(
+            G, tw, c,
+            from_global<T>{ static_cast<const cx<T>*>(ld.p) + (c.valid ? c.g + ld.b0 : 0) * ld.pdist, 1, c.valid });
+    else
+    {
+        block_load<!MIXED>(G, lds, first, batch, ld, ndiv);
+        __syncthreads();
+    }
+    fft_passes<T, false, MIXED>(G, tw, c, FL ? 1 : 0, G.np);
     if (!c.valid)
         return;
     const long long csize = G.n;
@@ -589,18 +597,18 @@ struct gpu_dft_real<T>::impl
             const bool mx    = is_mixed(f.S);
             timing::span ts([mx] { return timing::kernel_name("k_real_fwd", timing::type_name<T>(), mx); },
                             2 * (long long)sizeof(cx<T>) * batch * (long long)csize, s);
-            if (mx)
+            auto go = [&](auto kernel)
             {
-                allow_lds(k_real_fwd<T, true>, sh);
-                hipLaunchKernelGGL((k_real_fwd<T, true>), grid, block, sh, s, G, f.tw.template as<cx<T>>(), batch, ld,
-                                   out, odist, rtw.template as<cx<T>>(), fmt, nd);
-            }
+                allow_lds(kernel, sh);
+                hipLaunchKernelGGL(kernel, grid, block, sh, s, G, f.tw.template as<cx<T>>(), batch, ld, out, odist,
+                                   rtw.template as<cx<T>>(), fmt, nd);
+            };
+            if (!mx)
+                go(k_real_fwd<T, false, false>);
+            else if (plain(ld) && G.tpt >= 16 && G.pass[0].kind == pass_radix)
+                go(k_real_fwd<T, true, true>);
             else
-            {
-                allow_lds(k_real_fwd<T, false>, sh);
-                hipLaunchKernelGGL((k_real_fwd<T, false>), grid, block, sh, s, G, f.tw.template as<cx<T>>(), batch, ld,
-                                   out, odist, rtw.template as<cx<T>>(), fmt, nd);
-            }
+                go(k_real_fwd<T, true, false>);
             hip_check(hipGetLastError(), "real forward launch");
             return;
         }

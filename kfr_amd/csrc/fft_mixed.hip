@@ -128,13 +128,6 @@ __device__ __forceinline__ int laddr(int tb, int i)
     return x + (x >> 4);
 }
 
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 struct margs
 {
     const cx<float>* in = nullptr;

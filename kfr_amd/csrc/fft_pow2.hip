@@ -394,15 +394,6 @@ __device__ __forceinline__ void bfly16_mfma(cx<float> (&u)[16], const mfma16& K)
     }
 }
 
-// Workgroup barrier for the LDS exchanges: the fences cover the local address space only, so it
-// does not wait for outstanding global memory operations.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // the thread whose positions feed the second butterfly of thread t in a mirrored last pass
 template <int MODE, int TP>
 __device__ __forceinline__ int mirror_lane(int t)
