@@ -1336,6 +1336,162 @@ __global__ void k_update_history(T* nhist, const T* hist, const T* in, long long
     nhist[i]            = pos < nh1 ? hist[pos] : in[pos - nh1];
 }
 
+// Short calls: the filter in the time domain, one launch. A streaming call of n samples against nt taps is
+// bound by latency, not work: 1024 samples and 4095 taps are 4.2 million multiply-adds, about 0.1 us of
+// the card's rate, while the overlap-save path ran six dependent launches on one workgroup each
+// (37 us of kernels per call, 47 us in all; this kernel takes 10 us and a call 23 us, most of it the wait
+// that the synchronous entry point ends with). A wave computes fir_outs * 64/G adjacent outputs: the G
+// lanes of a group split the taps in runs of fir_taps and add their partial sums with a butterfly of
+// lane exchanges, so no sum runs over more than nt/G terms. Samples and taps sit in LDS; a run of taps
+// and its window of samples are read with 16-byte loads (the samples are stored so that every window
+// starts on such a boundary; 4-byte reads at this stride met eight lanes per bank and took 3 us more).
+// The workgroups also write the history of the next call.
+constexpr int fir_outs = 8, fir_taps = 8, fir_block = 256; // runs and windows of fir_read8
+
+// values of the two LDS arrays: taps padded to whole runs of G lanes, samples of one workgroup's outputs
+__host__ __device__ inline int fir_padded_taps(int nt, int G) { return (nt + G * fir_taps - 1) / (G * fir_taps) * (G * fir_taps); }
+__host__ __device__ inline int fir_block_outs(int G) { return fir_block / G * fir_outs; }
+__host__ __device__ inline int fir_lds_values(int nt, int G) { return 2 * fir_padded_taps(nt, G) + fir_block_outs(G); }
+
+template <typename T>
+__device__ __forceinline__ void fir_add(T& acc, T h, T x)
+{
+    acc += h * x;
+}
+template <typename T>
+__device__ __forceinline__ void fir_add(cx<T>& acc, cx<T> h, cx<T> x)
+{
+    acc.re += h.re * x.re - h.im * x.im;
+    acc.im += h.re * x.im + h.im * x.re;
+}
+template <typename T>
+__device__ __forceinline__ T fir_lane_add(T v, int o)
+{
+    return v + __shfl_xor(v, o);
+}
+template <typename T>
+__device__ __forceinline__ cx<T> fir_lane_add(cx<T> v, int o)
+{
+    return { fir_lane_add(v.re, o), fir_lane_add(v.im, o) };
+}
+
+// eight values from a 16-byte boundary of LDS
+template <typename V>
+__device__ __forceinline__ void fir_read8(const V* p, V* o)
+{
+    constexpr int W = 16 / sizeof(V);
+    struct alignas(16) wide
+    {
+        V v[W];
+    };
+#pragma unroll
+    for (int k = 0; k < 8 / W; ++k)
+    {
+        const wide a = reinterpret_cast<const wide*>(p)[k];
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+            o[k * W + i] = a.v[i];
+    }
+}
+
+template <typename V>
+__global__ void __launch_bounds__(fir_block) k_fir(V* __restrict__ out, V* __restrict__ nhist, const V* __restrict__ hist,
+                                                  const V* __restrict__ in, const V* __restrict__ taps, int nt,
+                                                  long long n, int G)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int np      = fir_padded_taps(nt, G);
+    const int outs    = fir_block_outs(G);
+    V* h              = reinterpret_cast<V*>(smem_raw); // taps, zero to np
+    V* x              = h + np;                         // sample o0 - np + 1 + i of the call at x[i] (i < np + outs)
+    const int tid     = threadIdx.x;
+    const long long o0  = (long long)blockIdx.x * outs;
+    const long long nh1 = nt - 1;
+    // many loads in flight per thread (one at a time, their latencies were most of the kernel)
+    constexpr int F = 128 / sizeof(V) > 24 ? 24 : 128 / sizeof(V);
+    for (int i0 = tid; i0 < 2 * np + outs; i0 += F * fir_block)
+    {
+        V v[F];
+#pragma unroll
+        for (int k = 0; k < F; ++k)
+        {
+            const int i         = i0 + k * fir_block;
+            const long long pos = o0 - 2 * np + 1 + i; // sample of this call (negative: history) from i = np on
+            const V* p          = nullptr;
+            if (i < np)
+                p = i < nt ? taps + i : nullptr;
+            else if (pos >= 0)
+                p = pos < n && i < 2 * np + outs ? in + pos : nullptr;
+            else
+                p = pos + nh1 >= 0 ? hist + (pos + nh1) : nullptr;
+            v[k] = p ? *p : V{};
+        }
+#pragma unroll
+        for (int k = 0; k < F; ++k)
+            if (i0 + k * fir_block < 2 * np + outs)
+                h[i0 + k * fir_block] = v[k];
+    }
+    __syncthreads();
+    const int g  = tid & (G - 1);
+    const int ob = (tid / G) * fir_outs; // this thread's first output
+    V acc[fir_outs] = {};
+    for (int k0 = g * fir_taps; k0 < np; k0 += G * fir_taps)
+    {
+        // output ob + q takes sample ob + q - (k0 + k), stored at np - 1 + ob + q - k0 - k
+        const V* w = x + (np - fir_taps + ob - k0); // window, a multiple of 8 values from x
+        V hv[8], xv[16];
+        fir_read8(h + k0, hv);
+        fir_read8(w, xv);
+        fir_read8(w + 8, xv + 8);
+#pragma unroll
+        for (int k = 0; k < fir_taps; ++k)
+#pragma unroll
+            for (int q = 0; q < fir_outs; ++q)
+                fir_add(acc[q], hv[k], xv[fir_taps - 1 + q - k]);
+    }
+    for (int o = 1; o < G; o <<= 1)
+#pragma unroll
+        for (int q = 0; q < fir_outs; ++q)
+            acc[q] = fir_lane_add(acc[q], o);
+#pragma unroll
+    for (int q = 0; q < fir_outs; ++q)
+        if (g == (q & (G - 1)) && o0 + ob + q < n)
+            out[o0 + ob + q] = acc[q];
+    for (long long i = (long long)blockIdx.x * fir_block + tid; i < nh1; i += (long long)gridDim.x * fir_block)
+    {
+        const long long pos = n + i; // position in [history | input]
+        nhist[i]            = pos < nh1 ? hist[pos] : in[pos - nh1];
+    }
+}
+
+// Runs the call in the time domain if that is the faster way: at most fir_most multiply-adds, the taps and
+// samples within fir_lds of LDS, and buffers that do not overlap (workgroups write outputs while others
+// read samples). False: the caller's overlap-save path.
+// fir_most: 4095 taps cross over near 40,000 samples (f32; 47 us either way) and 20,000 (f64, twice the
+// LDS reads); 512 taps near a million.
+constexpr long long fir_most = 1ll << 29; // bytes of the values that the multiply-adds take
+constexpr size_t fir_lds     = 140 * 1024;
+template <typename V>
+bool run_fir(V* out, V* nhist, const V* hist, const V* in, const V* taps, size_t nt, size_t n, hipStream_t s)
+{
+    if (nt > (size_t)1 << 20 || (long long)n > fir_most / (long long)(nt * sizeof(V)))
+        return false;
+    const uintptr_t a = reinterpret_cast<uintptr_t>(in), b = reinterpret_cast<uintptr_t>(out);
+    if (a < b + n * sizeof(V) && b < a + n * sizeof(V))
+        return false;
+    int G = 1; // lanes per output group: runs of about 64 taps and more per lane
+    while (G < 64 && (size_t)G * 64 < nt)
+        G <<= 1;
+    const size_t bytes = (size_t)fir_lds_values((int)nt, G) * sizeof(V);
+    if (bytes > fir_lds)
+        return false;
+    allow_lds(k_fir<V>, bytes);
+    hipLaunchKernelGGL(k_fir<V>, dim3(nblocks((long long)n, fir_block_outs(G))), dim3(fir_block), bytes, s, out, nhist,
+                       hist, in, taps, (int)nt, (long long)n, G);
+    hip_check(hipGetLastError(), "time-domain filter launch");
+    return true;
+}
+
 template <typename T>
 __global__ void k_zero(T* p, long long count)
 {
@@ -1392,6 +1548,12 @@ struct gpu_conv_filter<T>::impl
     {
         if (n == 0)
             return;
+        if (run_fir(out, hist[1 - cur].template as<T>(), hist[cur].template as<T>(), in, taps_dev.template as<T>(),
+                    ntaps, n, s))
+        {
+            cur = 1 - cur;
+            return;
+        }
         const long long nseg = (long long)((n + L - 1) / L);
         const long long cs   = (long long)(S / 2 + 1);
         seg.ensure((size_t)nseg * S * sizeof(T));
@@ -1474,6 +1636,12 @@ struct gpu_conv_filter_complex<T>::impl
     {
         if (n == 0)
             return;
+        if (run_fir(out, hist[1 - cur].template as<cx<T>>(), hist[cur].template as<cx<T>>(), in,
+                    taps_dev.template as<cx<T>>(), ntaps, n, s))
+        {
+            cur = 1 - cur;
+            return;
+        }
         const long long nseg = (long long)((n + L - 1) / L);
         seg.ensure((size_t)nseg * S * sizeof(cx<T>));
         yseg.ensure((size_t)nseg * S * sizeof(cx<T>));
