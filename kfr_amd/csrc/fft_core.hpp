@@ -1176,6 +1176,36 @@ struct core_fft
         }
     }
 
+    // ---- one axis of a multidimensional array in place along its stride: `outer` arrays of n rows of
+    // `inner` values, every column transformed by the four-step column kernel without its twiddle
+    bool supports_axis() const { return !fourstep; }
+    template <bool INV>
+    void run_axis(const cx<T>* in, cx<T>* out, long long inner, long long outer, hipStream_t s)
+    {
+        const long long cols = inner * outer;
+        if (fourstep || cols > 0x7fffffffll)
+            throw std::logic_error("this plan cannot transform a strided axis");
+        if (cols <= 0)
+            return;
+        // up to 16 columns per workgroup (whole 128-byte lines), fewer if that leaves CUs without work: the
+        // 1080-point axis of a 1080 x 961 spectrum runs 4 (241 workgroups of 288 threads)
+        int c          = 16;
+        const int most = max_block_of(is_mixed(S));
+        while (c > 1 && ((size_t)c * n * sizeof(cx<T>) > lds_budget() || c * S.tpt > most))
+            c /= 2;
+        while (c > (sizeof(T) == 4 ? 4 : 2) && (cols + c - 1) / c < 256)
+            c /= 2;
+        lds_geom G = make_geom(S, c, 1, c, 1);
+        fourstep_args<T> fs;
+        fs.scratch = out;
+        fs.n1div   = make_fastdiv((uint32_t)inner);
+        fs.n1      = (int)inner;
+        fs.n       = (long long)n * inner;
+        launch_fft<T, INV, role_col>(is_mixed(S), G, tw.as<cx<T>>(), cols, load_plain<T>(in, fs.n), xstore<T>{}, fs,
+                                     nblocks(cols, c), (unsigned)(S.tpt * c), lds_padded_elems((size_t)c * n) * sizeof(cx<T>),
+                                     s);
+    }
+
     // ---- progressive execution (one reference stage per call, include/kfr/dft/fft.hpp:393-439): one
     // item in place on `data`, as units of one launch each. Lengths in one workgroup run one pass of a
     // finer Stockham schedule per unit (about `want` passes); four-step lengths run their column and

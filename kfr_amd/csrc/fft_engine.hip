@@ -419,6 +419,23 @@ void gpu_dft<T>::execute_workspace(void* out, const void* in, long long batch, b
 }
 
 template <typename T>
+bool gpu_dft<T>::supports_axis(long long inner, long long outer) const
+{
+    return p->algo == impl::CORE && p->core->supports_axis() && inner > 0 && outer > 0 &&
+           inner <= 0x7fffffffll / outer;
+}
+template <typename T>
+void gpu_dft<T>::execute_axis(void* out, const void* in, long long inner, long long outer, bool inverse, hipStream_t s)
+{
+    if (!supports_axis(inner, outer))
+        throw std::logic_error("this plan cannot transform a strided axis");
+    if (inverse)
+        p->core->template run_axis<true>(static_cast<const cx<T>*>(in), static_cast<cx<T>*>(out), inner, outer, s);
+    else
+        p->core->template run_axis<false>(static_cast<const cx<T>*>(in), static_cast<cx<T>*>(out), inner, outer, s);
+}
+
+template <typename T>
 int gpu_dft<T>::progressive_prepare(int want)
 {
     return p->prog_prepare(want);

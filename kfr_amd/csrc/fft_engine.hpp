@@ -114,6 +114,10 @@ public:
     // execute() with the intermediates in `w` (no allocation by the plan); Bluestein lengths whose
     // transform does not fit one workgroup are refused
     void execute_workspace(void* out, const void* in, long long batch, bool inverse, hipStream_t s, workspace w);
+    // one axis of a row-major array along its stride: `outer` arrays of n rows of `inner` values, in place
+    // allowed; false from supports_axis if this length (or this many columns) needs contiguous transforms
+    bool supports_axis(long long inner, long long outer) const;
+    void execute_axis(void* out, const void* in, long long inner, long long outer, bool inverse, hipStream_t s);
     // Progressive execution of one transform in place on device data (n values): progressive_prepare
     // lowers the transform to about `want` units (one launch each; Stockham passes of a finer schedule
     // for lengths in one workgroup, the column and the row kernel of a four-step, the whole transform

@@ -1,9 +1,8 @@
-// Multidimensional DFTs on device data. Like the reference (dft_plan_md::execute_dim,
-// include/kfr/dft/fft.hpp:641-690), every axis is transformed as contiguous rows followed by a
-// transpose that rotates the next axis to the end, so each axis reuses the batched 1-D engine (and
-// its power-of-two fast path). Here each transform reads the previous step's array and writes a
-// scratch array that the LDS-tiled transpose turns back into the destination, so every step is one
-// HBM round trip for the transform and one for the transpose.
+// Multidimensional DFTs on device data. The last axis runs as contiguous rows; every other axis whose
+// length fits one workgroup is transformed along its stride by a column kernel, one HBM round trip per
+// axis. Shapes with an axis that needs contiguous transforms go the reference's way
+// (dft_plan_md::execute_dim, include/kfr/dft/fft.hpp:641-690): every axis as contiguous rows, followed by
+// an LDS-tiled transpose that rotates the next axis to the end, a second round trip per axis.
 #include "fft_md.hpp"
 
 #include "fft_core.hpp"
@@ -100,26 +99,80 @@ std::string axis_text(const std::map<size_t, std::unique_ptr<gpu_dft<T>>>& plans
 } // namespace
 
 template <typename T>
+bool axis_set<T>::plan(const std::vector<size_t>& shape, std::map<size_t, std::unique_ptr<gpu_dft<T>>>& plans)
+{
+    long long inner = (long long)shape.back(), total = 1;
+    for (size_t n : shape)
+        total *= (long long)n;
+    hipStream_t s = library_stream();
+    for (size_t i = shape.size() - 1; i-- > 0; inner *= (long long)shape[i])
+    {
+        const size_t n = shape[i];
+        if (n == 1)
+            continue;
+        const long long outer = total / inner / (long long)n;
+        if ((inner & (inner - 1)) == 0 && pow2_fft<T>::supports_axis(n))
+        {
+            auto& p = pow2[n];
+            if (!p)
+                p.reset(new pow2_fft<T>(n, s));
+            list.push_back({ i, n, inner, outer, p.get(), nullptr });
+            continue;
+        }
+        // columns of 64-byte runs and more: below that the transposes, whose runs are 256 bytes
+        if (inner * (long long)sizeof(cx<T>) < 64)
+            return false;
+        auto& g = plans[n];
+        if (!g)
+            g.reset(new gpu_dft<T>(n));
+        if (!g->supports_axis(inner, outer))
+            return false;
+        list.push_back({ i, n, inner, outer, nullptr, g.get() });
+    }
+    hip_check(hipStreamSynchronize(s), "multidimensional plan initialisation");
+    return true;
+}
+
+template <typename T>
+bool axis_set<T>::run(void* out, const void* in, bool inverse, hipStream_t s) const
+{
+    for (const entry& e : list)
+    {
+        if (e.p2)
+        {
+            int l = 0;
+            while ((1ll << l) < e.inner)
+                ++l;
+            e.p2->run_axis(inverse, in, out, l, e.outer, s);
+        }
+        else
+            e.g->execute_axis(out, in, e.inner, e.outer, inverse, s);
+        in = out;
+    }
+    return !list.empty();
+}
+
+template <typename T>
+std::string axis_set<T>::describe(size_t i) const
+{
+    for (const entry& e : list)
+        if (e.axis == i)
+            return "in place along its stride, " + (e.p2 ? e.p2->describe() : e.g->schedule().text());
+    return "identity";
+}
+template class axis_set<float>;
+template class axis_set<double>;
+
+template <typename T>
 gpu_dft_md<T>::gpu_dft_md(const std::vector<size_t>& shape) : sh(shape)
 {
     check_shape(sh);
     total = product(sh);
-    // power-of-two axes of one-kernel length: the axes before the last run in place along their
-    // stride (one HBM round trip per axis, no transposes)
-    strided = (sh.back() & (sh.back() - 1)) == 0;
-    for (size_t i = 0; i + 1 < sh.size(); ++i)
-        strided = strided && (sh[i] == 1 || pow2_fft<T>::supports_axis(sh[i]));
+    if (sh.back() > 1)
+        plans[sh.back()].reset(new gpu_dft<T>(sh.back()));
+    strided = axes.plan(sh, plans);
     if (strided)
-    {
-        if (sh.back() > 1)
-            plans[sh.back()].reset(new gpu_dft<T>(sh.back()));
-        hipStream_t s = library_stream();
-        for (size_t i = 0; i + 1 < sh.size(); ++i)
-            if (sh[i] > 1 && !axis.count(sh[i]))
-                axis[sh[i]].reset(new pow2_fft<T>(sh[i], s));
-        hip_check(hipStreamSynchronize(s), "multidimensional plan initialisation");
         return;
-    }
     for (size_t n : sh)
         if (n > 1 && !plans.count(n))
             plans[n].reset(new gpu_dft<T>(n));
@@ -139,11 +192,9 @@ std::string gpu_dft_md<T>::schedule() const
     if (strided)
     {
         std::string t;
-        for (size_t i = 0; i + 1 < sh.size(); ++i)
-            t += "axis " + std::to_string(i) + " (" + std::to_string(sh[i]) + "): " +
-                 (sh[i] > 1 ? "in place along its stride, " + axis.at(sh[i])->describe() : std::string("identity")) +
-                 "\n";
         const size_t n = sh.size() - 1;
+        for (size_t i = 0; i < n; ++i)
+            t += "axis " + std::to_string(i) + " (" + std::to_string(sh[i]) + "): " + axes.describe(i) + "\n";
         return t + "axis " + std::to_string(n) + " (" + std::to_string(sh.back()) + "): " +
                (sh.back() > 1 ? plans.at(sh.back())->schedule().text() : std::string("identity"));
     }
@@ -160,23 +211,7 @@ void gpu_dft_md<T>::execute(void* out, const void* in, bool inverse, hipStream_t
             plans.at(last)->execute(out, in, (long long)(total / last), inverse, s);
         else if (out != in)
             hip_check(hipMemcpyAsync(out, in, total * sizeof(cx<T>), hipMemcpyDeviceToDevice, s), "copy");
-        int inner_log = 0;
-        for (size_t j = sh.size() - 1; j-- > 0;)
-        {
-            size_t t = sh[j + 1];
-            while (t > 1)
-            {
-                ++inner_log;
-                t >>= 1;
-            }
-            if (sh[j] > 1)
-            {
-                long long outer = 1;
-                for (size_t q = 0; q < j; ++q)
-                    outer *= (long long)sh[q];
-                axis.at(sh[j])->run_axis(inverse, out, out, inner_log, outer, s);
-            }
-        }
+        axes.run(out, out, inverse, s);
         return;
     }
     scratch.ensure(total * sizeof(cx<T>));
@@ -205,6 +240,11 @@ gpu_dft_md_real<T>::gpu_dft_md_real(const std::vector<size_t>& shape) : sh(shape
     rtotal = product(sh);
     last.reset(new gpu_dft_real<T>(sh.back(), 1 /* CCs */));
     ctotal = rtotal / sh.back() * last->complex_size();
+    std::vector<size_t> csh = sh;
+    csh.back()              = last->complex_size();
+    strided                 = axes.plan(csh, plans);
+    if (strided)
+        return;
     for (size_t i = 0; i + 1 < sh.size(); ++i)
         if (sh[i] > 1 && !plans.count(sh[i]))
             plans[sh[i]].reset(new gpu_dft<T>(sh[i]));
@@ -226,18 +266,33 @@ size_t gpu_dft_md_real<T>::complex_size() const
 template <typename T>
 std::string gpu_dft_md_real<T>::schedule() const
 {
-    return axis_text(plans, sh, sh.size() - 1) + "axis " + std::to_string(sh.size() - 1) + " (" +
-           std::to_string(sh.back()) + ", real): " + last->schedule().text() + "\ntranspose after every axis";
+    const std::string lt = "axis " + std::to_string(sh.size() - 1) + " (" + std::to_string(sh.back()) +
+                           ", real): " + last->schedule().text();
+    if (strided)
+    {
+        std::string t;
+        for (size_t i = 0; i + 1 < sh.size(); ++i)
+            t += "axis " + std::to_string(i) + " (" + std::to_string(sh[i]) + "): " + axes.describe(i) + "\n";
+        return t + lt;
+    }
+    return axis_text(plans, sh, sh.size() - 1) + lt + "\ntranspose after every axis";
 }
 
 template <typename T>
 void gpu_dft_md_real<T>::forward(void* cout, const void* rin, hipStream_t s)
 {
     a.ensure(ctotal * sizeof(cx<T>));
-    b.ensure(ctotal * sizeof(cx<T>));
     const size_t ck    = last->complex_size();
     const size_t rows0 = rtotal / sh.back();
+    // through `a`: the spectrum's rows are longer than the real rows, and the caller may pass one buffer
     last->forward(a.ptr, rin, (long long)rows0, s);
+    if (strided)
+    {
+        if (!axes.run(cout, a.ptr, false, s))
+            hip_check(hipMemcpyAsync(cout, a.ptr, ctotal * sizeof(cx<T>), hipMemcpyDeviceToDevice, s), "copy");
+        return;
+    }
+    b.ensure(ctotal * sizeof(cx<T>));
     std::vector<size_t> cur(sh.begin(), sh.end() - 1);
     cur.insert(cur.begin(), ck); // after the transpose: (ck, d0, ..., d_{k-1})
     const size_t naxes = sh.size() - 1;
@@ -260,6 +315,13 @@ template <typename T>
 void gpu_dft_md_real<T>::inverse(void* rout, const void* cin, hipStream_t s)
 {
     a.ensure(ctotal * sizeof(cx<T>));
+    if (strided)
+    {
+        if (!axes.run(a.ptr, cin, true, s))
+            hip_check(hipMemcpyAsync(a.ptr, cin, ctotal * sizeof(cx<T>), hipMemcpyDeviceToDevice, s), "copy");
+        last->inverse(rout, a.ptr, (long long)(rtotal / sh.back()), s);
+        return;
+    }
     b.ensure(ctotal * sizeof(cx<T>));
     const size_t ck    = last->complex_size();
     const size_t naxes = sh.size() - 1;

@@ -58,3 +58,50 @@ def test_mixed_real(n, dt):
     bound = bound_fp64(n, dt)
     assert max(oracle.rel_rms(y[b], ref[b]) for b in range(batch)) <= bound
     assert oracle.rel_rms(zd.cpu().numpy() / n, x) <= 2 * bound
+
+
+# axes transformed along their stride: mixed and power-of-two lengths before odd and narrow dimensions,
+# more and fewer columns than a workgroup takes, batches of arrays, one-pass axes; (97, 33) and (6, 5, 100)
+# run a direct prime pass and a one-pass axis, (30, 12, 4) has an axis below the 64-byte run
+MD_SHAPES = [(1080, 241), (45, 128), (64, 45, 33), (9, 8), (97, 33), (6, 5, 100), (30, 12, 4), (512, 15, 9), (5, 1, 80)]
+
+
+@pytest.mark.parametrize("shape", MD_SHAPES)
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_strided_axes(shape, dtype):
+    torch = pytest.importorskip("torch")
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal((2,) + shape) + 1j * rng.standard_normal((2,) + shape)).astype(dtype)
+    axes = tuple(range(1, len(shape) + 1))
+    p = kfr_amd.dft_plan_md(shape, dtype)
+    xd = torch.from_numpy(x).cuda()
+    for inverse in (False, True):
+        ref = np.fft.ifftn(x.astype(np.complex128), axes=axes) * n if inverse else np.fft.fftn(
+            x.astype(np.complex128), axes=axes)
+        yd = torch.full_like(xd, float("nan"))
+        p.execute_batch(yd, xd, 2, inverse)
+        zd = xd.clone()
+        p.execute_batch(zd, zd, 2, inverse)
+        assert oracle.rel_rms(yd.cpu().numpy(), ref) <= bound_fp64(n, dtype)
+        assert torch.equal(yd, zd)
+
+
+@pytest.mark.parametrize("shape", [(1080, 242), (45, 30, 16), (7, 64, 30), (1, 30)])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_strided_real_axes(shape, dt):
+    torch = pytest.importorskip("torch")
+    n = int(np.prod(shape))
+    x = oracle.gaussian(800 + n, n, dt).reshape(shape)
+    cdt = torch.complex64 if dt == np.float32 else torch.complex128
+    p = kfr_amd.dft_plan_md_real(shape, False, dt)
+    xd = torch.from_numpy(x.copy()).cuda()
+    yd = torch.empty(p.complex_size(), dtype=cdt, device="cuda")
+    keep = torch.full_like(xd, float("nan"))
+    p.execute(yd, xd)
+    spectrum = yd.clone()
+    p.execute(keep, yd)
+    assert torch.equal(yd, spectrum)  # the input spectrum is left as it was
+    bound = bound_fp64(n, dt)
+    assert oracle.rel_rms(yd.cpu().numpy(), np.fft.rfftn(x.astype(np.float64))) <= bound
+    assert oracle.rel_rms(keep.cpu().numpy() / n, x) <= 4 * bound
