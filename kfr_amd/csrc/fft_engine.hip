@@ -557,6 +557,69 @@ __global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) 
     }
 }
 
+// fused inverse real transform for LDS-resident half lengths: the spectrum is unpacked (from_fmt,
+// src/dft/fft-impl.hpp:1853-1896) pair by pair into LDS, both values of a pair from one read of X[k],
+// X[csize-k] and the factor (the load phase of the plain transform read them twice), then the inverse
+// passes run. FS: plain output, written by the last pass itself (mixed radices)
+template <typename T, bool MIXED, bool FS>
+__global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) k_real_inv(lds_geom G, const cx<T>* __restrict__ tw,
+                                                                   long long batch, xload<T> ld, xstore<T> st,
+                                                                   fastdiv ndiv)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    cx<T>* lds            = reinterpret_cast<cx<T>*>(smem_raw);
+    const long long first = (long long)blockIdx.x * G.tpb;
+    const fft_ctx<T, !MIXED> c = make_ctx<!MIXED, T>(G, lds, first, batch);
+    constexpr int U       = stage_values<T> / 2; // pairs in flight per thread
+    const int csize       = G.n;
+    const long long b     = c.g + ld.b0;
+    for (int k0 = c.t; 2 * k0 <= csize; k0 += U * G.tpt)
+    {
+        cx<T> x[U], y[U], w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            const int k = k0 + u * G.tpt;
+            x[u] = y[u] = w[u] = { T(0), T(0) };
+            if (2 * k <= csize && c.valid)
+            {
+                x[u] = ld.spec(b, k);
+                if (k > 0 || ld.flag == 1) // the partner of X[0] is X[csize] (CCs) or none (Perm)
+                    y[u] = ld.spec(b, csize - k);
+                w[u] = ld.r[k];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            const int k = k0 + u * G.tpt;
+            if (2 * k > csize)
+                continue;
+            if (k == 0)
+                c.at(0) = ld.flag == 1 ? cx<T>{ x[u].re + y[u].re, x[u].re - y[u].re }
+                                       : cx<T>{ x[u].re + x[u].im, x[u].re - x[u].im };
+            else if (2 * k == csize)
+                c.at(k) = { T(2) * x[u].re, T(-2) * x[u].im };
+            else
+            {
+                const cx<T> f1 = cadd(x[u], cconj(y[u]));
+                const cx<T> f2 = csub(x[u], cconj(y[u]));
+                const cx<T> t  = cmulc(f2, w[u]);
+                c.at(k)         = cadd(f1, t);
+                c.at(csize - k) = cconj(csub(f1, t));
+            }
+        }
+    }
+    __syncthreads();
+    fft_passes<T, true, MIXED>(G, tw, c, 0, FS ? G.np - 1 : G.np);
+    if constexpr (FS)
+        last_pass<T, true, MIXED>(
+            G, tw, c,
+            to_global<T>{ static_cast<cx<T>*>(st.p) + (c.valid ? c.g + st.b0 : 0) * st.pdist, 1, c.valid });
+    else
+        block_store<!MIXED>(G, lds, first, batch, st, ndiv);
+}
+
 template <typename T>
 struct gpu_dft_real<T>::impl
 {
@@ -672,7 +735,25 @@ struct gpu_dft_real<T>::impl
         if (fused_forward())
         {
             // one workgroup per transform: the unpacking runs in the load phase of the same kernel
-            c->run(src, st, batch, true, s);
+            core_fft<T>& f   = *c->core;
+            lds_geom G       = make_geom(f.S, f.tpb, 0, 1, (int)csize);
+            const size_t sh  = lds_padded_elems((size_t)f.tpb * csize) * sizeof(cx<T>);
+            const bool mx    = is_mixed(f.S);
+            auto go          = [&](auto kernel)
+            {
+                allow_lds(kernel, sh);
+                hipLaunchKernelGGL(kernel, dim3(nblocks(batch, f.tpb)), dim3(f.S.tpt * f.tpb), sh, s, G,
+                                   f.tw.template as<cx<T>>(), batch, src, st, make_fastdiv((uint32_t)csize));
+            };
+            timing::span ts([mx] { return timing::kernel_name("k_real_inv", timing::type_name<T>(), mx); },
+                            2 * (long long)sizeof(cx<T>) * batch * (long long)csize, s);
+            if (!mx)
+                go(k_real_inv<T, false, false>);
+            else if (plain(st) && G.tpt >= 16 && G.np >= 2 && G.pass[G.np - 1].kind == pass_radix)
+                go(k_real_inv<T, true, true>);
+            else
+                go(k_real_inv<T, true, false>);
+            hip_check(hipGetLastError(), "real inverse launch");
             return;
         }
         // Longer lengths: the from_fmt unpacking as a pass of its own into plain half-length
