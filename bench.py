@@ -157,7 +157,7 @@ def uneven_batch(torch, kfr_amd, stream, reps: int, check: bool):
 
 def precision_config(torch, kfr_amd, stream, reps: int):
     """Complex C2C N = 2^20, batch 64, unit-variance complex Gaussian data (seed 4) stored in bfloat16 and
-    binary16 (radix-16 passes on MFMA) against the FP32 path on the same values; errors against the
+    binary16 against the FP32 path on the same values; errors against the
     FP64 transform of the stored input, on 4 sampled transforms."""
     n, batch = 1 << 20, 64
     g = torch.Generator(device="cuda")
@@ -205,16 +205,6 @@ def precision_config(torch, kfr_amd, stream, reps: int):
     for name in ("bf16", "f16"):
         out[name]["speedup_vs_f32"] = round(out["f32"]["ms"] / out[name]["ms"], 3)
     res.update(out)
-    # MFMA utilisation of the half-precision kernels of this workload, from the committed counter run
-    # (rocprofv3 cannot run inside this process); per dispatch, in percent of the chip's SIMD cycles
-    from kfr_amd.rocprof_summary import read_table
-    mfile = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "half_c2c_2p20x64_mfma_counters.md")
-    rows = [r for r in read_table(mfile) if r["kernel"].startswith("k_pow2<float") and r["kernel"].endswith((", 1>", ", 2>"))]
-    if rows:
-        res["mfma_counters"] = {"source": "profiles/half_c2c_2p20x64_mfma_counters.md",
-                                "kernels": {r["kernel"]: {"mfma_util_pct": float(r["MfmaUtil"]),
-                                                          "valu_busy_pct": float(r["VALUBusy"]),
-                                                          "wait_share": float(r["wait share"])} for r in rows}}
     return res
 
 

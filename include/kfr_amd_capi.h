@@ -256,10 +256,8 @@ KFR_AMD_API int kfr_amd_batch_describe(KFR_AMD_BATCH* batch, char* buf, size_t b
 KFR_AMD_API void kfr_amd_batch_delete(KFR_AMD_BATCH* batch);
 
 /* Complex transforms of power-of-two size stored in half precision: each value is a pair (re, im) of
- * bfloat16 (storage 1) or IEEE binary16 (storage 2), 4 bytes per complex value; arithmetic is FP32 and
- * the radix-16 passes run as 16-point DFT-matrix products on MFMA with the matrix and the data split
- * into bf16 hi + lo parts (FP32 accumulation). Transforms longer than one workgroup keep their
- * intermediate in binary16 with a power-of-two scale per group of columns. Unscaled, in place allowed,
+ * bfloat16 (storage 1) or IEEE binary16 (storage 2), 4 bytes per complex value; arithmetic and the
+ * intermediates of transforms longer than one workgroup are FP32. Unscaled, in place allowed,
  * contiguous batches; device pointers run on `stream` without synchronising, host pointers are staged
  * synchronously. No counterpart in the reference (whose transforms are float and double only). */
 typedef struct KFR_AMD_DFT_HALF { int opaque; } KFR_AMD_DFT_HALF;

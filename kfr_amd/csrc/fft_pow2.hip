@@ -26,7 +26,7 @@
 // contiguous output runs through LDS.
 //
 // Half-precision storage (bfloat16 or binary16 pairs, T = float) reuses the same kernels with
-// conversions at load and store; their radix-16 passes run as 16-point DFT-matrix products on MFMA.
+// conversions at load and store; the intermediates of the four-step and multi-pass lengths are f32.
 #include "fft_pow2.hpp"
 #include "fft_timing.hpp"
 
@@ -116,15 +116,16 @@ struct geom
             return 1;
         if (ROLE == role_direct)
             return S1::TPT >= 256 ? 1 : 256 / S1::TPT;
-        // full-precision rows that would exceed the budget exchange in two rounds (ex() below), holding
+        // rows that would exceed the budget exchange in two rounds (ex() below), holding
         // half of each row in LDS at a time: twice the rows per workgroup and twice the run length of
         // the transposed store (measured 2-6% faster for rows of 2^11..2^13 points); the same for the
         // columns of which the budget holds fewer than 16 (f32 2^23 2.5%, f64 2^22 and 2^23 4-7% faster)
-        constexpr int grow = (ROLE == role_row || (ROLE == role_col && 16 * S1::N > lds_budget<T>)) && PREC == 0 &&
+        constexpr int grow = (ROLE == role_row || (ROLE == role_col && 16 * S1::N > lds_budget<T>)) &&
                                      S1::LE >= log_e<T>
                                  ? 2
                                  : 1;
-        // half-precision passes hold 32 butterflies: 128-byte runs of 4-byte values
+        // half-precision passes hold 32 butterflies: 128-byte runs of 4-byte values (32 rows per row
+        // kernel measured within 2% of 16 either way)
         int w = ROLE == role_pass && PREC != 0 ? 32 : 16;
         while (w > 1 && (w * S1::N > grow * lds_budget<T> || w * S1::TPT > grow * 1024))
             w /= 2;
@@ -141,9 +142,8 @@ struct geom
     static constexpr int ex()
     {
         // measured: column kernels of which the budget holds 16 columns (their strided loads, twiddles
-        // and stores hold the most registers) and the half-precision kernels (MFMA operands) run faster
-        // with the full workgroup
-        if (ROLE == role_pass || ROLE == role_conv || PREC != 0 || S1::LE < log_e<T> ||
+        // and stores hold the most registers) run faster with the full workgroup
+        if (ROLE == role_pass || ROLE == role_conv || S1::LE < log_e<T> ||
             (ROLE == role_col && 16 * S1::N <= lds_budget<T>))
             return 1;
         if (ROLE == role_direct || ROLE == role_block) // measured: f64 from 128 threads, f32 from 512
@@ -190,25 +190,22 @@ struct args
     const cx<T>* tw  = nullptr; // pass tables of this kernel's length
     const cx<T>* ta  = nullptr; // four-step: W_n^(h*2^lbits)
     const cx<T>* tb  = nullptr; // four-step: W_n^l, l < 2^lbits
-    int* scales      = nullptr; // half-precision four-step: power-of-two scale of each column group
     long long count  = 0;       // transforms
     int lo           = 0;       // four-step: log2 of the other dimension (col: n1, row: n2)
     int lbits        = 0;
-    int gshift       = 0; // half-precision row kernel: log2 of the column kernel's columns per workgroup
     int ns_log       = 0; // multi-pass: log2 of the stride Ns of this pass (twiddles W_{Ns*R} from ta, tb)
     unsigned nblk    = 0; // workgroups with work (the grid of split kernels is a multiple of 8)
-    // half-precision multi-pass: the input is the previous pass's binary16 intermediate, element o of
-    // item b scaled by in_scales[workgroup of the previous pass that wrote it]; that pass had radix
-    // 2^in_l, stride 2^in_ns and 2^in_wlog butterflies per workgroup
-    const int* in_scales = nullptr;
-    int in_l = 0, in_ns = 0, in_wlog = 0;
-    int out_mid = 0; // write a binary16 intermediate with one power-of-two scale per workgroup (a.scales)
+    // half-precision multi-pass: the input (output) is an f32 intermediate
+    int in_mid = 0, out_mid = 0;
 };
 
 // ---- storage precision of the data in HBM (the arithmetic is T throughout)
 //   prec_full: cx<T>; prec_bf16 / prec_f16: complex values of two bfloat16 / binary16 (T = float only).
-// The half-precision four-step keeps its intermediate as binary16 with one power-of-two scale per
-// column-kernel workgroup, so values of any range keep 11-bit precision.
+// Half-precision lengths beyond one workgroup keep their intermediates in f32. Binary16 intermediates with
+// a power-of-two scale per workgroup, and radix-16 passes as DFT-matrix products on the matrix cores
+// (three bf16 products of split operands), moved two thirds of the bytes but were bound by instructions:
+// bf16 2^20 x 64 took 713 us, 600 us with plain butterflies instead of the products, and 499 us with
+// f32 intermediates; 2^15 x 2048, now in one workgroup, 560 -> 274 us.
 enum storage_prec : int
 {
     prec_full = 0,
@@ -258,142 +255,6 @@ __device__ __forceinline__ void st_elem(void* p, long long i, cx<T> v)
         static_cast<hcx<_Float16>*>(p)[i] = { (_Float16)(float)v.re, (_Float16)(float)v.im };
 }
 
-// precision of the four-step intermediate
-template <int PREC>
-inline constexpr int mid_prec = PREC == prec_full ? prec_full : prec_f16;
-
-// ---- radix-16 butterflies on MFMA (half-precision storage): the 16-point DFT of 32 butterflies is
-// the real product [Re y; Im y] = [[Re F, -Im F], [Im F, Re F]] [Re x; Im x] with the 32x32 matrix as
-// the A operand of v_mfma_f32_32x32x16_bf16 (lane l, slot s: A[l%32][8(l/32)+s]; B[8(l/32)+s][l%32];
-// D slot v: D[8(v/4)+4(l/32)+v%4][l%32]). Matrix and data are each split into bf16 hi + lo parts and
-// three products are accumulated in FP32 (hi*hi + hi*lo + lo*hi), about 16 significant bits.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-struct mfma16
-{
-    bf16x8 a0h, a0l, a1h, a1l; // chunk 0 multiplies Re x, chunk 1 Im x
-};
-
-__device__ __forceinline__ void split_bf16(float x, __bf16& hi, __bf16& lo)
-{
-    hi = (__bf16)x;
-    lo = (__bf16)(x - (float)hi);
-}
-
-template <bool INV>
-__device__ __forceinline__ mfma16 make_mfma16()
-{
-    // cos and sin of 2*pi*q/16
-    constexpr float cq[16] = { (float)ccos2pi(0, 16),  (float)ccos2pi(1, 16),  (float)ccos2pi(2, 16),
-                               (float)ccos2pi(3, 16),  (float)ccos2pi(4, 16),  (float)ccos2pi(5, 16),
-                               (float)ccos2pi(6, 16),  (float)ccos2pi(7, 16),  (float)ccos2pi(8, 16),
-                               (float)ccos2pi(9, 16),  (float)ccos2pi(10, 16), (float)ccos2pi(11, 16),
-                               (float)ccos2pi(12, 16), (float)ccos2pi(13, 16), (float)ccos2pi(14, 16),
-                               (float)ccos2pi(15, 16) };
-    constexpr float sq[16] = { (float)csin2pi(0, 16),  (float)csin2pi(1, 16),  (float)csin2pi(2, 16),
-                               (float)csin2pi(3, 16),  (float)csin2pi(4, 16),  (float)csin2pi(5, 16),
-                               (float)csin2pi(6, 16),  (float)csin2pi(7, 16),  (float)csin2pi(8, 16),
-                               (float)csin2pi(9, 16),  (float)csin2pi(10, 16), (float)csin2pi(11, 16),
-                               (float)csin2pi(12, 16), (float)csin2pi(13, 16), (float)csin2pi(14, 16),
-                               (float)csin2pi(15, 16) };
-    const int l      = __lane_id();
-    const int i      = l & 31;
-    const int h      = l >> 5;
-    const int m      = i & 15;
-    const bool imrow = i >= 16;
-    mfma16 K;
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-    {
-        const int q    = (m * (8 * h + s)) & 15;
-        const float c  = cq[q];
-        const float sg = INV ? -sq[q] : sq[q]; // forward F = cos - i sin
-        // row i < 16: Re y_m = sum c Re x + sg Im x ; row i >= 16: Im y_m = sum -sg Re x + c Im x
-        const float a0 = imrow ? -sg : c;
-        const float a1 = imrow ? c : sg;
-        __bf16 hi, lo;
-        split_bf16(a0, hi, lo);
-        K.a0h[s] = hi;
-        K.a0l[s] = lo;
-        split_bf16(a1, hi, lo);
-        K.a1h[s] = hi;
-        K.a1l[s] = lo;
-    }
-    return K;
-}
-
-// 16-point DFTs of the 32 butterflies whose inputs r in [8h, 8h+8) this lane holds in g
-__device__ __forceinline__ f32x16 mfma16_group(const cx<float> (&g)[8], const mfma16& K)
-{
-    bf16x8 b0h, b0l, b1h, b1l;
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-    {
-        __bf16 hi, lo;
-        split_bf16(g[s].re, hi, lo);
-        b0h[s] = hi;
-        b0l[s] = lo;
-        split_bf16(g[s].im, hi, lo);
-        b1h[s] = hi;
-        b1l[s] = lo;
-    }
-    f32x16 acc = {};
-    acc        = __builtin_amdgcn_mfma_f32_32x32x16_bf16(K.a0h, b0h, acc, 0, 0, 0);
-    acc        = __builtin_amdgcn_mfma_f32_32x32x16_bf16(K.a0h, b0l, acc, 0, 0, 0);
-    acc        = __builtin_amdgcn_mfma_f32_32x32x16_bf16(K.a0l, b0h, acc, 0, 0, 0);
-    acc        = __builtin_amdgcn_mfma_f32_32x32x16_bf16(K.a1h, b1h, acc, 0, 0, 0);
-    acc        = __builtin_amdgcn_mfma_f32_32x32x16_bf16(K.a1h, b1l, acc, 0, 0, 0);
-    acc        = __builtin_amdgcn_mfma_f32_32x32x16_bf16(K.a1l, b1h, acc, 0, 0, 0);
-    return acc;
-}
-
-// v_permlane32_swap on the pair (a, b): the upper half-wave of a and the lower half-wave of b trade
-// places. Lane l < 32 keeps its a and receives the a of lane l + 32 in b; lane l >= 32 keeps its b
-// and receives the b of lane l - 32 in a. One instruction moves both registers.
-__device__ __forceinline__ void swap32(float& a, float& b)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a            = __uint_as_float(r[0]);
-    b            = __uint_as_float(r[1]);
-}
-
-// Wave-cooperative radix-16 butterfly: every lane of the wave holds the 16 inputs of its own
-// butterfly in u and gets its 16 outputs back. Swapping the pair (u[s], u[8+s]) leaves lane l < 32
-// with input s of butterflies l and l + 32, and lane l >= 32 with input 8 + s of butterflies l - 32 and
-// l: inputs [8h, 8h+8) of butterflies l%32 (group 0) and 32 + l%32 (group 1), the B operand layout.
-// Both groups run on MFMA; lane h then holds outputs m(h, q) of both groups, and swapping each pair
-// (group 0, group 1) returns outputs m(0, q) and m(1, q) of its own butterfly to every lane.
-__device__ __forceinline__ void bfly16_mfma(cx<float> (&u)[16], const mfma16& K)
-{
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-    {
-        swap32(u[s].re, u[8 + s].re);
-        swap32(u[s].im, u[8 + s].im);
-    }
-    cx<float> g0[8], g1[8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-    {
-        g0[s] = u[s];
-        g1[s] = u[8 + s];
-    }
-    const f32x16 d0 = mfma16_group(g0, K);
-    const f32x16 d1 = mfma16_group(g1, K);
-    // slot q holds output m = 4h + q (q < 4) or 8 + 4h + q - 4 (q >= 4): Re in d[q], Im in d[8 + q]
-#pragma unroll
-    for (int q = 0; q < 8; ++q)
-    {
-        cx<float> a = { d0[q], d0[8 + q] };
-        cx<float> b = { d1[q], d1[8 + q] };
-        swap32(a.re, b.re);
-        swap32(a.im, b.im);
-        u[q < 4 ? q : 4 + q]     = a; // output m(0, q)
-        u[q < 4 ? 4 + q : 8 + q] = b; // output m(1, q)
-    }
-}
-
 // the thread whose positions feed the second butterfly of thread t in a mirrored last pass
 template <int MODE, int TP>
 __device__ __forceinline__ int mirror_lane(int t)
@@ -412,8 +273,7 @@ __device__ __forceinline__ int mirror_lane(int t)
 // themselves).
 constexpr int mirror_none = 0, mirror_rev = 1, mirror_neg = 2;
 template <typename T, int L, bool INV, int ROLE, int PREC, int P, bool MIRROR0 = false, int MIRRORL = mirror_none>
-__device__ __forceinline__ void run_pass(regs<T, L, ROLE, PREC>& v, cx<T>* lds, int tb, int t, const cx<T>* tw,
-                                         const mfma16& K)
+__device__ __forceinline__ void run_pass(regs<T, L, ROLE, PREC>& v, cx<T>* lds, int tb, int t, const cx<T>* tw)
 {
     using G          = geom<T, L, ROLE, PREC>;
     using S          = typename G::S;
@@ -456,10 +316,7 @@ __device__ __forceinline__ void run_pass(regs<T, L, ROLE, PREC>& v, cx<T>* lds, 
 #pragma unroll
         for (int r = 0; r < R; ++r)
             u[r] = v[m + r * M];
-        if constexpr (PREC != prec_full && R == 16)
-            bfly16_mfma(u, K);
-        else
-            butterfly<R, INV>(u);
+        butterfly<R, INV>(u);
 #pragma unroll
         for (int r = 0; r < R; ++r)
             v[m + r * M] = u[r];
@@ -512,46 +369,12 @@ __device__ __forceinline__ void run_pass(regs<T, L, ROLE, PREC>& v, cx<T>* lds, 
             for (int k = 0; k < E; ++k)
                 v[k] = u[k];
         }
-        run_pass<T, L, INV, ROLE, PREC, P + 1, false, MIRRORL>(v, lds, tb, t, tw, K);
+        run_pass<T, L, INV, ROLE, PREC, P + 1, false, MIRRORL>(v, lds, tb, t, tw);
     }
     static_assert(!MIRROR0 || (P == 0 && NS == 1 && M % 2 == 0 && P + 1 < S::NP),
                   "mirrored first pass: an even number of butterflies");
     static_assert(MIRRORL == mirror_none || (S::NP >= 2 && E / (1 << S::lr(S::NP - 1)) == 2),
                   "mirrored last pass: two butterflies");
-}
-
-// power-of-two scale 2^k of a value array whose largest |re|, |im| is mx: the scaled values stay below
-// 2^15, inside binary16's range
-__device__ __forceinline__ int mid_scale_exp(float mx)
-{
-    int e = 0;
-    (void)frexpf(mx, &e); // mx < 2^e
-    return mx > 0.f ? 15 - e : 0;
-}
-
-// the scale exponent of all values the workgroup holds (every thread calls it): wave maxima, then one
-// value per wave through LDS; the LDS is free again when it returns
-template <typename T, int E, int BS>
-__device__ __forceinline__ int workgroup_scale(const cx<T> (&v)[E], cx<T>* lds)
-{
-    float mx = 0.f;
-#pragma unroll
-    for (int k = 0; k < E; ++k)
-        mx = fmaxf(mx, fmaxf(fabsf((float)v[k].re), fabsf((float)v[k].im)));
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, off));
-    float* red = reinterpret_cast<float*>(lds);
-    lds_barrier();
-    if (__lane_id() == 0)
-        red[threadIdx.x >> 6] = mx;
-    lds_barrier();
-    float bm = 0.f;
-#pragma unroll
-    for (int w = 0; w < (BS + 63) / 64; ++w)
-        bm = fmaxf(bm, red[w]);
-    lds_barrier();
-    return mid_scale_exp(bm);
 }
 
 template <typename T, int L, bool INV, int ROLE, int PREC>
@@ -568,9 +391,6 @@ __global__ void __launch_bounds__((geom<T, L, ROLE, PREC>::BS),
     constexpr int BS = G::BS;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-    mfma16 K{};
-    if constexpr (PREC != prec_full)
-        K = make_mfma16<INV>();
 
     unsigned blk = blockIdx.x;
     if constexpr (ROLE != role_direct)
@@ -620,28 +440,11 @@ __global__ void __launch_bounds__((geom<T, L, ROLE, PREC>::BS),
         const long long bl   = g >> a.lo;
         const long long col  = g & ((1ll << a.lo) - 1);
         const long long base = (bl << (a.lo + L)) + col;
-        bool scaled_in       = false;
-        if constexpr (ROLE == role_pass && PREC != prec_full)
-            scaled_in = a.in_scales != nullptr;
-        if (scaled_in)
+        if (ROLE == role_pass && PREC != prec_full && a.in_mid)
         {
-            // binary16 intermediate of the previous pass: element o was written by its butterfly
-            // j' = (o >> (ns' + l')) << ns' | (o mod 2^ns'), i.e. by workgroup (bl 2^(Ltot - l') + j') >> wlog'
-            const long long nsm = (1ll << a.in_ns) - 1;
 #pragma unroll
             for (int k = 0; k < E; ++k)
-            {
-                v[k] = { T(0), T(0) };
-                if (valid)
-                {
-                    const long long o  = col + ((long long)(t + k * TP) << a.lo);
-                    const long long jp = ((o >> (a.in_ns + a.in_l)) << a.in_ns) | (o & nsm);
-                    const long long gp = (bl << (a.lo + L - a.in_l)) + jp;
-                    const int sc       = a.in_scales[gp >> a.in_wlog];
-                    const cx<T> h      = ld_elem<T, prec_f16>(a.in, base + ((long long)(t + k * TP) << a.lo));
-                    v[k]               = { ldexpf(h.re, -sc), ldexpf(h.im, -sc) };
-                }
-            }
+                v[k] = valid ? ld_elem<T, prec_full>(a.in, base + ((long long)(t + k * TP) << a.lo)) : cx<T>{ T(0), T(0) };
         }
         else
         {
@@ -679,35 +482,16 @@ __global__ void __launch_bounds__((geom<T, L, ROLE, PREC>::BS),
             }
         }
     }
-    else if constexpr (ROLE == role_row && PREC != prec_full)
-    {
-        // binary16 intermediate: element (col = i) carries the scale of its column-kernel workgroup
-        const long long base = g * N;
-#pragma unroll
-        for (int k = 0; k < E; ++k)
-        {
-            v[k] = { T(0), T(0) };
-            if (valid)
-            {
-                const long long e  = base + t + k * TP;
-                const long long bl = g >> a.lo;
-                const long long gc = (bl << L) + t + k * TP; // column (bl, col) over the batch
-                const int sc      = a.scales[gc >> a.gshift];
-                const cx<T> h     = ld_elem<T, prec_f16>(a.in, e);
-                v[k]              = { ldexpf(h.re, -sc), ldexpf(h.im, -sc) };
-            }
-        }
-    }
     else
     {
         const long long base = g * N + t;
 #pragma unroll
         for (int k = 0; k < E; ++k)
-            v[k] = valid ? ld_elem<T, ROLE == role_row ? mid_prec<PREC> : PREC>(a.in, base + k * TP)
+            v[k] = valid ? ld_elem<T, ROLE == role_row ? (int)prec_full : PREC>(a.in, base + k * TP)
                          : cx<T>{ T(0), T(0) };
     }
 
-    run_pass<T, L, INV, ROLE, PREC, 0>(v, lds, tb, t, a.tw, K);
+    run_pass<T, L, INV, ROLE, PREC, 0>(v, lds, tb, t, a.tw);
     // v[k] = X[t + k*TPT]
 
     if constexpr (ROLE == role_direct && G::staged)
@@ -740,30 +524,12 @@ __global__ void __launch_bounds__((geom<T, L, ROLE, PREC>::BS),
     {
         const long long bl  = g >> a.lo;
         const long long col = g & ((1ll << a.lo) - 1);
-        // half precision: an intermediate is written as binary16 scaled by 2^sc, one sc per workgroup
-        int sc = 0;
-        bool mid = false;
-        if constexpr (PREC != prec_full)
-        {
-            mid = a.out_mid != 0;
-            if (mid)
-            {
-                sc = workgroup_scale<T, E, BS>(v, lds);
-                if (tid == 0)
-                    a.scales[blk] = sc;
-            }
-        }
         auto put = [&](long long idx, cx<T> x)
         {
-            if constexpr (PREC != prec_full)
-            {
-                if (mid)
-                {
-                    st_elem<T, prec_f16>(a.out, idx, { ldexpf(x.re, sc), ldexpf(x.im, sc) });
-                    return;
-                }
-            }
-            st_elem<T, PREC, NT>(a.out, idx, x);
+            if (PREC != prec_full && a.out_mid)
+                st_elem<T, prec_full, NT>(a.out, idx, x);
+            else
+                st_elem<T, PREC, NT>(a.out, idx, x);
         };
         if (a.ns_log == 0)
         {
@@ -836,43 +602,11 @@ __global__ void __launch_bounds__((geom<T, L, ROLE, PREC>::BS),
             for (int k = 0; k < E; ++k)
                 v[k] = ctw<INV>(v[k], w[k]);
         }
-        if constexpr (PREC == prec_full)
+        if (valid)
         {
-            if (valid)
-            {
-#pragma unroll
-                for (int k = 0; k < E; ++k)
-                    st_elem<T, PREC, NT>(a.out, base + ((long long)(t + k * TP) << a.lo), v[k]);
-            }
-        }
-        else
-        {
-            // one scale for the workgroup's columns: wave maxima through LDS (free after the passes)
-            float mx = 0.f;
 #pragma unroll
             for (int k = 0; k < E; ++k)
-                mx = fmaxf(mx, fmaxf(fabsf((float)v[k].re), fabsf((float)v[k].im)));
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1)
-                mx = fmaxf(mx, __shfl_xor(mx, off));
-            float* red = reinterpret_cast<float*>(lds);
-            if (__lane_id() == 0)
-                red[tid >> 6] = mx;
-            lds_barrier();
-            float bm = 0.f;
-#pragma unroll
-            for (int w = 0; w < BS / 64; ++w)
-                bm = fmaxf(bm, red[w]);
-            const int sc = mid_scale_exp(bm);
-            if (tid == 0)
-                a.scales[blk] = sc;
-            if (valid)
-            {
-#pragma unroll
-                for (int k = 0; k < E; ++k)
-                    st_elem<T, prec_f16>(a.out, base + ((long long)(t + k * TP) << a.lo),
-                                         { ldexpf(v[k].re, sc), ldexpf(v[k].im, sc) });
-            }
+                st_elem<T, prec_full, NT>(a.out, base + ((long long)(t + k * TP) << a.lo), v[k]);
         }
     }
     else
@@ -953,35 +687,6 @@ void launch_any(bool inv, int L, const args<T>& a, long long count, hipStream_t 
         launch_len<T, true, ROLE, PREC, LO, HI>(L, a, count, s);
     else
         launch_len<T, false, ROLE, PREC, LO, HI>(L, a, count, s);
-}
-
-// columns per workgroup of the column kernel of 2^L points at precision PREC (the row kernel's scale
-// grouping; the full-precision and half-precision column kernels differ in width)
-template <typename T, int PREC, int LO, int HI>
-int col_width(int L)
-{
-    if constexpr (LO <= HI)
-    {
-        if (L == LO)
-            return geom<T, LO, role_col, PREC>::W;
-        return col_width<T, PREC, LO + 1, HI>(L);
-    }
-    else
-        return 1;
-}
-
-// butterflies per workgroup of the multi-pass kernel of radix 2^L
-template <typename T, int PREC, int LO, int HI>
-int pass_width(int L)
-{
-    if constexpr (LO <= HI)
-    {
-        if (L == LO)
-            return geom<T, LO, role_pass, PREC>::W;
-        return pass_width<T, PREC, LO + 1, HI>(L);
-    }
-    else
-        return 1;
 }
 
 // threads per transform of the one-workgroup kernel of 2^L points
@@ -1066,7 +771,6 @@ k_dct2(const T* __restrict__ x, T* __restrict__ y, const cx<T>* __restrict__ tw,
     static_assert(!G::staged && E % 2 == 0 && G::H <= 2, "fused DCT needs whole-thread transforms");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-    const mfma16 K{};
     const int tid     = threadIdx.x;
     const int tb      = tid / TP;
     const int t       = tid % TP;
@@ -1100,7 +804,7 @@ k_dct2(const T* __restrict__ x, T* __restrict__ y, const cx<T>* __restrict__ tw,
                 v[(M0 - 1 - m) + (R0 - 1 - r) * M0] = { q4.d, q4.b };
             }
         }
-        run_pass<T, L, false, role_direct, prec_full, 0, true, ML>(v, lds, tb, fresh(t), tw, K);
+        run_pass<T, L, false, role_direct, prec_full, 0, true, ML>(v, lds, tb, fresh(t), tw);
     }
     else
     {
@@ -1118,7 +822,7 @@ k_dct2(const T* __restrict__ x, T* __restrict__ y, const cx<T>* __restrict__ tw,
         for (int k = E / 2; k < E; ++k)
             v[k] = at((k - E / 2) * TP + t);
         lds_barrier();
-        run_pass<T, L, false, role_direct, prec_full, 0, false, ML>(v, lds, tb, fresh(t), tw, K);
+        run_pass<T, L, false, role_direct, prec_full, 0, false, ML>(v, lds, tb, fresh(t), tw);
     }
     // v[k] = Z[t + k TPT]. Output pair i, n - i needs Z[i] and Z[N - i] (Z[0] for i = 0).
     T* yb     = y + g * n;
@@ -1234,7 +938,6 @@ k_dct3(const T* __restrict__ y, T* __restrict__ x, const cx<T>* __restrict__ tw,
     static_assert(!G::staged && E % 2 == 0 && G::H <= 2, "fused DCT needs whole-thread transforms");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-    const mfma16 K{};
     const int tid     = threadIdx.x;
     const int tb      = tid / TP;
     const int t       = tid % TP;
@@ -1317,7 +1020,7 @@ k_dct3(const T* __restrict__ y, T* __restrict__ x, const cx<T>* __restrict__ tw,
         // u[j_m + 2r TPT] (j_0 = t, j_1 = 2 TPT-1-t), and u[N-1-q] of q = j_m + 2r TPT is output R-1-r
         // of the other butterfly, so every quad leaves from registers
         constexpr int R = E / 2;
-        run_pass<T, L, true, role_direct, prec_full, 0, false, mirror_rev>(v, lds, tb, fresh(t), tw, K);
+        run_pass<T, L, true, role_direct, prec_full, 0, false, mirror_rev>(v, lds, tb, fresh(t), tw);
         if (!valid)
             return;
         const int ts = fresh(t);
@@ -1332,7 +1035,7 @@ k_dct3(const T* __restrict__ y, T* __restrict__ x, const cx<T>* __restrict__ tw,
     }
     else
     {
-        run_pass<T, L, true, role_direct, prec_full, 0>(v, lds, tb, fresh(t), tw, K);
+        run_pass<T, L, true, role_direct, prec_full, 0>(v, lds, tb, fresh(t), tw);
         // v[k] = u[t + k TPT]; the upper half of the slots crosses to the lower half in mirror order
         const int ts = fresh(t);
 #pragma unroll
@@ -1432,7 +1135,6 @@ k_rfft_fwd(const cx<T>* __restrict__ x, cx<T>* __restrict__ out, long long odist
     static_assert(!G::staged && E % 2 == 0 && G::H <= 2, "fused real transform needs whole-thread transforms");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-    const mfma16 K{};
     const int tid     = threadIdx.x;
     const int tb      = tid / TP;
     const int t       = tid % TP;
@@ -1444,7 +1146,7 @@ k_rfft_fwd(const cx<T>* __restrict__ x, cx<T>* __restrict__ out, long long odist
 #pragma unroll
     for (int k = 0; k < E; ++k)
         v[k] = valid ? xb[k * TP] : cx<T>{ T(0), T(0) };
-    run_pass<T, L, false, role_direct, prec_full, 0>(v, lds, tb, fresh(t), tw, K);
+    run_pass<T, L, false, role_direct, prec_full, 0>(v, lds, tb, fresh(t), tw);
     cx<T>* o  = out + g * odist;
     // X[0] (and X[N]) from Z[0]
     auto emit_ends = [&](cx<T> a)
@@ -1514,7 +1216,6 @@ k_rfft_inv(const cx<T>* __restrict__ spec, long long idist, cx<T>* __restrict__ 
     static_assert(!G::staged && E % 2 == 0 && G::H <= 2, "fused real transform needs whole-thread transforms");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-    const mfma16 K{};
     const int tid     = threadIdx.x;
     const int tb      = tid / TP;
     const int t       = tid % TP;
@@ -1578,7 +1279,7 @@ k_rfft_inv(const cx<T>* __restrict__ spec, long long idist, cx<T>* __restrict__ 
         v[k]        = i == HN ? unpack(HN, v[k], v[k]) : at(i - HN);
     }
     lds_barrier();
-    run_pass<T, L, true, role_direct, prec_full, 0>(v, lds, tb, t, tw, K);
+    run_pass<T, L, true, role_direct, prec_full, 0>(v, lds, tb, t, tw);
     if (valid)
     {
         cx<T>* yb = y + g * N + t;
@@ -1670,7 +1371,6 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_os(conv_o
     constexpr int TP = S::TPT;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-    const mfma16 K{};
     const long long w = blockIdx.x;
     if (w >= a.count)
         return;
@@ -1690,7 +1390,7 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_os(conv_o
         v[k].re = (pa >= 0 && pa < a.nu) ? u[pa] : T(0);
         v[k].im = (pb >= 0 && pb < a.nu) ? u[pb] : T(0);
     }
-    run_pass<T, L, false, role_block, prec_full, 0>(v, lds, 0, t, a.tw, K);
+    run_pass<T, L, false, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
     // v[k] = Z[t + k*TPT]
     const cx<T>* H = a.H + item * a.hd;
 #pragma unroll
@@ -1700,7 +1400,7 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_os(conv_o
         const cx<T> p = cmul(v[k], h);
         v[k]          = { p.re * a.scale, p.im * a.scale };
     }
-    run_pass<T, L, true, role_block, prec_full, 0>(v, lds, 0, t, a.tw, K);
+    run_pass<T, L, true, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
     T* y = a.y + item * a.dy;
 #pragma unroll
     for (int k = 0; k < E; ++k)
@@ -1749,7 +1449,6 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_xcorr(xco
     static_assert(E % 2 == 0 && G::H <= 2, "mirror exchange in halves");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-    const mfma16 K{};
     const long long w = blockIdx.x;
     if (w >= a.count)
         return;
@@ -1769,7 +1468,7 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_xcorr(xco
         v[k].re           = (n < a.P && p < a.nx) ? x[p] : T(0);
         v[k].im           = p < a.ng ? g[p] : T(0);
     }
-    run_pass<T, L, false, role_block, prec_full, 0>(v, lds, 0, t, a.tw, K);
+    run_pass<T, L, false, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
     // v[k] = Z[i], i = t + k*TPT. R[i] = G[i] conj(X[i]) / N needs Z[N - i]. X and G are spectra of
     // real signals, so R[N - i] = conj(R[i]): the upper slots (i >= N/2) publish Z, each lower slot
     // reads its partner, forms R[i] and leaves conj(R[i]) = R[N - i] in the position it read, and the
@@ -1806,7 +1505,7 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_xcorr(xco
         v[k]        = i == HN ? prod(v[k], v[k]) : at(i - HN);
     }
     lds_barrier();
-    run_pass<T, L, true, role_block, prec_full, 0>(v, lds, 0, t, a.tw, K);
+    run_pass<T, L, true, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
     T* out = a.part + w * a.nh;
 #pragma unroll
     for (int k = 0; k < E; ++k)
@@ -1918,8 +1617,7 @@ struct pow2_fft<T>::impl
     int lbits = 0;
     dev_mem tw;
     long long o_row = 0, o_ta = 0, o_tb = 0;
-    dev_mem scratch, scales;
-    int gshift      = 0;
+    dev_mem scratch;
     long long chunk = 1;
     // multi-pass Stockham over HBM (long lengths): log2 radix of every pass, its sub-DFT tables and
     // its W_{Ns*R} two-level tables
@@ -1950,7 +1648,7 @@ pow2_fft<T>::pow2_fft(size_t n, hipStream_t s, int prec) : p(new impl)
     const int le = p2::log_e<T>;
     p->L         = L;
     p->prec      = prec;
-    if (L <= (prec == p2::prec_full ? p2::direct_max_log<T> : p2::max_log<T>))
+    if (L <= p2::direct_max_log<T>)
     {
         const int cnt = p2::pass_twoff(L, le, p2::pass_count(L, le));
         p->tw.reset((size_t)std::max(1, cnt) * sizeof(cx<T>));
@@ -1964,10 +1662,8 @@ pow2_fft<T>::pow2_fft(size_t n, hipStream_t s, int prec) : p(new impl)
     int mp_min = 24;
     if (const char* e = std::getenv("KFR_AMD_MULTIPASS_MIN_LOG"))
         mp_min = atoi(e);
-    // half-precision storage: the multi-pass kernels (32 butterflies per workgroup, 128-byte runs of
-    // 4-byte values) take 2^24 points, where they beat the four-step (0.94 against 1.00 ms per
-    // 256 MiB of bf16 data); from 2^17 to 2^23 the four-step's two passes are 30-50% faster than
-    // three multi-pass passes, whose kernels are bound by instructions, not bytes.
+    // half-precision storage: the same threshold (bf16 2^24 x 4 0.66 ms; below it three passes move more
+    // bytes than two)
     // KFR_AMD_HALF_MULTIPASS_MIN_LOG moves the threshold.
     int half_mp_min = 24;
     if (const char* e = std::getenv("KFR_AMD_HALF_MULTIPASS_MIN_LOG"))
@@ -2012,8 +1708,7 @@ pow2_fft<T>::pow2_fft(size_t n, hipStream_t s, int prec) : p(new impl)
         size_t cap = (size_t)1 << 30; // rounds of at most 1 GiB, as the four-step below
         if (const char* e = std::getenv("KFR_AMD_FOURSTEP_CHUNK_MB"))
             cap = (size_t)std::max(1, atoi(e)) << 20;
-        const size_t mid = prec == p2::prec_full ? sizeof(cx<T>) : 2 * sizeof(_Float16);
-        p->chunk         = (long long)std::max<size_t>(1, cap / (n * mid));
+        p->chunk = (long long)std::max<size_t>(1, cap / (n * sizeof(cx<T>)));
         return;
     }
     p->four = true;
@@ -2030,8 +1725,12 @@ pow2_fft<T>::pow2_fft(size_t n, hipStream_t s, int prec) : p(new impl)
         if (sizeof(T) == 8 && L >= 14 && L <= 22)
             p->L2 = best_f64[L - 14];
     }
-    else if (L == 20)
-        p->L2 = 12; // half precision, 2^20: measured 6% faster than 2^10 x 2^10
+    else if (L >= 16 && L <= 23)
+    {
+        // half-precision storage, the same sweep (2^20 x 64: 499 us with 2^11-point columns, 512 with 2^8)
+        static constexpr int best_half[] = { 7, 9, 10, 10, 11, 10, 10, 11 };
+        p->L2                            = best_half[L - 16];
+    }
     if (const char* e = std::getenv("KFR_AMD_FOURSTEP_L2"))
         p->L2 = std::atoi(e);
     p->L2 = std::min(std::max(p->L2, std::max(p2::min_split_log, L - p2::max_log<T>)),
@@ -2051,19 +1750,13 @@ pow2_fft<T>::pow2_fft(size_t n, hipStream_t s, int prec) : p(new impl)
     p2::gen_pass_tables<T>(p->L1, t + p->o_row, s);
     gen_twiddles(t + p->o_ta, nTA, (long long)n, nTB, 0, tw_linear, 0, s);
     gen_twiddles(t + p->o_tb, nTB, (long long)n, 1, 0, tw_linear, 0, s);
-    // binary16 and bfloat16 storage share one geometry
-    int w = prec == p2::prec_full ? p2::col_width<T, p2::prec_full, p2::min_split_log, p2::max_log<T>>(p->L2)
-                                  : p2::col_width<T, p2::prec_bf16, p2::min_split_log, p2::max_log<T>>(p->L2);
-    while ((1 << p->gshift) < w)
-        ++p->gshift;
     // rounds of at most 1 GiB of intermediate: few launches and round boundaries (measured 4-16% faster
     // than 512 MiB rounds from 2^20 up, which were faster than rounds small enough to stay in the
     // last-level cache), bounded scratch
     size_t cap = (size_t)1 << 30;
     if (const char* e = std::getenv("KFR_AMD_FOURSTEP_CHUNK_MB"))
         cap = (size_t)std::max(1, atoi(e)) << 20;
-    const size_t mid = prec == p2::prec_full ? sizeof(cx<T>) : 2 * sizeof(_Float16);
-    p->chunk         = (long long)std::max<size_t>(1, cap / (n * mid));
+    p->chunk = (long long)std::max<size_t>(1, cap / (n * sizeof(cx<T>)));
 }
 
 template <typename T>
@@ -2077,104 +1770,56 @@ void pow2_fft<T>::impl::run(bool inverse, const void* in, void* out, long long b
     constexpr int ML = p2::max_log<T>;
     const size_t es  = PREC == p2::prec_full ? sizeof(cx<T>) : 2 * sizeof(_Float16); // HBM element size
     const cx<T>* t   = tw.template as<cx<T>>();
-    if constexpr (PREC != p2::prec_full)
+    if (multi)
     {
-        if (multi)
+        if (w.p && PREC != p2::prec_full)
+            throw std::logic_error("half-precision transforms keep their own intermediate");
+        const long long n     = 1ll << L;
+        const int nbuf        = mp_log.size() > 2 ? 2 : 1;
+        const long long chunk = rounds_in(w, this->chunk, (size_t)n * sizeof(cx<T>), nbuf);
+        void* buf[2]          = { nullptr, nullptr };
+        if (w.p)
         {
-            // binary16 intermediates, one power-of-two scale per workgroup, ping-pong between two
-            // buffers (and two scale arrays)
-            if (w.p)
-                throw std::logic_error("half-precision transforms keep their own intermediate");
-            const long long n = 1ll << L;
-            const int np      = (int)mp_log.size();
-            const int nbuf    = np > 2 ? 2 : 1;
-            const long long c = std::min(chunk, batch);
-            scratch.ensure((size_t)c * n * es);
+            buf[0] = workspace_part(w, 0, nbuf);
+            buf[1] = nbuf > 1 ? workspace_part(w, 1, nbuf) : nullptr;
+        }
+        else
+        {
+            const size_t bytes = (size_t)std::min(chunk, batch) * n * sizeof(cx<T>);
+            scratch.ensure(bytes);
             if (nbuf > 1)
-                scratch2.ensure((size_t)c * n * es);
-            long long maxwg = 1;
-            for (int q = 0; q + 1 < np; ++q)
-                maxwg = std::max(maxwg, ((c << (L - mp_log[q])) + 31) / p2::pass_width<T, PREC, 5, 8>(mp_log[q]) + 1);
-            scales.ensure((size_t)(2 * maxwg) * sizeof(int));
-            void* buf[2] = { scratch.ptr, scratch2.ptr };
-            int* scb[2]  = { scales.template as<int>(), scales.template as<int>() + maxwg };
-            for (long long b0 = 0; b0 < batch; b0 += chunk)
-            {
-                const long long nb = std::min(chunk, batch - b0);
-                int nsl = 0, prev_l = 0, prev_ns = 0, prev_w = 0;
-                for (int q = 0; q < np; ++q)
-                {
-                    const int l = mp_log[q];
-                    args<T> a;
-                    a.in        = q == 0 ? static_cast<const char*>(in) + b0 * n * es : buf[(q - 1) & 1];
-                    a.out       = q == np - 1 ? static_cast<char*>(out) + b0 * n * es : buf[q & 1];
-                    a.tw        = t + mp_tw[q];
-                    a.ta        = t + mp_ta[q];
-                    a.tb        = t + mp_tb[q];
-                    a.lbits     = mp_lbits[q];
-                    a.lo        = L - l;
-                    a.ns_log    = nsl;
-                    a.out_mid   = q + 1 < np ? 1 : 0;
-                    a.scales    = q + 1 < np ? scb[q & 1] : nullptr;
-                    a.in_scales = q > 0 ? scb[(q - 1) & 1] : nullptr;
-                    a.in_l      = prev_l;
-                    a.in_ns     = prev_ns;
-                    a.in_wlog   = prev_w;
-                    p2::launch_any<T, role_pass, PREC, 5, 8>(inverse, l, a, nb << (L - l), s);
-                    prev_l  = l;
-                    prev_ns = nsl;
-                    prev_w  = p2::ilog2c(p2::pass_width<T, PREC, 5, 8>(l));
-                    nsl += l;
-                }
-            }
-            return;
+                scratch2.ensure(bytes);
+            buf[0] = scratch.ptr;
+            buf[1] = scratch2.ptr;
         }
-    }
-    if constexpr (PREC == p2::prec_full)
-    {
-        if (multi)
+        const int np = (int)mp_log.size();
+        for (long long b0 = 0; b0 < batch; b0 += chunk)
         {
-            const long long n     = 1ll << L;
-            const int nbuf        = mp_log.size() > 2 ? 2 : 1;
-            const long long chunk = rounds_in(w, this->chunk, (size_t)n * sizeof(cx<T>), nbuf);
-            void* buf[2]          = { nullptr, nullptr };
-            if (w.p)
+            const long long nb = std::min(chunk, batch - b0);
+            int nsl            = 0;
+            for (int q = 0; q < np; ++q)
             {
-                buf[0] = workspace_part(w, 0, nbuf);
-                buf[1] = nbuf > 1 ? workspace_part(w, 1, nbuf) : nullptr;
-            }
-            else
-            {
-                const size_t bytes = (size_t)std::min(chunk, batch) * n * sizeof(cx<T>);
-                scratch.ensure(bytes);
-                if (nbuf > 1)
-                    scratch2.ensure(bytes);
-                buf[0] = scratch.ptr;
-                buf[1] = scratch2.ptr;
-            }
-            const int np = (int)mp_log.size();
-            for (long long b0 = 0; b0 < batch; b0 += chunk)
-            {
-                const long long nb = std::min(chunk, batch - b0);
-                int nsl            = 0;
-                for (int q = 0; q < np; ++q)
-                {
-                    const int l = mp_log[q];
-                    args<T> a;
-                    a.in     = q == 0 ? static_cast<const char*>(in) + b0 * n * es : buf[(q - 1) & 1];
-                    a.out    = q == np - 1 ? static_cast<char*>(out) + b0 * n * es : buf[q & 1];
-                    a.tw     = t + mp_tw[q];
-                    a.ta     = t + mp_ta[q];
-                    a.tb     = t + mp_tb[q];
-                    a.lbits  = mp_lbits[q];
-                    a.lo     = L - l;
-                    a.ns_log = nsl;
+                const int l = mp_log[q];
+                args<T> a;
+                a.in     = q == 0 ? static_cast<const char*>(in) + b0 * n * es : buf[(q - 1) & 1];
+                a.out    = q == np - 1 ? static_cast<char*>(out) + b0 * n * es : buf[q & 1];
+                a.tw     = t + mp_tw[q];
+                a.ta     = t + mp_ta[q];
+                a.tb     = t + mp_tb[q];
+                a.lbits  = mp_lbits[q];
+                a.lo     = L - l;
+                a.ns_log = nsl;
+                a.in_mid  = q > 0 ? 1 : 0;
+                a.out_mid = q + 1 < np ? 1 : 0;
+                // half-precision storage: f32 intermediates, so the middle passes are the f32 kernels
+                if (q > 0 && q + 1 < np)
+                    p2::launch_any<T, role_pass, p2::prec_full, 5, 8>(inverse, l, a, nb << (L - l), s);
+                else
                     p2::launch_any<T, role_pass, PREC, 5, 8>(inverse, l, a, nb << (L - l), s);
-                    nsl += l;
-                }
+                nsl += l;
             }
-            return;
         }
+        return;
     }
     if (!four)
     {
@@ -2182,12 +1827,11 @@ void pow2_fft<T>::impl::run(bool inverse, const void* in, void* out, long long b
         a.in  = in;
         a.out = out;
         a.tw  = t;
-        constexpr int DL = PREC == p2::prec_full ? p2::direct_max_log<T> : ML;
-        p2::launch_any<T, role_direct, PREC, 1, DL>(inverse, L, a, batch, s);
+        p2::launch_any<T, role_direct, PREC, 1, p2::direct_max_log<T>>(inverse, L, a, batch, s);
         return;
     }
     const long long n = 1ll << L;
-    const size_t mid  = PREC == p2::prec_full ? sizeof(cx<T>) : 2 * sizeof(_Float16);
+    const size_t mid  = sizeof(cx<T>);
     if (w.p && PREC != p2::prec_full)
         throw std::logic_error("half-precision transforms keep their own intermediate");
     const long long chunk = rounds_in(w, this->chunk, (size_t)n * mid, 1);
@@ -2197,8 +1841,6 @@ void pow2_fft<T>::impl::run(bool inverse, const void* in, void* out, long long b
         scratch.ensure((size_t)std::min(chunk, batch) * n * mid);
         midbuf = scratch.ptr;
     }
-    if (PREC != p2::prec_full)
-        scales.ensure((size_t)(std::min(chunk, batch) << L1 >> gshift) * sizeof(int));
     for (long long b0 = 0; b0 < batch; b0 += chunk)
     {
         const long long nb = std::min(chunk, batch - b0);
@@ -2206,8 +1848,6 @@ void pow2_fft<T>::impl::run(bool inverse, const void* in, void* out, long long b
         a.ta     = t + o_ta;
         a.tb     = t + o_tb;
         a.lbits  = lbits;
-        a.scales = scales.template as<int>();
-        a.gshift = gshift;
         a.in     = static_cast<const char*>(in) + b0 * n * es;
         a.out    = midbuf;
         a.tw     = t;
@@ -2305,8 +1945,8 @@ std::string pow2_fft<T>::describe() const
             r += (q ? "x" : "") + std::to_string(1 << p2::pass_lr(L, le, q));
         return r;
     };
-    const std::string pr = p->prec == p2::prec_bf16 ? " storage=bf16 radix16=mfma"
-                           : p->prec == p2::prec_f16 ? " storage=f16 radix16=mfma"
+    const std::string pr = p->prec == p2::prec_bf16 ? " storage=bf16"
+                           : p->prec == p2::prec_f16 ? " storage=f16"
                                                       : "";
     if (p->multi)
     {
@@ -2316,15 +1956,14 @@ std::string pow2_fft<T>::describe() const
         const int w = p->prec == p2::prec_full ? 16 : 32;
         return "pow2 multi-pass radices=" + r + " (" + std::to_string(w) +
                " butterflies per workgroup, one HBM pass each) chunk=" + std::to_string(p->chunk) + pr +
-               (p->prec != p2::prec_full ? " intermediate=f16 scaled per workgroup" : "");
+               (p->prec != p2::prec_full ? " intermediate=f32" : "");
     }
     if (!p->four)
         return "pow2 radices=" + radices(p->L) + " threads/transform=" +
                std::to_string(p2::direct_threads<T, 1, p2::direct_max_log<T>>(p->L)) + pr;
     return "pow2 four-step n1=" + std::to_string(1ll << p->L1) + " n2=" + std::to_string(1ll << p->L2) +
            " radices=" + radices(p->L2) + "|" + radices(p->L1) + " chunk=" + std::to_string(p->chunk) + pr +
-           (p->prec != p2::prec_full ? " intermediate=f16 scaled per " + std::to_string(1 << p->gshift) + " columns"
-                                     : "");
+           (p->prec != p2::prec_full ? " intermediate=f32" : "");
 }
 
 template class pow2_fft<float>;

@@ -18,8 +18,7 @@ public:
     // true for N = 2^L that one kernel (L <= 15 for f32, 14 for f64), the two-kernel four-step split
     // (up to twice that) or the multi-pass Stockham over HBM (the longest lengths) covers
     static bool supports(size_t n);
-    // prec: storage of the data in HBM, 0 = complex T, 1 = bfloat16 pairs, 2 = binary16 pairs (T = float,
-    // radix-16 passes on MFMA)
+    // prec: storage of the data in HBM, 0 = complex T, 1 = bfloat16 pairs, 2 = binary16 pairs (T = float)
     pow2_fft(size_t n, hipStream_t s, int prec = 0);
     ~pow2_fft();
     // batch transforms: in and out hold batch*n complex values each, item b at offset b*n; in == out

@@ -444,7 +444,7 @@ class dft_batch:
 
 class dft_plan_half:
     """Complex DFT of a power-of-two size on half-precision data (kfr_amd_dft_half_*): pairs of
-    bfloat16 (storage "bf16") or binary16 ("f16"), computed in FP32 with the radix-16 passes on MFMA.
+    bfloat16 (storage "bf16") or binary16 ("f16"), computed in FP32.
     Buffers are torch tensors (torch.bfloat16 / torch.float16, interleaved re, im) or any array of
     4-byte complex values. No counterpart in the reference."""
 
