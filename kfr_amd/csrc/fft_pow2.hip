@@ -1344,7 +1344,10 @@ bool rfft_any(int L, const cx<T>* in, long long idist, cx<T>* out, long long odi
 // workgroup takes two adjacent segments of one signal as the real and imaginary parts of one complex
 // sequence (f is real, so both convolutions come out separated), runs the forward transform, the
 // product with the filter spectrum, and the inverse transform in registers and LDS, and writes
-// the valid outputs: every signal value is read (N / lv) times and every output written once.
+// the valid outputs: every signal value is read (N / lv) times and every output written once. Compiled for
+// the two workgroups per CU that its LDS allows (128 VGPRs; 240 without the bound), with 32-bit bounds and
+// the filter spectrum in groups, so that few values are held beside the transform: 2^20 x 128 with 4095 taps
+// 553 -> 500 us per call. The arithmetic of its two transforms alone is about 350 us.
 template <typename T>
 struct conv_os_args
 {
@@ -1363,8 +1366,12 @@ struct conv_os_args
     T scale          = T(1); // 1 / N
 };
 
+// values of one group of the spectrum product (k_conv_os)
+constexpr int conv_group = 8;
+
 template <typename T, int L>
-__global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_os(conv_os_args<T> a)
+__global__ void __launch_bounds__((geom<T, L, role_block>::BS), (geom<T, L, role_block>::lds_waves))
+k_conv_os(conv_os_args<T> a)
 {
     using S          = typename geom<T, L, role_block>::S;
     constexpr int E  = S::E;
@@ -1379,51 +1386,69 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_os(conv_o
     const int t          = threadIdx.x;
     const T* u           = a.u + item * a.du;
     const long long sa   = 2 * pair;
-    const long long ia   = a.o0 + sa * a.lv - (a.nf - 1); // input index of z[0], first segment
-    const long long ib   = ia + a.lv;                      // second segment
+    // z[n] of the first segment is u[ia + n], of the second u[ia + lv + n]: valid for n in
+    // [-ia, nu - ia) and [-ib, nu - ib), as 32-bit bounds
+    const long long ia = a.o0 + sa * a.lv - (a.nf - 1);
+    const long long ib = ia + a.lv;
+    auto bound         = [](long long v) { return (int)(v < 0 ? 0 : v > (1 << L) ? (1 << L) : v); };
+    const int la = bound(-ia), ha = bound(a.nu - ia), lb = bound(-ib), hb = bound(a.nu - ib);
+    const T *ua = u + ia, *ub = u + ib;
     cx<T> v[E];
 #pragma unroll
     for (int k = 0; k < E; ++k)
     {
-        const long long n = t + k * TP;
-        const long long pa = ia + n, pb = ib + n;
-        v[k].re = (pa >= 0 && pa < a.nu) ? u[pa] : T(0);
-        v[k].im = (pb >= 0 && pb < a.nu) ? u[pb] : T(0);
+        const int n = t + k * TP;
+        v[k].re = (n >= la && n < ha) ? ua[n] : T(0);
+        v[k].im = (n >= lb && n < hb) ? ub[n] : T(0);
     }
-    run_pass<T, L, false, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
-    // v[k] = Z[t + k*TPT]
+    run_pass<T, L, false, role_block, prec_full, 0>(v, lds, 0, fresh(t), a.tw);
+    // v[k] = Z[t + k*TPT]. The product with the filter spectrum in groups of conv_group values, each group's
+    // loads from a fresh copy of t: all E factors at once would take twice the registers of v.
     const cx<T>* H = a.H + item * a.hd;
 #pragma unroll
-    for (int k = 0; k < E; ++k)
+    for (int k0 = 0; k0 < E; k0 += conv_group)
     {
-        const cx<T> h = H[t + k * TP];
-        const cx<T> p = cmul(v[k], h);
-        v[k]          = { p.re * a.scale, p.im * a.scale };
+        const int th = fresh(t);
+#pragma unroll
+        for (int k = k0; k < k0 + conv_group && k < E; ++k)
+        {
+            const cx<T> p = cmul(v[k], H[th + k * TP]);
+            v[k]          = { p.re * a.scale, p.im * a.scale };
+        }
+#pragma unroll
+        for (int k = k0; k < k0 + conv_group && k < E; ++k)
+            settle(v[k]);
     }
-    run_pass<T, L, true, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
-    T* y = a.y + item * a.dy;
+    run_pass<T, L, true, role_block, prec_full, 0>(v, lds, 0, fresh(t), a.tw);
+    // output sa*lv + n - (nf-1) and lv further, for n >= nf-1
+    const long long oa = sa * a.lv - (a.nf - 1);
+    T* y               = a.y + item * a.dy + oa;
+    const int ea = bound(a.nout - oa), eb = bound(a.nout - oa - a.lv);
+    const int ts = fresh(t);
 #pragma unroll
     for (int k = 0; k < E; ++k)
     {
-        const int n = t + k * TP;
+        const int n = ts + k * TP;
         if (n >= a.nf - 1)
         {
-            const long long j  = n - (a.nf - 1);
-            const long long ma = sa * a.lv + j;
-            const long long mb = ma + a.lv;
-            if (ma < a.nout)
-                y[ma] = v[k].re;
-            if (mb < a.nout)
-                y[mb] = v[k].im;
+            if (n < ea)
+                y[n] = v[k].re;
+            if (n < eb)
+                y[a.lv + n] = v[k].im;
         }
     }
 }
 
 // Partial cross-correlations for the filter gradient: segment s of length P = N - nh + 1 of item b
-// gives part[(b*nseg + s)*nh + j] = sum_{i<P} g[sP + i + j] x[sP + i], j < nh. One complex transform
-// of z = x_s + i g_s (x zero beyond P) gives both spectra, X = (Z(k) + conj Z(-k))/2 and
-// G = (Z(k) - conj Z(-k))/(2i); the inverse transform of G conj(X) is the circular correlation, which
-// does not wrap for j < nh because P + nh - 1 = N.
+// contributes sum_{i<P} g[sP + i + j] x[sP + i], j < nh. One complex transform of z = x_s + i g_s (x zero
+// beyond P) gives both spectra, X = (Z(k) + conj Z(-k))/2 and G = (Z(k) - conj Z(-k))/(2i); the inverse
+// transform of G conj(X) is the circular correlation, which does not wrap for j < nh because
+// P + nh - 1 = N. A workgroup takes `per` adjacent segments of an item and adds their products before the
+// one inverse transform, part[w*nh + j]: 128 signals of 2^20 samples and 4095 taps run 86 forward and 8
+// inverse transforms each instead of 86 of both, and 8 partial results instead of 86. With the sums in
+// registers, whole-length LDS and 1024 threads at 2^14 points (92 VGPRs) the kernel takes 656 us (978
+// with one segment per workgroup; 755 at 512 threads in 128 VGPRs, which spill the sums, and 657 in 166;
+// 751 with the next segment's loads issued ahead), its arithmetic alone about 350.
 template <typename T>
 struct xcorr_args
 {
@@ -1432,15 +1457,16 @@ struct xcorr_args
     T* part         = nullptr;
     const cx<T>* tw = nullptr;
     long long dx = 0, dg = 0, nx = 0, ng = 0;
-    long long nseg  = 0, count = 0;
-    int P = 1, nh = 1;
+    long long nseg = 0, groups = 0, count = 0; // segments and workgroups per item, workgroups
+    int P = 1, nh = 1, per = 1;
     T scale = T(1); // 1 / N
 };
 
 template <typename T, int L>
-__global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_xcorr(xcorr_args<T> a)
+__global__ void __launch_bounds__((geom<T, L, role_conv>::BS), (geom<T, L, role_conv>::lds_waves))
+k_conv_xcorr(xcorr_args<T> a)
 {
-    using G          = geom<T, L, role_block>;
+    using G          = geom<T, L, role_conv>;
     using S          = typename G::S;
     constexpr int N  = S::N;
     constexpr int E  = S::E;
@@ -1452,27 +1478,15 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_xcorr(xco
     const long long w = blockIdx.x;
     if (w >= a.count)
         return;
-    const long long item = w / a.nseg;
-    const long long seg  = w - item * a.nseg;
+    const long long item = w / a.groups;
+    const long long s0   = (w - item * a.groups) * a.per;
     const int t          = threadIdx.x;
     const T* x           = a.x + item * a.dx;
     const T* g           = a.g + item * a.dg;
-    const long long base = seg * a.P;
-    auto at              = [&](int i) -> cx<T>& { return lds[laddr<role_block, 1, G::LD>(0, i)]; };
-    cx<T> v[E];
-#pragma unroll
-    for (int k = 0; k < E; ++k)
-    {
-        const int n       = t + k * TP;
-        const long long p = base + n;
-        v[k].re           = (n < a.P && p < a.nx) ? x[p] : T(0);
-        v[k].im           = p < a.ng ? g[p] : T(0);
-    }
-    run_pass<T, L, false, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
-    // v[k] = Z[i], i = t + k*TPT. R[i] = G[i] conj(X[i]) / N needs Z[N - i]. X and G are spectra of
-    // real signals, so R[N - i] = conj(R[i]): the upper slots (i >= N/2) publish Z, each lower slot
-    // reads its partner, forms R[i] and leaves conj(R[i]) = R[N - i] in the position it read, and the
-    // upper slots collect theirs (slot 0 pairs with itself, as does N/2).
+    auto at              = [&](int i) -> cx<T>& { return lds[laddr<role_conv, 1, G::LD>(0, i)]; };
+    // R[i] = G[i] conj(X[i]) / N needs Z[N - i]. X and G are spectra of real signals, so
+    // R[N - i] = conj(R[i]) and the sums are kept for i < N/2 only (slot 0 pairs with itself; rm is
+    // R[N/2], which does too, in thread 0)
     auto prod = [&](cx<T> z, cx<T> zm) -> cx<T>
     {
         const cx<T> X   = { T(0.5) * (z.re + zm.re), T(0.5) * (z.im - zm.im) };
@@ -1480,37 +1494,68 @@ __global__ void __launch_bounds__((geom<T, L, role_block>::BS)) k_conv_xcorr(xco
         const cx<T> Gs  = { T(0.5) * dgi.im, -T(0.5) * dgi.re };
         return { (Gs.re * X.re + Gs.im * X.im) * a.scale, (Gs.im * X.re - Gs.re * X.im) * a.scale };
     };
+    cx<T> r[E / 2], rm = { T(0), T(0) };
 #pragma unroll
-    for (int k = E / 2; k < E; ++k)
-        at(t + k * TP - HN) = v[k];
-    lds_barrier();
+    for (int k = 0; k < E / 2; ++k)
+        r[k] = { T(0), T(0) };
+    cx<T> v[E];
+    auto bound = [](long long q) { return (int)(q < 0 ? 0 : q > N ? N : q); };
+    for (long long s = s0; s < s0 + a.per && s < a.nseg; ++s)
+    {
+        // x_s ends after P values or with the signal, g with its own (32-bit bounds)
+        const long long base = s * a.P;
+        const int hx = bound(a.nx - base < a.P ? a.nx - base : a.P), hg = bound(a.ng - base);
+        const T *xs = x + base, *gs = g + base;
+        const int tl = fresh(t);
+#pragma unroll
+        for (int k = 0; k < E; ++k)
+        {
+            const int n = tl + k * TP;
+            v[k].re     = n < hx ? xs[n] : T(0);
+            v[k].im     = n < hg ? gs[n] : T(0);
+        }
+        run_pass<T, L, false, role_conv, prec_full, 0>(v, lds, 0, fresh(t), a.tw);
+        // v[k] = Z[i], i = t + k*TPT: the upper slots publish Z, each lower slot reads its partner
+        const int tm = fresh(t);
+#pragma unroll
+        for (int k = E / 2; k < E; ++k)
+            at(tm + k * TP - HN) = v[k];
+        lds_barrier();
+#pragma unroll
+        for (int k = 0; k < E / 2; ++k)
+        {
+            const int i   = tm + k * TP;
+            const cx<T> p = prod(v[k], i == 0 ? v[k] : at(i == 0 ? 0 : N - i - HN));
+            r[k]          = cadd(r[k], p);
+            settle(r[k]);
+        }
+        rm = cadd(rm, prod(v[E / 2], v[E / 2])); // meant in thread 0
+        lds_barrier();
+    }
+    const int tm = fresh(t);
 #pragma unroll
     for (int k = 0; k < E / 2; ++k)
     {
-        const int i = t + k * TP;
-        if (i == 0)
-            v[k] = prod(v[k], v[k]);
-        else
-        {
-            cx<T>& slot = at(N - i - HN);
-            v[k]        = prod(v[k], slot);
-            slot        = cconj(v[k]); // R[N - i], for the slot that published Z[N - i]
-        }
+        v[k]        = r[k];
+        const int i = tm + k * TP;
+        if (i > 0)
+            at(N - i - HN) = cconj(r[k]); // R[N - i]
     }
     lds_barrier();
 #pragma unroll
     for (int k = E / 2; k < E; ++k)
     {
-        const int i = t + k * TP;
-        v[k]        = i == HN ? prod(v[k], v[k]) : at(i - HN);
+        const int i = tm + k * TP;
+        v[k]        = i == HN ? rm : at(i - HN);
     }
     lds_barrier();
-    run_pass<T, L, true, role_block, prec_full, 0>(v, lds, 0, t, a.tw);
-    T* out = a.part + w * a.nh;
+    run_pass<T, L, true, role_conv, prec_full, 0>(v, lds, 0, fresh(t), a.tw);
+    T* out       = a.part + w * a.nh;
+    const int ts = fresh(t);
 #pragma unroll
     for (int k = 0; k < E; ++k)
     {
-        const int n = t + k * TP;
+        const int n = ts + k * TP;
         if (n < a.nh)
             out[n] = v[k].re;
     }
@@ -1563,14 +1608,14 @@ void conv_os_launch(const conv_os_args<T>& a, hipStream_t s)
 template <typename T, int L>
 void conv_xcorr_launch(const xcorr_args<T>& a, hipStream_t s)
 {
-    using G                  = geom<T, L, role_block>;
+    using G                  = geom<T, L, role_conv>;
     constexpr size_t bytes   = G::lds_bytes;
     static const bool lds_ok = (allow_lds(k_conv_xcorr<T, L>, bytes), true);
     (void)lds_ok;
     if (a.count > 0x7fffffffll)
         throw std::runtime_error("correlation too large for one launch");
     timing::span ts([] { return timing::kernel_name("k_conv_xcorr", timing::type_name<T>(), L); },
-                    (long long)sizeof(T) * (a.count / a.nseg) * (a.nx + a.ng) +
+                    (long long)sizeof(T) * (a.count / a.groups) * (a.nx + a.ng) +
                         (long long)sizeof(T) * a.count * a.nh,
                     s);
     hipLaunchKernelGGL((k_conv_xcorr<T, L>), dim3((unsigned)a.count), dim3(G::BS), bytes, s, a);
@@ -2104,7 +2149,13 @@ void os_conv<T>::backward(T* dx, T* dh, const T* g, const T* x, const T* h, long
         a.P     = (int)(N - (long long)q.nh + 1);
         a.nh    = (int)q.nh;
         a.nseg  = ((long long)q.nx + a.P - 1) / a.P;
-        a.count = a.nseg * batch;
+        // about 2^20 threads over the whole call (four rounds of the card's 1024 per CU), each workgroup
+        // with its share of an item's segments (one inverse transform and one partial result each)
+        const long long bs   = std::max<long long>(64, N >> p2::log_e<T>);
+        const long long want = std::min<long long>(a.nseg, std::max<long long>(1, (1ll << 20) / bs / batch));
+        a.per                = (int)((a.nseg + want - 1) / want);
+        a.groups             = (a.nseg + a.per - 1) / a.per;
+        a.count              = a.groups * batch;
         a.scale = T(1) / T(N);
         q.part.ensure((size_t)(a.count * a.nh) * sizeof(T));
         a.part = q.part.template as<T>();
@@ -2119,7 +2170,7 @@ void os_conv<T>::backward(T* dx, T* dh, const T* g, const T* x, const T* h, long
             per_item = q.sum.template as<T>();
         }
         hipLaunchKernelGGL(p2::k_conv_xcorr_sum<T>, dim3(nblocks(batch * nh, 256)), dim3(256), 0, s, per_item,
-                           a.part, nh, a.nseg, batch);
+                           a.part, nh, a.groups, batch);
         hip_check(hipGetLastError(), "gradient reduction");
         if (h_dist == 0)
         {
