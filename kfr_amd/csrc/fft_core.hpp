@@ -486,8 +486,9 @@ inline bool plan_mixed(long long nn, stockham& S, int pm, int max_threads)
         for (int i = from; i < choices; ++i)
         {
             const int r = menu[i].r;
-            // f64 butterflies above radix 10 hold more values than the kernels have registers for
-            if (rest % r != 0 || (pm < 16 && r > 10))
+            // no 16-point butterfly in the f64 builds (check_pass_radices); with 12, 14 and 15 points f64
+            // 30240 x 277 (180 x 168 = 15*12 x 14*12) takes 112 us, 173 with at most 10 points
+            if (rest % r != 0 || (pm < 16 && r == 16))
                 continue;
             cur.push_back(r);
             self(self, rest / r, i);
@@ -1133,6 +1134,15 @@ struct core_fft
         run_fourstep<INV>(ld, st, batch, scratch.as<cx<T>>(), 3, s);
     }
 
+    // columns or rows per workgroup of a launch of `count`: `most` (whole lines), halved down to 32-byte runs
+    // while the launch has fewer workgroups than the card has CUs
+    static int group_width(int most, long long count)
+    {
+        while (most > (sizeof(T) == 4 ? 4 : 2) && (count + most - 1) / most < 256)
+            most /= 2;
+        return most;
+    }
+
     // four-step in rounds of at most `chunk` items through `mid`: phases bit 0 runs the column kernels,
     // bit 1 the row kernels (one of them alone only within one round)
     template <bool INV>
@@ -1141,10 +1151,6 @@ struct core_fft
     {
         const long long chunk = round > 0 ? round : this->chunk;
         const cx<T>* t   = tw.as<cx<T>>();
-        lds_geom GA      = make_geom(SA, C, 1, C, 1);
-        lds_geom GB      = make_geom(SB, R, 0, 1, (int)n1 | 1); // an odd distance: the transposed reads spread
-        const size_t shA = lds_padded_elems((size_t)C * n2) * sizeof(cx<T>);
-        const size_t shB = lds_padded_elems((size_t)R * (n1 + 1)) * sizeof(cx<T>);
         fourstep_args<T> fs;
         fs.scratch = mid;
         fs.ta      = t + twTA;
@@ -1163,16 +1169,18 @@ struct core_fft
             la.b0 += b0;
             xstore<T> sb = st;
             sb.b0 += b0;
-            const long long ga = nb * (long long)n1;
-            fs.ndiv            = make_fastdiv((uint32_t)n2);
+            const long long ga = nb * (long long)n1, gb = nb * (long long)n2;
+            const int cw = group_width(C, ga), rw = group_width(R, gb);
+            const lds_geom GA = make_geom(SA, cw, 1, cw, 1);
+            const lds_geom GB = make_geom(SB, rw, 0, 1, (int)n1 | 1); // an odd distance: the transposed reads spread
+            fs.ndiv           = make_fastdiv((uint32_t)n2);
             if (phases & 1)
-                launch_fft<T, INV, role_col>(mA, GA, t + twA, ga, la, st, fs, nblocks(ga, C), (unsigned)(SA.tpt * C),
-                                             shA, s);
-            const long long gb = nb * (long long)n2;
-            fs.ndiv            = make_fastdiv((uint32_t)n1);
+                launch_fft<T, INV, role_col>(mA, GA, t + twA, ga, la, st, fs, nblocks(ga, cw), (unsigned)(SA.tpt * cw),
+                                             lds_padded_elems((size_t)cw * n2) * sizeof(cx<T>), s);
+            fs.ndiv = make_fastdiv((uint32_t)n1);
             if (phases & 2)
-                launch_fft<T, INV, role_row>(mB, GB, t + twB, gb, ld, sb, fs, nblocks(gb, R), (unsigned)(SB.tpt * R),
-                                             shB, s);
+                launch_fft<T, INV, role_row>(mB, GB, t + twB, gb, ld, sb, fs, nblocks(gb, rw), (unsigned)(SB.tpt * rw),
+                                             lds_padded_elems((size_t)rw * (n1 + 1)) * sizeof(cx<T>), s);
         }
     }
 
@@ -1193,8 +1201,7 @@ struct core_fft
         const int most = max_block_of(is_mixed(S));
         while (c > 1 && ((size_t)c * n * sizeof(cx<T>) > lds_budget() || c * S.tpt > most))
             c /= 2;
-        while (c > (sizeof(T) == 4 ? 4 : 2) && (cols + c - 1) / c < 256)
-            c /= 2;
+        c = group_width(c, cols);
         lds_geom G = make_geom(S, c, 1, c, 1);
         fourstep_args<T> fs;
         fs.scratch = out;

@@ -421,7 +421,7 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, const fastdiv& f)
 // phase with element operations stages through LDS instead. What bounded these kernels was instructions
 // and LDS trips: staging both ends and radices of at most 7 for odd factors, 960 points made five trips
 // and took 172 us for 16384 f32 transforms; as 15 x 16 x 4 with two trips they take 57 us (4.4 TB/s, a
-// copy of the same bytes 49 us). f64 30240 x 256 (four-step, 168 x 180) 229 -> 163 us, the uneven batch of
+// copy of the same bytes 49 us). f64 30240 x 256 (four-step, 168 x 180) 229 -> 111 us, the uneven batch of
 // 20,000 transforms 429 -> 338 us.
 
 constexpr int max_passes = 20;
@@ -471,7 +471,7 @@ struct lds_geom
 
 // Radices with a butterfly, and butterflies per thread of a radix-R pass: as many as a thread's pm
 // values hold, rounded up for the small radices so that every length up to 512*pm runs on at most 512
-// threads; one of radix 12, 14 and 15 (f32), whose tables and temporaries are the largest.
+// threads; one of radix 12, 14 and 15, whose tables and temporaries are the largest.
 __host__ __device__ constexpr bool lds_radix(int r)
 {
     return (r >= 2 && r <= 10) || r == 12 || r == 14 || r == 15 || r == 16;

@@ -105,3 +105,29 @@ def test_strided_real_axes(shape, dt):
     bound = bound_fp64(n, dt)
     assert oracle.rel_rms(yd.cpu().numpy(), np.fft.rfftn(x.astype(np.float64))) <= bound
     assert oracle.rel_rms(keep.cpu().numpy() / n, x) <= 4 * bound
+
+
+# the longest one-workgroup powers of two run a few transforms as two kernels and many in one workgroup
+# each (they change over at 96), and stay in one workgroup under capture
+@pytest.mark.parametrize("n,dtype", [(1 << 14, np.complex64), (1 << 15, np.complex64), (1 << 14, np.complex128)])
+@pytest.mark.parametrize("batch", [1, 95, 96])
+def test_longest_one_workgroup_lengths(n, dtype, batch):
+    torch = pytest.importorskip("torch")
+    x = oracle.complex_uniform(620 + batch, (batch, n), dtype)
+    p = kfr_amd.dft_plan(n, dtype)
+    xd = torch.from_numpy(x).cuda()
+    for inverse in (False, True):
+        ref = np.fft.ifft(x.astype(np.complex128)) * n if inverse else np.fft.fft(x.astype(np.complex128))
+        yd = torch.full_like(xd, float("nan"))
+        p.execute_batch(yd, xd, batch, inverse)
+        assert oracle.rel_rms(yd.cpu().numpy(), ref) <= bound_fp64(n, dtype)
+    zd = torch.full_like(xd, float("nan"))
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        p.execute_batch(zd, xd, batch, inverse=True)
+    for _ in range(3):
+        zd.fill_(0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert oracle.rel_rms(zd.cpu().numpy(), ref) <= bound_fp64(n, dtype)
