@@ -51,6 +51,7 @@ inline constexpr int direct_max_log = max_log<T> + 1;
 template <typename T>
 inline constexpr int lds_budget = sizeof(T) == 4 ? 16384 : 8192; // complex values per workgroup
 constexpr int min_split_log = 7;                                 // shortest four-step factor
+constexpr int both_min_log  = 2 * min_split_log; // shortest length with both a one-workgroup and a four-step kernel
 
 // pass schedule of 2^L points (also used on the host to lay out the twiddle tables)
 __host__ __device__ constexpr int pass_le(int L, int le) { return L < le ? L : le; }
@@ -1658,6 +1659,14 @@ struct pow2_fft<T>::impl
     int L     = 0;
     int prec  = p2::prec_full;
     bool four = false;
+    // the longest one-workgroup lengths also have the four-step's tables: fewer than split_below transforms
+    // leave most CUs idle with one workgroup each, so those run as the two kernels (one f32 transform of
+    // 2^15 points 23.6 -> 12.3 us, of 2^14 15.3 -> 12.1, f64 2^14 20.6 -> 11.7; they cross near 100
+    // transforms, 130 at f32 2^14). Calls with a workspace and calls under stream capture stay in one
+    // workgroup, which needs no intermediate.
+    bool both = false;
+    static constexpr long long split_below = 96;
+    dev_mem twd; // one-workgroup pass tables
     int L1 = 0, L2 = 0; // four-step: rows of n1 = 2^L1 points, columns of n2 = 2^L2 points
     int lbits = 0;
     dev_mem tw;
@@ -1696,9 +1705,11 @@ pow2_fft<T>::pow2_fft(size_t n, hipStream_t s, int prec) : p(new impl)
     if (L <= p2::direct_max_log<T>)
     {
         const int cnt = p2::pass_twoff(L, le, p2::pass_count(L, le));
-        p->tw.reset((size_t)std::max(1, cnt) * sizeof(cx<T>));
-        p2::gen_pass_tables<T>(L, p->tw.template as<cx<T>>(), s);
-        return;
+        p->twd.reset((size_t)std::max(1, cnt) * sizeof(cx<T>));
+        p2::gen_pass_tables<T>(L, p->twd.template as<cx<T>>(), s);
+        if (L < p2::both_min_log)
+            return;
+        p->both = true;
     }
     // the longest lengths (measured with 1 GiB rounds: from 2^24; at 2^23 the four-step is 10% (f32)
     // and 2% (f64) faster): HBM passes of radix 2^5..2^8 with 16 butterflies per workgroup (128-byte
@@ -1756,7 +1767,7 @@ pow2_fft<T>::pow2_fft(size_t n, hipStream_t s, int prec) : p(new impl)
         p->chunk = (long long)std::max<size_t>(1, cap / (n * sizeof(cx<T>)));
         return;
     }
-    p->four = true;
+    p->four = !p->both;
     p->L2   = std::max(p2::min_split_log, L / 2);
     // column length 2^L2 measured fastest per length (sweep of L2 over 7..14 on MI355X, full
     // precision): the column and row kernels of 2^8..2^9 points run near half of peak, those of
@@ -1866,12 +1877,19 @@ void pow2_fft<T>::impl::run(bool inverse, const void* in, void* out, long long b
         }
         return;
     }
-    if (!four)
+    bool direct = !four;
+    if (both && batch < split_below && !w.p)
+    {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        hip_check(hipStreamIsCapturing(s, &cs), "stream capture status");
+        direct = cs != hipStreamCaptureStatusNone;
+    }
+    if (direct)
     {
         args<T> a;
         a.in  = in;
         a.out = out;
-        a.tw  = t;
+        a.tw  = twd.template as<cx<T>>();
         p2::launch_any<T, role_direct, PREC, 1, p2::direct_max_log<T>>(inverse, L, a, batch, s);
         return;
     }
@@ -1938,7 +1956,7 @@ void pow2_fft<T>::run_axis(bool inverse, const void* in, void* out, int inner_lo
     p2::args<T> a;
     a.in  = in;
     a.out = out;
-    a.tw  = p->tw.template as<cx<T>>();
+    a.tw  = p->twd.template as<cx<T>>();
     a.ta  = nullptr; // no four-step twiddles
     a.lo  = inner_log;
     constexpr int ML = p2::max_log<T>;
@@ -1955,7 +1973,7 @@ bool pow2_fft<T>::dct(bool inverse, const void* x, void* y, const void* wn, cons
     if (batch <= 0)
         return true;
     return p2::dct2_any<T, p2::dct_min_log<T>, p2::direct_max_log<T>>(
-        inverse, p->L, static_cast<const T*>(x), static_cast<T*>(y), p->tw.template as<cx<T>>(),
+        inverse, p->L, static_cast<const T*>(x), static_cast<T*>(y), p->twd.template as<cx<T>>(),
         static_cast<const cx<T>*>(wn), static_cast<const cx<T>*>(w4n), batch, s);
 }
 
@@ -1968,7 +1986,7 @@ bool pow2_fft<T>::real(bool inverse, const void* in, long long idist, void* out,
         return false;
     if (batch <= 0)
         return true;
-    const cx<T>* t = p->tw.template as<cx<T>>();
+    const cx<T>* t = p->twd.template as<cx<T>>();
     const auto* i  = static_cast<const cx<T>*>(in);
     auto* o        = static_cast<cx<T>*>(out);
     const auto* r  = static_cast<const cx<T>*>(rtw);
