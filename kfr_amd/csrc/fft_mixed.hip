@@ -1,8 +1,8 @@
 // Mixed-radix C2C kernels specialised per length (f32).
 //
-// A transform of N points (a menu length) runs its Stockham passes with compile-time radices (16,
-// then the power-of-two remainder, then 7, 5, 3), strides and loop bounds. Each pass gives every thread
-// ceil(16/R) butterflies of radix R; butterfly j reads x[j + r*N/R]. The first pass reads those
+// A transform of N points (a menu length) runs its Stockham passes with compile-time radices (2..10, 12,
+// 14, 15 and 16), strides and loop bounds. Each pass gives every thread ceil(16/R) butterflies of radix R
+// (one from 12 points on); butterfly j reads x[j + r*N/R]. The first pass reads those
 // operands straight from HBM (consecutive threads, consecutive addresses), passes exchange through
 // padded LDS, and the last pass, whose output r of butterfly j is element j + r*N/R in natural order,
 // writes straight to HBM. Longer lengths use the four-step split n = n1*n2 with both factors from the
@@ -34,29 +34,65 @@ struct radix_list
     int r[24] = {};
 };
 
+// butterflies per thread of a radix-R pass
+constexpr int mbf(int R) { return R >= 12 ? 1 : (pm + R - 1) / R; }
+
+// Passes of N points: the product of butterfly radices with the least modelled work per point, as the
+// run-time schedules of other lengths (a pass costs its butterfly, its twiddles and one LDS exchange, times
+// its idle lanes). 3840 points run as 16 x 16 x 15 instead of 16 x 16 x 5 x 3, 4000 in four passes instead
+// of five.
+struct radix_search
+{
+    int n = 0;
+    radix_list cur, best;
+    double best_cost = 1e300;
+
+    constexpr double butterfly_cost(int r) const
+    {
+        const int rs[]    = { 16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2 };
+        const double cs[] = { 10.5, 13, 16, 9, 10, 11, 7, 14, 7, 8, 4, 5, 2 };
+        for (int i = 0; i < 13; ++i)
+            if (rs[i] == r)
+                return cs[i];
+        return 0;
+    }
+    constexpr void run(int rest, int largest)
+    {
+        if (rest == 1)
+        {
+            int tpt = 1;
+            for (int p = 0; p < cur.n; ++p)
+            {
+                const int t = (n / cur.r[p] + mbf(cur.r[p]) - 1) / mbf(cur.r[p]);
+                tpt         = t > tpt ? t : tpt;
+            }
+            double cost = 0;
+            for (int p = 0; p < cur.n; ++p)
+                cost += (butterfly_cost(cur.r[p]) + 17) * tpt * mbf(cur.r[p]) * cur.r[p] / n;
+            if (cost < best_cost)
+            {
+                best_cost = cost;
+                best      = cur;
+            }
+            return;
+        }
+        for (int r = largest; r >= 2; --r)
+        {
+            if (rest % r != 0 || r == 13 || r == 11)
+                continue;
+            cur.r[cur.n++] = r;
+            run(rest / r, r);
+            --cur.n;
+        }
+    }
+};
+
 constexpr radix_list make_radices(int N)
 {
-    radix_list L;
-    int m = N, a = 0;
-    while (m % 2 == 0)
-    {
-        m /= 2;
-        ++a;
-    }
-    while (a >= 4)
-    {
-        L.r[L.n++] = 16;
-        a -= 4;
-    }
-    if (a)
-        L.r[L.n++] = 1 << a;
-    for (int p : { 7, 5, 3 })
-        while (m % p == 0)
-        {
-            L.r[L.n++] = p;
-            m /= p;
-        }
-    return L;
+    radix_search s;
+    s.n = N;
+    s.run(N, 16);
+    return s.best;
 }
 
 template <int N>
@@ -72,7 +108,7 @@ struct mshape
             s *= RL.r[q];
         return s;
     }
-    static constexpr int bf(int p) { return (pm + radix(p) - 1) / radix(p); } // butterflies per thread
+    static constexpr int bf(int p) { return mbf(radix(p)); } // butterflies per thread
     static constexpr int tpt()
     {
         int t = 1;
@@ -105,13 +141,20 @@ struct mgeom
     {
         if (ROLE == role_direct)
             return S::TPT >= 256 ? 1 : 256 / S::TPT;
-        // row kernels: at most 512 threads (measured: two workgroups per CU without register spills beat
-        // the wider runs of 1024 threads for the 4000-point rows; column kernels keep the wider runs)
-        const int maxbs = ROLE == role_row ? 512 : 1024;
-        int w           = 16;
-        while (w > 1 && (w * N > lds_values || w * S::TPT > maxbs))
-            w /= 2;
-        return w;
+        // row kernels: at most 512 threads (measured: two workgroups per CU beat the wider runs of 1024
+        // threads for the 1000- and 4000-point rows, 607 against 652 us for 10^6 x 67 and 736 against 771 for
+        // 16 x 10^6 x 4), unless that leaves rows of three passes runs of under 32 bytes (15,360,000 x 4 with
+        // 3840-point rows: 678 us with 4 rows and 1024 threads, 727 with 2); column kernels keep the wider runs
+        auto fit = [](int threads)
+        {
+            int w = 16;
+            while (w > 1 && (w * N > lds_values || w * S::TPT > threads))
+                w /= 2;
+            return w;
+        };
+        if (ROLE != role_row || (fit(512) < 4 && S::NP <= 3))
+            return fit(1024);
+        return fit(512);
     }
     static constexpr int W       = width();
     static constexpr int BS      = S::TPT * W;
@@ -441,10 +484,10 @@ void gen_tables(int idx, cx<float>* tw, hipStream_t s)
     }
 }
 
-// four-step split: both factors menu lengths, widest narrower run, then balance
+// four-step split: both factors menu lengths, widest narrower run, then fewest row passes, then balance
 bool split(size_t n, int& i2, int& i1)
 {
-    int best_w = -1;
+    int best_w = -1, best_rp = 0;
     double best_bal = 1e300;
     i2 = i1 = -1;
     for (int a = 0; a < menu_size; ++a)
@@ -457,9 +500,11 @@ bool split(size_t n, int& i2, int& i1)
             continue;
         const int w      = std::min(width_col[a], width_row[b]);
         const double bal = std::fabs(std::log((double)d) - std::log((double)(n / d)));
-        if (w > best_w || (w == best_w && bal < best_bal))
+        const int rp     = lists[b].n; // passes of the row kernel
+        if (w > best_w || (w == best_w && (rp < best_rp || (rp == best_rp && bal < best_bal))))
         {
             best_w   = w;
+            best_rp  = rp;
             best_bal = bal;
             i2       = a; // column length n2
             i1       = b; // row length n1
