@@ -109,7 +109,9 @@ hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 // Bluestein buffers) across streams: work enqueued on a stream other than the one that used the
 // plan last first waits for that stream's last work on this plan. Enqueues from several host
 // threads are serialised by the mutex, which also guards the lazily grown scratch. Inside a stream
-// capture nothing is recorded (the captured stream orders its own work).
+// capture nothing is recorded (the captured stream orders its own work). Calls that use no scratch
+// (one-workgroup lengths, which only read the plan's tables) are neither waited for nor recorded: an
+// event after every launch held back the next one (4096 x 256 f32 forward and back 20.2 -> 14.0 us).
 struct stream_order
 {
     std::mutex mu;
@@ -124,9 +126,14 @@ struct stream_order
             (void)hipEventDestroy(ev);
     }
     template <typename Fn>
-    void run(hipStream_t s, Fn&& fn)
+    void run(hipStream_t s, bool scratch, Fn&& fn)
     {
         std::lock_guard<std::mutex> lock(mu);
+        if (!scratch)
+        {
+            fn();
+            return;
+        }
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         hip_check(hipStreamIsCapturing(s, &cs), "stream capture status");
         const bool capturing = cs != hipStreamCaptureStatusNone;
@@ -219,7 +226,7 @@ struct dft_obj : plan_ref
     stream_order ord;
     void execute(void* out, const void* in, long long batch, bool inverse, hipStream_t s)
     {
-        ord.run(s,
+        ord.run(s, !g || g->needs_scratch(batch),
                 [&]
                 {
                     if (g)
@@ -283,7 +290,7 @@ struct real_obj : plan_ref
     stream_order ord;
     void forward(void* out, const void* in, long long batch, hipStream_t s)
     {
-        ord.run(s,
+        ord.run(s, !g || g->needs_scratch(),
                 [&]
                 {
                     if (g)
@@ -298,7 +305,7 @@ struct real_obj : plan_ref
     }
     void inverse(void* out, const void* in, long long batch, hipStream_t s)
     {
-        ord.run(s,
+        ord.run(s, !g || g->needs_scratch(),
                 [&]
                 {
                     if (g)
@@ -322,7 +329,7 @@ struct dct_obj : plan_ref
     explicit dct_obj(size_t n) : desc(describe_dct(sizeof(T) == 4 ? dtype_t::f32 : dtype_t::f64, n)), g(n) {}
     void execute(void* out, const void* in, long long batch, bool inverse, hipStream_t s)
     {
-        ord.run(s, [&] { g.execute(out, in, batch, inverse, s); });
+        ord.run(s, g.needs_scratch(), [&] { g.execute(out, in, batch, inverse, s); });
     }
 };
 template <typename T>
@@ -638,7 +645,7 @@ struct dft_progressive : progressive_obj
         const size_t bytes = plan->size() * 2 * sizeof(T);
         if (i == 0)
             hip_check(hipDeviceSynchronize(), "progressive start"); // device inputs may still be in production
-        plan->ord.run(s,
+        plan->ord.run(s, true,
                       [&]
                       {
                           if (i == 0)
@@ -682,7 +689,7 @@ struct real_progressive : progressive_obj
         const size_t cb   = plan->complex_size() * 2 * sizeof(T);
         if (i == 0)
             hip_check(hipDeviceSynchronize(), "progressive start");
-        plan->ord.run(s,
+        plan->ord.run(s, true,
                       [&]
                       {
                           if (i == 0)
@@ -720,7 +727,7 @@ struct batch_obj
     size_t elem() const { return f ? sizeof(float) * 2 : sizeof(double) * 2; }
     void run(void* out, const void* in, hipStream_t s)
     {
-        ord.run(s,
+        ord.run(s, true,
                 [&]
                 {
                     if (f)
@@ -740,7 +747,7 @@ struct half_obj
     stream_order ord;
     void run(bool inverse, const void* in, void* out, long long batch, hipStream_t s)
     {
-        ord.run(s, [&] { f->run(inverse, in, out, batch, s); });
+        ord.run(s, f->needs_scratch(batch), [&] { f->run(inverse, in, out, batch, s); });
     }
 };
 
@@ -1288,7 +1295,7 @@ extern "C"
                 check_plan(conv);
                 auto* c       = reinterpret_cast<conv_obj*>(conv);
                 hipStream_t s = as_stream(stream);
-                c->ord.run(s,
+                c->ord.run(s, true,
                            [&]
                            {
                                if (c->f)
@@ -1309,7 +1316,7 @@ extern "C"
                 check_plan(conv);
                 auto* c       = reinterpret_cast<conv_obj*>(conv);
                 hipStream_t s = as_stream(stream);
-                c->ord.run(s,
+                c->ord.run(s, true,
                            [&]
                            {
                                if (c->f)

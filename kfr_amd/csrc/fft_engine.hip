@@ -391,6 +391,15 @@ size_t gpu_dft<T>::size() const
     return p->n;
 }
 template <typename T>
+bool gpu_dft<T>::needs_scratch(long long batch) const
+{
+    if (p->algo != impl::CORE)
+        return p->algo == impl::BS_CHAIN;
+    if (p->core->pow2)
+        return p->core->pow2->needs_scratch(batch);
+    return p->core->mixed ? p->core->mixed->needs_scratch() : p->core->fourstep;
+}
+template <typename T>
 const schedule_info& gpu_dft<T>::schedule() const
 {
     return p->info;
@@ -847,6 +856,12 @@ int gpu_dft_real<T>::format() const
     return p->fmt;
 }
 template <typename T>
+bool gpu_dft_real<T>::needs_scratch() const
+{
+    const pow2_fft<T>* h = p->pow2_half();
+    return !p->fused_forward() && !(h && h->fuses_real());
+}
+template <typename T>
 const schedule_info& gpu_dft_real<T>::schedule() const
 {
     return p->c->info;
@@ -1089,6 +1104,11 @@ template <typename T>
 size_t gpu_dct<T>::size() const
 {
     return p->n;
+}
+template <typename T>
+bool gpu_dct<T>::needs_scratch() const
+{
+    return !p->fused;
 }
 template <typename T>
 const schedule_info& gpu_dct<T>::schedule() const

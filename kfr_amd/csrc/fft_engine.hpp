@@ -108,6 +108,9 @@ public:
     size_t size() const;
     const schedule_info& schedule() const;
     void execute(void* out, const void* in, long long batch, bool inverse, hipStream_t s);
+    // whether execute() of this many transforms writes device memory of the plan (intermediates); calls
+    // that do not may overlap on several streams
+    bool needs_scratch(long long batch) const;
     // general strided batches: element i of transform b at base + b*dist + i (complex units)
     void execute_dist(void* out, long long odist, const void* in, long long idist, long long batch,
                       bool inverse, hipStream_t s);
@@ -142,6 +145,7 @@ public:
     size_t complex_size() const;
     int format() const;
     const schedule_info& schedule() const;
+    bool needs_scratch() const; // as gpu_dft's, for forward and inverse
     void forward(void* cout, const void* rin, long long batch, hipStream_t s);
     void inverse(void* rout, const void* cin, long long batch, hipStream_t s);
     // Progressive execution of one transform: the half-length complex units plus one unit that repacks
@@ -164,6 +168,7 @@ public:
     ~gpu_dct();
     size_t size() const;
     const schedule_info& schedule() const;
+    bool needs_scratch() const; // as gpu_dft's
     void execute(void* out, const void* in, long long batch, bool inverse, hipStream_t s);
     struct impl;
     std::unique_ptr<impl> p;

@@ -633,6 +633,12 @@ void mixed_fft<T>::run(bool inverse, const void* in, void* out, long long batch,
 }
 
 template <typename T>
+bool mixed_fft<T>::needs_scratch() const
+{
+    return p->four;
+}
+
+template <typename T>
 std::string mixed_fft<T>::describe() const
 {
     auto radices = [](int idx)

@@ -22,6 +22,7 @@ public:
     ~mixed_fft();
     // batch transforms of contiguous items (distance n), in == out allowed, unscaled
     void run(bool inverse, const void* in, void* out, long long batch, hipStream_t s, workspace w = {});
+    bool needs_scratch() const; // run() keeps an intermediate in the plan's scratch (four-step lengths)
     std::string describe() const;
 
 private:

@@ -1940,6 +1940,19 @@ void pow2_fft<T>::run(bool inverse, const void* in, void* out, long long batch, 
 }
 
 template <typename T>
+bool pow2_fft<T>::needs_scratch(long long batch) const
+{
+    return p->four || p->multi || (p->both && batch < impl::split_below);
+}
+
+template <typename T>
+bool pow2_fft<T>::fuses_real() const
+{
+    return !p->four && !p->multi && p->prec == p2::prec_full && p->L >= p2::dct_min_log<T> &&
+           p->L <= p2::direct_max_log<T>;
+}
+
+template <typename T>
 bool pow2_fft<T>::supports_axis(size_t n)
 {
     const int L = p2::log2_exact(n);
@@ -1967,8 +1980,7 @@ template <typename T>
 bool pow2_fft<T>::dct(bool inverse, const void* x, void* y, const void* wn, const void* w4n, long long batch,
                       hipStream_t s)
 {
-    if (p->four || p->multi || p->prec != p2::prec_full || p->L < p2::dct_min_log<T> ||
-        p->L > p2::direct_max_log<T>)
+    if (!fuses_real())
         return false;
     if (batch <= 0)
         return true;
@@ -1981,8 +1993,7 @@ template <typename T>
 bool pow2_fft<T>::real(bool inverse, const void* in, long long idist, void* out, long long odist, const void* rtw,
                        int fmt, long long batch, hipStream_t s)
 {
-    if (p->four || p->multi || p->prec != p2::prec_full || p->L < p2::dct_min_log<T> ||
-        p->L > p2::direct_max_log<T>)
+    if (!fuses_real())
         return false;
     if (batch <= 0)
         return true;

@@ -51,8 +51,9 @@ def _stream_ptr(stream):
     """A hipStream_t handle: the given torch stream or handle, else torch's current stream when torch
     is in use, else the default stream (NULL)."""
     if stream is None:
+        # before torch has initialised the GPU its current stream is the default one
         torch = sys.modules.get("torch")
-        if torch is not None and torch.cuda.is_available():
+        if torch is not None and torch.cuda.is_initialized():
             return torch.cuda.current_stream().cuda_stream or None
         return None
     h = getattr(stream, "cuda_stream", stream)
