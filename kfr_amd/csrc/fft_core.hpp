@@ -20,6 +20,8 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -464,16 +466,17 @@ inline bool plan_mixed(long long nn, stockham& S, int pm, int max_threads)
     {
         if (rest == 1)
         {
-            std::vector<int> all = cur;
-            all.insert(all.end(), direct.begin(), direct.end());
-            stockham t;
-            if (all.empty() || !stockham_from_radices(nn, all, t, pm) || t.tpt > max_threads)
+            // threads per transform as stockham_from_radices finds them
+            long long tpt = direct.empty() ? 1 : (nn + pm - 1) / pm;
+            for (int r : cur)
+                tpt = std::max(tpt, (nn / r + bflies(r, pm) - 1) / bflies(r, pm));
+            if ((cur.empty() && direct.empty()) || tpt > max_threads)
                 return;
             double cost = 0;
             for (int r : cur)
                 for (const choice& c : menu)
                     if (c.r == r)
-                        cost += (c.cost + 4 + 13) * ((double)t.tpt * bflies(r, pm) * r / (double)nn);
+                        cost += (c.cost + 4 + 13) * ((double)tpt * bflies(r, pm) * r / (double)nn);
             if (cost < best_cost)
             {
                 best_cost = cost;
@@ -505,14 +508,32 @@ inline bool plan_mixed(long long nn, stockham& S, int pm, int max_threads)
     return stockham_from_radices(nn, best, S, pm);
 }
 
-// Factor n into GPU passes: the fixed schedule for powers of two, the planned one for the others
+// Factor n into GPU passes: the fixed schedule for powers of two, the planned one for the others. Planned
+// pass lists are kept per process (lengths of one workgroup, so at most some ten thousand short lists):
+// the four-step planner asks for those of every divisor.
 inline bool make_stockham(long long nn, stockham& S, int pm)
 {
     std::vector<int> radix;
     if (!factor_radices(nn, radix, pm))
         return false;
-    if ((nn & (nn - 1)) == 0 || !plan_mixed(nn, S, pm, max_block_mixed))
+    if ((nn & (nn - 1)) == 0)
         return stockham_from_radices(nn, radix, S, pm);
+    static std::mutex mu;
+    static std::map<std::pair<long long, int>, std::vector<int>> planned;
+    const std::pair<long long, int> key{ nn, pm };
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        auto f = planned.find(key);
+        if (f != planned.end())
+            return stockham_from_radices(nn, f->second, S, pm);
+    }
+    if (!plan_mixed(nn, S, pm, max_block_mixed))
+        return stockham_from_radices(nn, radix, S, pm);
+    if (nn <= 1 << 14)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        planned[key] = S.radix;
+    }
     return true;
 }
 
