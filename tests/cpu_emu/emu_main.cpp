@@ -5,8 +5,10 @@
 //   emu_main prog f32|f64 n want inverse in.bin out.bin   (progressive units of one transform)
 //   emu_main ws   f32|f64 n batch inverse mb in.bin out.bin (execute with an mb-MiB caller workspace)
 //   emu_main half bf16|f16 n batch inverse in.bin out.bin   (half-precision storage, 4-byte values)
+//   emu_main constants f64 n out.bin   (cos and sin of 2*pi*k/n, k < n, as the butterflies' constants)
 // The input is copied into a buffer of exactly its size and the output buffer holds exactly the
 // output, so under AddressSanitizer every access beyond either is reported.
+#include "../../kfr_amd/csrc/fft_device.hpp"
 #include "../../kfr_amd/csrc/fft_engine.hpp"
 #include "../../kfr_amd/csrc/fft_pow2.hpp"
 
@@ -190,6 +192,20 @@ int main(int argc, char** argv)
         std::fclose(f);
         std::free(din);
         std::free(dout);
+        return 0;
+    }
+    if (kind == "constants")
+    {
+        const long n = std::atol(argv[3]);
+        FILE* f      = argc == 5 ? std::fopen(argv[4], "wb") : nullptr;
+        if (!f)
+            return 2;
+        for (long k = 0; k < n; ++k)
+        {
+            const double v[2] = { ccos2pi(k, n), csin2pi(k, n) };
+            std::fwrite(v, sizeof(v), 1, f);
+        }
+        std::fclose(f);
         return 0;
     }
     if (kind != "dft" && kind != "real" && kind != "dct" && kind != "prog" && kind != "ws")

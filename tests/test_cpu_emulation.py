@@ -80,6 +80,25 @@ def test_emulated_f64_lengths(variant, n, batch, tmp_path):
         assert e <= 1e-14
 
 
+# the constants of the butterflies are the rounded values: within half a unit of the last place, and a sliver
+# for the extended-precision reference's own rounding
+@pytest.mark.parametrize("n", [3, 5, 7, 8, 9, 12, 14, 15, 16, 127])
+def test_butterfly_constants(n, tmp_path):
+    out = tmp_path / "c.bin"
+    r = subprocess.run([str(emu_build.build("asan")), "constants", "f64", str(n), str(out)], timeout=900)
+    assert r.returncode == 0
+    got = np.fromfile(out, dtype=np.float64).reshape(n, 2)
+    pi = np.longdouble(3.141592653589793116) + np.longdouble(1.2246467991473532e-16)
+    # octants reduced in whole numbers, so that the extended sine and cosine see small angles
+    k = np.arange(n)
+    a = [(8 * v + n) // (2 * n) % 4 for v in k]                     # nearest quarter turn
+    t = 2 * pi * np.array([4 * v - n * ((8 * v + n) // (2 * n)) for v in k], dtype=np.longdouble) / (4 * n)
+    c, s = np.cos(t), np.sin(t)
+    ref = np.array([[(c, -s, -c, s)[q][i], (s, c, -s, -c)[q][i]] for i, q in enumerate(a)])
+    ulp = np.spacing(np.maximum(np.abs(ref.astype(np.float64)), 2.0 ** -60))
+    assert np.all(np.abs(got - ref) <= 0.501 * ulp)
+
+
 def test_emulated_real_and_dct(tmp_path):
     n, batch = 1 << 14, 3
     x = oracle.gaussian(71, batch * n, np.float32).reshape(batch, n)
