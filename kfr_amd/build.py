@@ -27,7 +27,8 @@ HIPFLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "
             "-munsafe-fp-atomics"]
 SOURCES = ["plan_desc.cpp", "capi.cpp", "fft_engine.hip", "fft_pow2.hip", "fft_batch.hip", "fft_md.hip", "fft_mixed.hip",
            "fft_noalloc.hip"]
-HEADERS = ["plan_desc.hpp", "fft_engine.hpp", "fft_core.hpp", "fft_device.hpp", "fft_pow2.hpp", "fft_batch.hpp", "fft_md.hpp", "fft_mixed.hpp", "fft_timing.hpp"]
+HEADERS = ["plan_desc.hpp", "fft_engine.hpp", "fft_core.hpp", "fft_device.hpp", "fft_pow2.hpp", "fft_batch.hpp", "fft_md.hpp", "fft_mixed.hpp", "fft_timing.hpp",
+           "stream_order.hpp"]
 
 
 def _compile(src: str) -> Path:

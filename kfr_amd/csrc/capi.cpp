@@ -4,6 +4,7 @@
 #include "fft_batch.hpp"
 #include "fft_engine.hpp"
 #include "fft_md.hpp"
+#include "stream_order.hpp"
 #include "fft_pow2.hpp"
 #include "fft_timing.hpp"
 #include "plan_desc.hpp"
@@ -104,52 +105,6 @@ bool is_device_ptr(const void* p)
 
 // NULL is the HIP default (null) stream, as in HIP and PyTorch (whose default stream handle is 0)
 hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
-
-// Orders the uses of one plan's device scratch (four-step intermediates, real and DCT half spectra,
-// Bluestein buffers) across streams: work enqueued on a stream other than the one that used the
-// plan last first waits for that stream's last work on this plan. Enqueues from several host
-// threads are serialised by the mutex, which also guards the lazily grown scratch. Inside a stream
-// capture nothing is recorded (the captured stream orders its own work). Calls that use no scratch
-// (one-workgroup lengths, which only read the plan's tables) are neither waited for nor recorded: an
-// event after every launch held back the next one (4096 x 256 f32 forward and back 20.2 -> 14.0 us).
-struct stream_order
-{
-    std::mutex mu;
-    hipEvent_t ev    = nullptr;
-    hipStream_t last = nullptr;
-    bool used        = false;
-    stream_order()   = default;
-    stream_order(const stream_order&) = delete;
-    ~stream_order()
-    {
-        if (ev)
-            (void)hipEventDestroy(ev);
-    }
-    template <typename Fn>
-    void run(hipStream_t s, bool scratch, Fn&& fn)
-    {
-        std::lock_guard<std::mutex> lock(mu);
-        if (!scratch)
-        {
-            fn();
-            return;
-        }
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        hip_check(hipStreamIsCapturing(s, &cs), "stream capture status");
-        const bool capturing = cs != hipStreamCaptureStatusNone;
-        if (!capturing && used && last != s)
-            hip_check(hipStreamWaitEvent(s, ev, 0), "stream ordering");
-        fn();
-        if (!capturing)
-        {
-            if (!ev)
-                hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
-            hip_check(hipEventRecord(ev, s), "stream ordering");
-            last = s;
-            used = true;
-        }
-    }
-};
 
 // Runs fn(dev_out, dev_in) on device buffers: the user's pointers when both are device memory,
 // otherwise one staging buffer (the transforms are safe in place for a single item) with copies.

@@ -6,11 +6,14 @@
 //   emu_main ws   f32|f64 n batch inverse mb in.bin out.bin (execute with an mb-MiB caller workspace)
 //   emu_main half bf16|f16 n batch inverse in.bin out.bin   (half-precision storage, 4-byte values)
 //   emu_main constants f64 n out.bin   (cos and sin of 2*pi*k/n, k < n, as the butterflies' constants)
+//   emu_main order calls out.txt   (stream_order's launches, event records and waits for calls like 0-,5s,0-:
+//                                   stream handle, then s with or - without scratch)
 // The input is copied into a buffer of exactly its size and the output buffer holds exactly the
 // output, so under AddressSanitizer every access beyond either is reported.
 #include "../../kfr_amd/csrc/fft_device.hpp"
 #include "../../kfr_amd/csrc/fft_engine.hpp"
 #include "../../kfr_amd/csrc/fft_pow2.hpp"
+#include "../../kfr_amd/csrc/stream_order.hpp"
 
 #include <cstdio>
 #include <cstdlib>
@@ -192,6 +195,24 @@ int main(int argc, char** argv)
         std::fclose(f);
         std::free(din);
         std::free(dout);
+        return 0;
+    }
+    if (kind == "order")
+    {
+        stream_order ord;
+        char* p = argv[2];
+        while (*p)
+        {
+            const auto s = reinterpret_cast<hipStream_t>((uintptr_t)std::strtoull(p, &p, 10));
+            ord.run(s, *p == 's', [&] { emu::event_log.push_back("launch " + emu::stream_text(s)); });
+            p += p[1] == ',' ? 2 : 1;
+        }
+        FILE* f = std::fopen(argv[3], "wb");
+        if (!f)
+            return 2;
+        for (const std::string& l : emu::event_log)
+            std::fprintf(f, "%s\n", l.c_str());
+        std::fclose(f);
         return 0;
     }
     if (kind == "constants")

@@ -25,6 +25,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <memory>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -292,14 +293,32 @@ inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* c)
     *c = hipStreamCaptureStatusNone;
     return hipSuccess;
 }
-inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+namespace emu
+{
+// event operations in order: "record <stream>" and "wait <stream>", streams as their handles' values
+inline std::vector<std::string> event_log;
+inline std::string stream_text(hipStream_t s) { return std::to_string(reinterpret_cast<uintptr_t>(s)); }
+} // namespace emu
+inline hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned)
+{
+    emu::event_log.push_back("wait " + emu::stream_text(s));
+    return hipSuccess;
+}
 inline hipError_t hipEventCreate(hipEvent_t* e)
 {
     *e = nullptr;
     return hipErrorInvalidValue; // no timing in the emulation
 }
-inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
-inline hipError_t hipEventRecord(hipEvent_t, hipStream_t = nullptr) { return hipSuccess; }
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
+{
+    *e = reinterpret_cast<hipEvent_t>(uintptr_t(1));
+    return hipSuccess;
+}
+inline hipError_t hipEventRecord(hipEvent_t, hipStream_t s = nullptr)
+{
+    emu::event_log.push_back("record " + emu::stream_text(s));
+    return hipSuccess;
+}
 inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 inline hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t)
 {
@@ -313,6 +332,7 @@ inline hipError_t hipGetDevice(int* d)
     *d = 0;
     return hipSuccess;
 }
+inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int)
 {
     *v = 256;

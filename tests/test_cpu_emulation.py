@@ -99,6 +99,33 @@ def test_butterfly_constants(n, tmp_path):
     assert np.all(np.abs(got - ref) <= 0.501 * ulp)
 
 
+# calls on one plan run in order whatever streams they are on, with scratch or without: every launch waits
+# for the one before, by its stream or by an event recorded after it. Streams 0 (the default one) and 5, 6; a
+# caller's stream may be destroyed after its last call, so its work is recorded before the call returns; two
+# calls in a row on the default stream without scratch record nothing
+@pytest.mark.parametrize("calls", ["5-,6-", "0-,5-", "5-,0-", "0-,0-,5-,0-,6s,0-,0s,5-,5-,0-", "0s,5-,6-,0-,5s", "5s,6-,5-"])
+def test_stream_order(calls, tmp_path):
+    out = tmp_path / "log.txt"
+    assert subprocess.run([str(emu_build.build("asan")), "order", calls, str(out)], timeout=900).returncode == 0
+    log = [line.split() for line in out.read_text().split("\n") if line]
+    seen, event, done = {}, set(), []      # launches each stream's next work runs after; those the event covers
+    for k, (op, s) in enumerate(log):
+        known = seen.setdefault(s, set())
+        if op == "launch":
+            assert set(done) <= known, (calls, log)
+            done.append(k)
+            known.add(k)
+            if s != "0":
+                assert log[k + 1] == ["record", s]
+        elif op == "record":
+            event = set(known)
+        else:
+            known |= event
+    assert len(done) == len(calls.split(","))
+    if calls.startswith("0-,0-"):
+        assert [op for op, _ in log[:2]] == ["launch", "launch"]
+
+
 def test_emulated_real_and_dct(tmp_path):
     n, batch = 1 << 14, 3
     x = oracle.gaussian(71, batch * n, np.float32).reshape(batch, n)

@@ -154,6 +154,34 @@ def test_one_plan_on_two_streams():
     assert oracle.rel_rms(a, fa) <= 1e-6 and oracle.rel_rms(b, fb) <= 1e-6
 
 
+# calls without scratch (one workgroup, and at 2^15 points 96 transforms and more) run in the order they
+# were made too: the inverse on another stream reads the spectrum that the forward, held back by other work of
+# its stream, writes. None is the default stream.
+@pytest.mark.parametrize("n,batches", [(1024, (64, 64)), (1920, (64, 64)), (1 << 15, (95, 96)), (1 << 15, (96, 95))])
+@pytest.mark.parametrize("order", ["ab", "0a", "a0"])
+def test_calls_of_one_plan_on_two_streams(n, batches, order):
+    torch = pytest.importorskip("torch")
+    streams = {"a": torch.cuda.Stream(), "b": torch.cuda.Stream(), "0": torch.cuda.default_stream()}
+    first, second = (streams[c] for c in order)
+    rows = max(batches)
+    x = oracle.complex_uniform(63 + n % 97, (rows, n), np.complex64)
+    xd = torch.from_numpy(x).cuda()
+    y, z = torch.zeros_like(xd), torch.zeros_like(xd)
+    p = kfr_amd.dft_plan(n, np.complex64)
+    p.execute_batch(y, xd, rows, False, first)
+    p.execute_batch(z, y, rows, True, first)
+    torch.cuda.synchronize()
+    y.zero_(), z.zero_()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(5_000_000)  # some milliseconds
+    p.execute_batch(y, xd, batches[0], False, first)
+    p.execute_batch(z, y, batches[1], True, second)
+    torch.cuda.synchronize()
+    got = z.cpu().numpy()[: batches[0]] / n
+    assert oracle.rel_rms(got[: min(batches)], x[: min(batches)]) <= 1e-6
+
+
 def test_injected_allocation_failure_reaches_last_error():
     """a device allocation failure (forced from the host) leaves NULL from the creator and the HIP
     error text in kfr_last_error; the next calls work and clear it"""
