@@ -1591,7 +1591,7 @@ __global__ void __launch_bounds__(fir_block) k_fir(V* __restrict__ out, V* __res
     const int g  = tid & (G - 1);
     const int ob = (tid / G) * fir_outs; // this thread's first output
     V acc[fir_outs] = {};
-    for (int k0 = g * fir_taps; k0 < np; k0 += G * fir_taps)
+    auto add_run = [&](int k0, auto whole)
     {
         // output ob + q takes sample ob + q - (k0 + k), stored at np - 1 + ob + q - k0 - k
         const V* w = x + (np - fir_taps + ob - k0); // window, a multiple of 8 values from x
@@ -1601,10 +1601,17 @@ __global__ void __launch_bounds__(fir_block) k_fir(V* __restrict__ out, V* __res
         fir_read8(w + 8, xv + 8);
 #pragma unroll
         for (int k = 0; k < fir_taps; ++k)
+            if (decltype(whole)::value || k0 + k < nt)
 #pragma unroll
-            for (int q = 0; q < fir_outs; ++q)
-                fir_add(acc[q], hv[k], xv[fir_taps - 1 + q - k]);
-    }
+                for (int q = 0; q < fir_outs; ++q)
+                    fir_add(acc[q], hv[k], xv[fir_taps - 1 + q - k]);
+    };
+    int k0 = g * fir_taps;
+    for (; k0 + fir_taps <= nt; k0 += G * fir_taps)
+        add_run(k0, std::true_type{});
+    // the run that holds the last tap stops there: a zero tap times a non-finite sample is no zero
+    if (k0 < nt)
+        add_run(k0, std::false_type{});
     for (int o = 1; o < G; o <<= 1)
 #pragma unroll
         for (int q = 0; q < fir_outs; ++q)

@@ -6,6 +6,7 @@
 //   emu_main ws   f32|f64 n batch inverse mb in.bin out.bin (execute with an mb-MiB caller workspace)
 //   emu_main half bf16|f16 n batch inverse in.bin out.bin   (half-precision storage, 4-byte values)
 //   emu_main constants f64 n out.bin   (cos and sin of 2*pi*k/n, k < n, as the butterflies' constants)
+//   emu_main filter f32|f64|c32|c64 taps n,n,... taps.bin in.bin out.bin   (streaming filter, calls of n samples)
 //   emu_main order calls out.txt   (stream_order's launches, event records and waits for calls like 0-,5s,0-:
 //                                   stream handle, then s with or - without scratch)
 // The input is copied into a buffer of exactly its size and the output buffer holds exactly the
@@ -158,6 +159,52 @@ static int run(const std::string& kind, int argc, char** argv)
     return 0;
 }
 
+// one stream through a filter, every call from and into buffers of exactly its samples
+template <typename V, typename F>
+static int run_filter(F&& f, const char* calls, const char* fin, const char* fout)
+{
+    const std::vector<char> in = read_file(fin);
+    std::vector<V> res;
+    size_t pos = 0;
+    for (char* p = const_cast<char*>(calls); *p; p += *p == ',' ? 1 : 0)
+    {
+        const size_t n = std::strtoull(p, &p, 10);
+        if ((pos + n) * sizeof(V) > in.size())
+            return 2;
+        V* din  = static_cast<V*>(std::malloc(n * sizeof(V)));
+        V* dout = static_cast<V*>(std::malloc(n * sizeof(V)));
+        std::memcpy(din, in.data() + pos * sizeof(V), n * sizeof(V));
+        f.process(dout, din, n, nullptr);
+        res.insert(res.end(), dout, dout + n);
+        std::free(din);
+        std::free(dout);
+        pos += n;
+    }
+    FILE* f2 = std::fopen(fout, "wb");
+    if (!f2 || std::fwrite(res.data(), sizeof(V), res.size(), f2) != res.size())
+        return 4;
+    std::fclose(f2);
+    return 0;
+}
+
+template <typename T>
+static int filter_main(bool complex, char** argv)
+{
+    const size_t nt         = std::strtoull(argv[3], nullptr, 10);
+    const std::vector<char> h = read_file(argv[5]);
+    if (h.size() != nt * sizeof(T) * (complex ? 2 : 1))
+        return 2;
+    if (complex)
+    {
+        struct value
+        {
+            T re, im;
+        };
+        return run_filter<value>(gpu_conv_filter_complex<T>(h.data(), nt, 1024), argv[4], argv[6], argv[7]);
+    }
+    return run_filter<T>(gpu_conv_filter<T>(reinterpret_cast<const T*>(h.data()), nt, 1024), argv[4], argv[6], argv[7]);
+}
+
 int main(int argc, char** argv)
 {
     if (argc < 4)
@@ -197,6 +244,8 @@ int main(int argc, char** argv)
         std::free(dout);
         return 0;
     }
+    if (kind == "filter" && argc == 8)
+        return t == "f32" || t == "c32" ? filter_main<float>(t == "c32", argv) : filter_main<double>(t == "c64", argv);
     if (kind == "order")
     {
         stream_order ord;

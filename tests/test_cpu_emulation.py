@@ -99,6 +99,37 @@ def test_butterfly_constants(n, tmp_path):
     assert np.all(np.abs(got - ref) <= 0.501 * ulp)
 
 
+# the streaming filter's time-domain kernel: taps around a run of eight and a lane's share, calls shorter and
+# longer than a workgroup's outputs and the history. One non-finite sample reaches the outputs of its own taps
+# and no others, which keep every bit
+@pytest.mark.parametrize("t", ["f32", "f64", "c32", "c64"])
+@pytest.mark.parametrize("nt", [1, 9, 100, 130])
+def test_emulated_filter(t, nt, tmp_path):
+    rt = np.float32 if t in ("f32", "c32") else np.float64
+    dt = np.result_type(rt, np.complex64) if t[0] == "c" else rt
+    calls = [300, 7, 140, 1, 65]
+    rng = np.random.default_rng(90 + nt)
+    h, x = (rng.standard_normal(k) + (1j * rng.standard_normal(k) if t[0] == "c" else 0) for k in (nt, sum(calls)))
+    h, x = h.astype(dt), x.astype(dt)
+    h.tofile(tmp_path / "h.bin")
+
+    def run(v):
+        return _run("asan", tmp_path, ["filter", t, nt, ",".join(map(str, calls)), tmp_path / "h.bin"], v, dt)
+
+    y = run(x)
+    ref = np.convolve(x.astype(np.complex128), h.astype(np.complex128))[: len(x)]
+    # sums of nt products in the data's precision
+    assert oracle.rel_rms(y, ref if t[0] == "c" else ref.real) <= (2e-6 if rt == np.float32 else 2e-14)
+    for at in (20, 290, 350):
+        zero, bad = x.copy(), x.copy()
+        zero[at], bad[at] = 0, np.nan if at != 290 else np.inf
+        got, clean = run(bad), run(zero)
+        hit = np.zeros(len(x), dtype=bool)
+        hit[at:at + nt] = True
+        assert not np.isfinite(got[hit]).any()
+        assert np.array_equal(got[~hit].view(rt), clean[~hit].view(rt))
+
+
 # calls on one plan run in order whatever streams they are on, with scratch or without: every launch waits
 # for the one before, by its stream or by an event recorded after it. Streams 0 (the default one) and 5, 6; a
 # caller's stream may be destroyed after its last call, so its work is recorded before the call returns; two
