@@ -188,7 +188,9 @@ KFR_AMD_API void kfr_filter_delete_plan_f64(KFR_FILTER_F64* plan);
 /* Batched transforms on device pointers, enqueued on `stream` (a hipStream_t; NULL = the default
  * stream) and not synchronised. Transforms are contiguous: item b starts at b*size (complex),
  * b*size reals / b*complex_size complex values (real), b*size reals (DCT). Returns 0 on success,
- * -1 on error (see kfr_last_error). */
+ * -1 on error (see kfr_last_error). Calls on one plan run in the order they were made, on whatever streams.
+ * Complex transforms of 2^14 and 2^15 points (double: 2^14) take other kernels for fewer than 80 transforms
+ * than for more, and than under stream capture: their results may differ in the last bits. */
 KFR_AMD_API int kfr_amd_dft_execute_batch_f32(KFR_DFT_PLAN_F32* plan, kfr_c32* out, const kfr_c32* in,
                                               size_t batch, int inverse, void* stream);
 KFR_AMD_API int kfr_amd_dft_execute_batch_f64(KFR_DFT_PLAN_F64* plan, kfr_c64* out, const kfr_c64* in,

@@ -1453,6 +1453,7 @@ extern "C"
                 {
                     h->n = size;
                     h->f.reset(new pow2_fft<float>(size, library_stream(), storage));
+                    h->f->reserve();
                     hip_check(hipStreamSynchronize(library_stream()), "plan initialisation");
                 }
                 catch (...)

@@ -382,6 +382,8 @@ struct gpu_dft<T>::impl
 template <typename T>
 gpu_dft<T>::gpu_dft(size_t n) : p(new impl(n))
 {
+    if (p->core && p->core->pow2)
+        p->core->pow2->reserve();
 }
 template <typename T>
 gpu_dft<T>::~gpu_dft() = default;

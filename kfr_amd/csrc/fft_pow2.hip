@@ -1659,13 +1659,10 @@ struct pow2_fft<T>::impl
     int L     = 0;
     int prec  = p2::prec_full;
     bool four = false;
-    // the longest one-workgroup lengths also have the four-step's tables: fewer than split_below transforms
-    // leave most CUs idle with one workgroup each, so those run as the two kernels (one f32 transform of
-    // 2^15 points 23.6 -> 12.3 us, of 2^14 15.3 -> 12.1, f64 2^14 20.6 -> 11.7; they cross near 100
-    // transforms, 130 at f32 2^14). Calls with a workspace and calls under stream capture stay in one
-    // workgroup, which needs no intermediate.
+    // the longest one-workgroup lengths also have the four-step's tables: a few transforms leave most CUs idle
+    // with one workgroup each, so fewer than split_below run as the two kernels (see few())
     bool both = false;
-    static constexpr long long split_below = 96;
+    static constexpr long long split_below = 80;
     dev_mem twd; // one-workgroup pass tables
     int L1 = 0, L2 = 0; // four-step: rows of n1 = 2^L1 points, columns of n2 = 2^L2 points
     int lbits = 0;
@@ -1679,6 +1676,16 @@ struct pow2_fft<T>::impl
     std::vector<int> mp_log, mp_lbits;
     std::vector<long long> mp_tw, mp_ta, mp_tb;
     dev_mem scratch2;
+
+    // whether so many transforms of a `both` length run as the two kernels: fewer than split_below, whose
+    // intermediate reserve() has allocated. One f32 transform of 2^15 points takes 11.9 us so and 25 in one
+    // workgroup, of 2^14 11.3 and 15.7, f64 2^14 11.6 and 23.3, bf16 2^15 13.1 and 18.1. One workgroup
+    // each stays level up to the card's 256 and is the faster from about 84 transforms (f32 2^15: 21 us), 95 (bf16
+    // 2^15), 73 (f32 2^14), 68 (f64 2^14) and 63 (bf16 2^14); at 79 and 80 the two differ by 11% at most.
+    bool few(long long batch) const
+    {
+        return both && batch < split_below && scratch.bytes >= (size_t)batch << L << (sizeof(T) == 4 ? 3 : 4);
+    }
 
     template <int PREC>
     void run(bool inverse, const void* in, void* out, long long batch, hipStream_t s, workspace w);
@@ -1878,10 +1885,12 @@ void pow2_fft<T>::impl::run(bool inverse, const void* in, void* out, long long b
         return;
     }
     bool direct = !four;
-    if (both && batch < split_below && !w.p)
+    if (few(batch) && (!w.p || (PREC == p2::prec_full && w.bytes >= (size_t)batch * sizeof(cx<T>) << L)))
     {
+        // under capture without a workspace: one workgroup, whose graph shares no intermediate with other calls
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        hip_check(hipStreamIsCapturing(s, &cs), "stream capture status");
+        if (!w.p)
+            hip_check(hipStreamIsCapturing(s, &cs), "stream capture status");
         direct = cs != hipStreamCaptureStatusNone;
     }
     if (direct)
@@ -1942,7 +1951,22 @@ void pow2_fft<T>::run(bool inverse, const void* in, void* out, long long batch, 
 template <typename T>
 bool pow2_fft<T>::needs_scratch(long long batch) const
 {
-    return p->four || p->multi || (p->both && batch < impl::split_below);
+    return p->four || p->multi || p->few(batch);
+}
+
+template <typename T>
+void pow2_fft<T>::reserve()
+{
+    if (!p->both)
+        return;
+    try
+    {
+        p->scratch.ensure((size_t)(impl::split_below - 1) * sizeof(cx<T>) << p->L);
+    }
+    catch (const hip_error&)
+    {
+        (void)hipGetLastError(); // those lengths run without it
+    }
 }
 
 template <typename T>

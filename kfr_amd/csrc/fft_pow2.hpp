@@ -24,6 +24,10 @@ public:
     // batch transforms: in and out hold batch*n complex values each, item b at offset b*n; in == out
     // is allowed. No scaling (the inverse is unnormalised).
     void run(bool inverse, const void* in, void* out, long long batch, hipStream_t s, workspace w = {});
+    // Allocates the intermediate with which a few transforms of the longest one-workgroup lengths run as two
+    // kernels (at most 20 MiB; nothing at other lengths). Such a length never allocates later, and runs in
+    // one workgroup if it has no intermediate.
+    void reserve();
     // whether run() of this many transforms keeps an intermediate in the plan's scratch
     bool needs_scratch(long long batch) const;
     // whether real() and dct() have kernels for this length

@@ -229,7 +229,9 @@ int main(int argc, char** argv)
         std::memcpy(din, in.data(), bytes);
         try
         {
-            pow2_fft<float>(n, nullptr, t == "bf16" ? 1 : 2).run(inverse, din, dout, batch, nullptr);
+            pow2_fft<float> f(n, nullptr, t == "bf16" ? 1 : 2);
+            f.reserve();
+            f.run(inverse, din, dout, batch, nullptr);
         }
         catch (const std::exception& e)
         {

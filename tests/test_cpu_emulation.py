@@ -99,6 +99,24 @@ def test_butterfly_constants(n, tmp_path):
     assert np.all(np.abs(got - ref) <= 0.501 * ulp)
 
 
+# the longest one-workgroup lengths: a few transforms as two kernels, with the plan's intermediate or a
+# workspace and the same bits, and under capture in one workgroup, with its two-round LDS exchange
+@pytest.mark.parametrize("dtype,n", [(np.complex64, 1 << 15), (np.complex64, 1 << 14), (np.complex128, 1 << 14)])
+def test_emulated_longest_one_workgroup(dtype, n, tmp_path):
+    t, batch = "f32" if dtype == np.complex64 else "f64", 2
+    x = oracle.complex_uniform(64, (batch, n), dtype)
+    for inverse in (False, True):
+        xx = x.astype(np.complex128)
+        ref = np.fft.ifft(xx) * n if inverse else np.fft.fft(xx)
+        args = [t, n, batch, int(inverse)]
+        two = _run("asan", tmp_path, ["dft"] + args, x, dtype)
+        ws = _run("asan", tmp_path, ["ws"] + args + [4], x, dtype)
+        one = _run("asan", tmp_path, ["dft"] + args, x, dtype, {"EMU_CAPTURING": "1"})
+        assert np.array_equal(two, ws) and not np.array_equal(two, one)
+        for y in (two, one):
+            assert oracle.rel_rms(y.reshape(batch, n), ref) <= (1e-6 if t == "f32" else 1e-14)
+
+
 # the streaming filter's time-domain kernel: taps around a run of eight and a lane's share, calls shorter and
 # longer than a workgroup's outputs and the history. One non-finite sample reaches the outputs of its own taps
 # and no others, which keep every bit

@@ -154,10 +154,10 @@ def test_one_plan_on_two_streams():
     assert oracle.rel_rms(a, fa) <= 1e-6 and oracle.rel_rms(b, fb) <= 1e-6
 
 
-# calls without scratch (one workgroup, and at 2^15 points 96 transforms and more) run in the order they
+# calls without scratch (one workgroup, and at 2^15 points 80 transforms and more) run in the order they
 # were made too: the inverse on another stream reads the spectrum that the forward, held back by other work of
 # its stream, writes. None is the default stream.
-@pytest.mark.parametrize("n,batches", [(1024, (64, 64)), (1920, (64, 64)), (1 << 15, (95, 96)), (1 << 15, (96, 95))])
+@pytest.mark.parametrize("n,batches", [(1024, (64, 64)), (1920, (64, 64)), (1 << 15, (79, 80)), (1 << 15, (80, 79))])
 @pytest.mark.parametrize("order", ["ab", "0a", "a0"])
 def test_calls_of_one_plan_on_two_streams(n, batches, order):
     torch = pytest.importorskip("torch")

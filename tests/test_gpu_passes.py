@@ -108,9 +108,9 @@ def test_strided_real_axes(shape, dt):
 
 
 # the longest one-workgroup powers of two run a few transforms as two kernels and many in one workgroup
-# each (they change over at 96), and stay in one workgroup under capture
+# each (they change over at 80), and stay in one workgroup under capture
 @pytest.mark.parametrize("n,dtype", [(1 << 14, np.complex64), (1 << 15, np.complex64), (1 << 14, np.complex128)])
-@pytest.mark.parametrize("batch", [1, 95, 96])
+@pytest.mark.parametrize("batch", [1, 79, 80, 95, 96])
 def test_longest_one_workgroup_lengths(n, dtype, batch):
     torch = pytest.importorskip("torch")
     x = oracle.complex_uniform(620 + batch, (batch, n), dtype)

@@ -40,6 +40,52 @@ def test_noalloc_matches_execute_batch(n, b1, b2):
         assert oracle.rel_rms(got, np.fft.ifft(x[-1].astype(np.complex128)) * n) <= 1e-6
 
 
+# lengths that run a few transforms as two kernels, on both sides of the change: the first calls of a new plan
+# allocate nothing either way
+@pytest.mark.parametrize("n", [1 << 14, 1 << 15])
+@pytest.mark.parametrize("batch", [1, 79, 80])
+def test_noalloc_matches_at_the_longest_one_workgroup_lengths(n, batch):
+    torch = pytest.importorskip("torch")
+    L = kfr_amd.lib()
+    x = oracle.complex_uniform(batch, (batch, n), np.complex64)
+    xd = torch.from_numpy(x).cuda()
+    for inverse in (False, True):
+        plan = kfr_amd.dft_plan(n, np.complex64)
+        y_ref, y_na = torch.zeros_like(xd), torch.zeros_like(xd)
+        L.kfr_amd_inject_alloc_failure(1)  # any allocation from here on fails
+        try:
+            assert _run(L.kfr_amd_dft_execute_batch_f32, plan, y_ref, xd, batch, inverse) == 0, kfr_amd.last_error()
+        finally:
+            L.kfr_amd_inject_alloc_failure(0)
+        assert _run(L.kfr_amd_dft_execute_batch_noalloc_f32, plan, y_na, xd, batch, inverse) == 0
+        assert torch.equal(y_ref, y_na), (n, batch, inverse)
+        ref = np.fft.ifft(x[-1].astype(np.complex128)) * n if inverse else np.fft.fft(x[-1].astype(np.complex128))
+        assert oracle.rel_rms(y_na.cpu().numpy()[-1], ref) <= 1e-6
+
+
+# a plan whose intermediate cannot be allocated runs those lengths in one workgroup
+@pytest.mark.parametrize("n", [1 << 14, 1 << 15])
+def test_longest_one_workgroup_lengths_without_an_intermediate(n):
+    torch = pytest.importorskip("torch")
+    L = kfr_amd.lib()
+    x = oracle.complex_uniform(3, (2, n), np.complex64)
+    xd = torch.from_numpy(x).cuda()
+    made = 0
+    for k in range(1, 12):
+        L.kfr_amd_inject_alloc_failure(k)  # the k-th allocation of the plan fails
+        try:
+            plan = kfr_amd.dft_plan(n, np.complex64)
+        except kfr_amd.KfrError:
+            continue
+        finally:
+            L.kfr_amd_inject_alloc_failure(0)
+        made += 1
+        y = torch.zeros_like(xd)
+        assert _run(L.kfr_amd_dft_execute_batch_f32, plan, y, xd, 2, False) == 0
+        assert oracle.rel_rms(y.cpu().numpy(), np.fft.fft(x.astype(np.complex128))) <= 1e-6
+    assert made >= 2
+
+
 def test_noalloc_refuses_what_does_not_fit():
     torch = pytest.importorskip("torch")
     L = kfr_amd.lib()
