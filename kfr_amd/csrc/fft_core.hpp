@@ -1155,11 +1155,11 @@ struct core_fft
         run_fourstep<INV>(ld, st, batch, scratch.as<cx<T>>(), 3, s);
     }
 
-    // columns or rows per workgroup of a launch of `count`: `most` (whole lines), halved down to 32-byte runs
-    // while the launch has fewer workgroups than the card has CUs
-    static int group_width(int most, long long count)
+    // columns or rows per workgroup of a launch of `count`: `most` (whole lines), halved down to `least` while
+    // the launch has fewer workgroups than the card has CUs
+    static int group_width(int most, long long count, int least = sizeof(T) == 4 ? 4 : 2)
     {
-        while (most > (sizeof(T) == 4 ? 4 : 2) && (count + most - 1) / most < 256)
+        while (most > least && (count + most - 1) / most < 256)
             most /= 2;
         return most;
     }
@@ -1206,23 +1206,46 @@ struct core_fft
     }
 
     // ---- one axis of a multidimensional array in place along its stride: `outer` arrays of n rows of
-    // `inner` values, every column transformed by the four-step column kernel without its twiddle
-    bool supports_axis() const { return !fourstep; }
+    // `inner` values, every column transformed by the four-step column kernel without its twiddle.
+    // Columns per workgroup: whole 128-byte lines (16 f32) and a wave of threads, fewer if that leaves CUs
+    // without work (the 1080-point axis of a 1080 x 961 spectrum runs 4: 241 workgroups of 288 threads), but
+    // 32-byte runs and a wave of threads
+    int axis_columns(long long cols) const
+    {
+        const int most = max_block_of(is_mixed(S));
+        int c          = 16;
+        while (c * S.tpt < 64)
+            c *= 2;
+        while (c > 1 && ((size_t)c * n * sizeof(cx<T>) > lds_budget() || c * S.tpt > most))
+            c /= 2;
+        int least = sizeof(T) == 4 ? 4 : 2;
+        while (least * S.tpt < 64)
+            least *= 2;
+        return group_width(c, cols, least);
+    }
+    // Lengths of one workgroup whose columns move in runs of 32 bytes or more; f32 powers of two from 256 points
+    // (the staged build of the kernel, which spills) 64 bytes, and no f64 powers of two from 4096. What is left
+    // takes contiguous transforms and transposes, whose runs are 256 bytes. Measured strided against
+    // transposed: 8-byte runs 6000 x 1024 f32 185 and 92 us, 16-byte runs 3000 x 4000 237 and 150, 2400 x
+    // 1024 f64 110 and 75, 3000 x 500 f32 45 and 47; 32-byte runs 1080 x 960 f32 34 and 59 (transposed by the kernels
+    // of before), 2000 x 2000 58 and 61; f32 powers of two with 32-byte runs 4096 x 2049 273 and 227, 512 x 300 26 and 23, 2048 x
+    // 700 41 and 43, with 64-byte runs 1024 x 2400 38 and 47; f64 4096 x 2049 482 and 418, 1024 x 1025 83 and 92.
+    bool supports_axis(long long inner, long long outer) const
+    {
+        if (fourstep || inner <= 0 || outer <= 0 || inner > 0x7fffffffll / outer)
+            return false;
+        const long long run = std::min<long long>(axis_columns(inner * outer), inner) * (long long)sizeof(cx<T>);
+        if (is_mixed(S))
+            return run >= 32;
+        return sizeof(T) == 4 ? run >= (n >= 256 ? 64 : 32) : run >= 32 && n < 4096;
+    }
     template <bool INV>
     void run_axis(const cx<T>* in, cx<T>* out, long long inner, long long outer, hipStream_t s)
     {
-        const long long cols = inner * outer;
-        if (fourstep || cols > 0x7fffffffll)
+        if (!supports_axis(inner, outer))
             throw std::logic_error("this plan cannot transform a strided axis");
-        if (cols <= 0)
-            return;
-        // up to 16 columns per workgroup (whole 128-byte lines), fewer if that leaves CUs without work: the
-        // 1080-point axis of a 1080 x 961 spectrum runs 4 (241 workgroups of 288 threads)
-        int c          = 16;
-        const int most = max_block_of(is_mixed(S));
-        while (c > 1 && ((size_t)c * n * sizeof(cx<T>) > lds_budget() || c * S.tpt > most))
-            c /= 2;
-        c = group_width(c, cols);
+        const long long cols = inner * outer;
+        const int c          = axis_columns(cols);
         lds_geom G = make_geom(S, c, 1, c, 1);
         fourstep_args<T> fs;
         fs.scratch = out;

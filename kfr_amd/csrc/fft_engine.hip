@@ -432,8 +432,7 @@ void gpu_dft<T>::execute_workspace(void* out, const void* in, long long batch, b
 template <typename T>
 bool gpu_dft<T>::supports_axis(long long inner, long long outer) const
 {
-    return p->algo == impl::CORE && p->core->supports_axis() && inner > 0 && outer > 0 &&
-           inner <= 0x7fffffffll / outer;
+    return p->algo == impl::CORE && p->core->supports_axis(inner, outer);
 }
 template <typename T>
 void gpu_dft<T>::execute_axis(void* out, const void* in, long long inner, long long outer, bool inverse, hipStream_t s)

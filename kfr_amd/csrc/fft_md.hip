@@ -120,14 +120,22 @@ bool axis_set<T>::plan(const std::vector<size_t>& shape, std::map<size_t, std::u
             continue;
         }
         // columns of 64-byte runs and more: below that the transposes, whose runs are 256 bytes
-        if (inner * (long long)sizeof(cx<T>) < 64)
+        bool fits = inner * (long long)sizeof(cx<T>) >= 64;
+        if (fits)
+        {
+            auto& g = plans[n];
+            if (!g)
+                g.reset(new gpu_dft<T>(n));
+            fits = g->supports_axis(inner, outer);
+            list.push_back({ i, n, inner, outer, nullptr, g.get() });
+        }
+        if (!fits)
+        {
+            hip_check(hipStreamSynchronize(s), "multidimensional plan initialisation");
+            list.clear();
+            pow2.clear();
             return false;
-        auto& g = plans[n];
-        if (!g)
-            g.reset(new gpu_dft<T>(n));
-        if (!g->supports_axis(inner, outer))
-            return false;
-        list.push_back({ i, n, inner, outer, nullptr, g.get() });
+        }
     }
     hip_check(hipStreamSynchronize(s), "multidimensional plan initialisation");
     return true;

@@ -20,7 +20,7 @@ HERE = Path(__file__).resolve().parent
 ROOT = HERE.parent.parent
 SRC = ROOT / "kfr_amd" / "csrc"
 CXX = os.environ.get("KFR_AMD_EMU_CXX", "/opt/rocm/llvm/bin/clang++")
-SOURCES = ["plan_desc.cpp", "fft_engine.hip", "fft_pow2.hip", "fft_mixed.hip"]
+SOURCES = ["plan_desc.cpp", "fft_engine.hip", "fft_pow2.hip", "fft_mixed.hip", "fft_md.hip"]
 VARIANTS = {
     "asan": ["-fsanitize=address"],
     "asan_pm16": ["-fsanitize=address", "-DKFR_AMD_PMAX_F64=16"],
@@ -54,7 +54,11 @@ def build(variant: str = "asan", jobs: int = 8) -> Path:
 
     def compile_one(src: Path) -> Path:
         obj = out / (src.name.replace(".", "_") + ".o")
-        cmd = [CXX] + flags + ["-x", "c++", "-c", str(src), "-o", str(obj)]
+        text = src.read_text()
+        if "    __shared__ " in text:  # static LDS arrays: workgroups run one at a time, so static objects serve
+            src = out / src.name
+            src.write_text(text.replace("    __shared__ ", "    static "))
+        cmd = [CXX] + flags + ["-I", str(SRC), "-x", "c++", "-c", str(src), "-o", str(obj)]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode:
             raise RuntimeError(f"emulation build of {src.name} failed:\n{r.stderr[-4000:]}")

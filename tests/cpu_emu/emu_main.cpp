@@ -7,12 +7,15 @@
 //   emu_main half bf16|f16 n batch inverse in.bin out.bin   (half-precision storage, 4-byte values)
 //   emu_main constants f64 n out.bin   (cos and sin of 2*pi*k/n, k < n, as the butterflies' constants)
 //   emu_main filter f32|f64|c32|c64 taps n,n,... taps.bin in.bin out.bin   (streaming filter, calls of n samples)
+//   emu_main md f32|f64 d0,d1,.. real inverse in.bin out.bin   (axes; its schedule on standard output)
+//   emu_main schedule f32|f64 n
 //   emu_main order calls out.txt   (stream_order's launches, event records and waits for calls like 0-,5s,0-:
 //                                   stream handle, then s with or - without scratch)
 // The input is copied into a buffer of exactly its size and the output buffer holds exactly the
 // output, so under AddressSanitizer every access beyond either is reported.
 #include "../../kfr_amd/csrc/fft_device.hpp"
 #include "../../kfr_amd/csrc/fft_engine.hpp"
+#include "../../kfr_amd/csrc/fft_md.hpp"
 #include "../../kfr_amd/csrc/fft_pow2.hpp"
 #include "../../kfr_amd/csrc/stream_order.hpp"
 
@@ -205,6 +208,49 @@ static int filter_main(bool complex, char** argv)
     return run_filter<T>(gpu_conv_filter<T>(reinterpret_cast<const T*>(h.data()), nt, 1024), argv[4], argv[6], argv[7]);
 }
 
+template <typename T>
+static int md_main(char** argv)
+{
+    std::vector<size_t> shape;
+    for (char* p = argv[3]; *p; p += *p == ',' ? 1 : 0)
+        shape.push_back(std::strtoull(p, &p, 10));
+    const bool real = std::atoi(argv[4]) != 0, inverse = std::atoi(argv[5]) != 0;
+    const std::vector<char> in = read_file(argv[6]);
+    size_t values = 1;
+    for (size_t d : shape)
+        values *= d;
+    const size_t spectrum = (real ? values / shape.back() * (shape.back() / 2 + 1) : values) * 2 * sizeof(T);
+    const size_t ib = real && !inverse ? values * sizeof(T) : spectrum, ob = real && inverse ? values * sizeof(T) : spectrum;
+    if (in.size() != ib)
+        return 2;
+    char* din  = static_cast<char*>(std::malloc(ib));
+    char* dout = static_cast<char*>(std::malloc(ob));
+    std::memcpy(din, in.data(), ib);
+    std::memset(dout, 0x7f, ob);
+    if (real)
+    {
+        gpu_dft_md_real<T> f(shape);
+        std::printf("%s\n", f.schedule().c_str());
+        if (inverse)
+            f.inverse(dout, din, nullptr);
+        else
+            f.forward(dout, din, nullptr);
+    }
+    else
+    {
+        gpu_dft_md<T> f(shape);
+        std::printf("%s\n", f.schedule().c_str());
+        f.execute(dout, din, inverse, nullptr);
+    }
+    FILE* f = std::fopen(argv[7], "wb");
+    if (!f || std::fwrite(dout, 1, ob, f) != ob)
+        return 4;
+    std::fclose(f);
+    std::free(din);
+    std::free(dout);
+    return 0;
+}
+
 int main(int argc, char** argv)
 {
     if (argc < 4)
@@ -248,6 +294,14 @@ int main(int argc, char** argv)
     }
     if (kind == "filter" && argc == 8)
         return t == "f32" || t == "c32" ? filter_main<float>(t == "c32", argv) : filter_main<double>(t == "c64", argv);
+    if (kind == "md" && argc == 8)
+        return t == "f64" ? md_main<double>(argv) : md_main<float>(argv);
+    if (kind == "schedule" && argc == 4)
+    {
+        const size_t n = std::strtoull(argv[3], nullptr, 10);
+        std::printf("%s\n", (t == "f64" ? gpu_dft<double>(n).schedule() : gpu_dft<float>(n).schedule()).text().c_str());
+        return 0;
+    }
     if (kind == "order")
     {
         stream_order ord;

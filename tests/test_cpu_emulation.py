@@ -117,6 +117,40 @@ def test_emulated_longest_one_workgroup(dtype, n, tmp_path):
             assert oracle.rel_rms(y.reshape(batch, n), ref) <= (1e-6 if t == "f32" else 1e-14)
 
 
+# axes along their stride (mixed lengths, a power of two before an odd dimension, a short axis whose workgroups
+# take a wave of columns, a batch of arrays) and the shapes that take transposes instead: runs under 32 bytes
+# (2400 and 8192 points), the staged power-of-two kernel under 64 (256 x 40 f32), f64 powers of two from 4096
+@pytest.mark.parametrize("t,shape,strided", [("f32", (1080, 40), True), ("f32", (3, 45, 9), True), ("f64", (9, 128, 33), True),
+                                             ("f32", (128, 40), True), ("f32", (4, 300), True), ("f64", (256, 40), True),
+                                             ("f32", (2400, 40), False), ("f32", (8192, 9), False),
+                                             ("f32", (256, 40), False), ("f64", (2400, 9), False), ("f64", (4096, 9), False)])
+def test_emulated_axes(t, shape, strided, tmp_path):
+    dt = np.complex64 if t == "f32" else np.complex128
+    rt = np.float32 if t == "f32" else np.float64
+    bound = 1e-6 if t == "f32" else 1e-14
+    rng = np.random.default_rng(91)
+    fin, fout = tmp_path / "in.bin", tmp_path / "out.bin"
+
+    def run(x, sh, real, inverse, out_dtype):
+        x.tofile(fin)
+        r = subprocess.run([str(emu_build.build("asan")), "md", t, ",".join(map(str, sh)), str(real), str(int(inverse)),
+                            str(fin), str(fout)], capture_output=True, text=True, timeout=900)
+        assert r.returncode == 0, r.stderr[-4000:]
+        assert ("along its stride" in r.stdout) == strided, r.stdout
+        return np.fromfile(fout, dtype=out_dtype)
+
+    x = (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(dt)
+    for inverse in (False, True):
+        ref = np.fft.ifftn(x.astype(np.complex128)) * x.size if inverse else np.fft.fftn(x.astype(np.complex128))
+        assert oracle.rel_rms(run(x, shape, 0, inverse, dt).reshape(shape), ref) <= bound
+    if shape[-1] % 2 == 0 or not strided:  # a real last axis with as many spectrum values as columns above
+        real = shape[:-1] + (2 * (shape[-1] - 1),)
+        v = rng.standard_normal(real).astype(rt)
+        ref = np.fft.rfftn(v.astype(np.float64))
+        assert oracle.rel_rms(run(v, real, 1, False, dt).reshape(ref.shape), ref) <= bound
+        assert oracle.rel_rms(run(ref.astype(dt), real, 1, True, rt).reshape(real) / v.size, v) <= 2 * bound
+
+
 # the streaming filter's time-domain kernel: taps around a run of eight and a lane's share, calls shorter and
 # longer than a workgroup's outputs and the history. One non-finite sample reaches the outputs of its own taps
 # and no others, which keep every bit
