@@ -70,7 +70,7 @@ __device__ __forceinline__ void run_item(const len_desc& D, const cx<T>* __restr
     if (!D.bluestein && G.np >= 2 && G.pass[0].kind == pass_radix && G.pass[G.np - 1].kind == pass_radix)
     {
         first_pass<T, false, true>(G, tw, c, from_global<T, true>{ in, 1, c.valid, inv });
-        fft_passes<T, false, true>(G, tw, c, 1, G.np - 1);
+        fft_passes<T, false, true, true>(G, tw, c, 1, G.np - 1);
         // nontemporal: the outputs are not read again by this launch (measured 4% faster)
         last_pass<T, false, true>(G, tw, c, to_global<T, true, true>{ out, 1, c.valid, inv });
         return;

@@ -751,11 +751,16 @@ __device__ __forceinline__ void block_store(const lds_geom& G, const cx<T>* lds,
 template <typename T, bool MIXED>
 inline constexpr int mixed_waves = MIXED && sizeof(T) == 4 ? 4 : 1;
 
+// whether a schedule has direct passes (its last passes)
+inline bool has_direct(const stockham& s) { return !s.kind.empty() && s.kind.back() == pass_generic; }
 // FL: the first pass reads HBM itself (plain loads; row kernels, whose input is the intermediate); FS: the
 // last of two or more passes writes HBM itself (plain stores; column kernels). Mixed-radix builds only:
-// powers of two with plain data have kernels of their own.
-template <typename T, bool INV, int ROLE, bool MIXED, bool FL, bool FS>
-__global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) k_fft(lds_geom G, const cx<T>* __restrict__ tw, long long batch,
+// powers of two with plain data have kernels of their own. GEN: whole transforms with direct passes, which
+// stage both ends; compiled without the bound of mixed_waves, in which they spill 68 to 92 bytes per lane (f32 2910 =
+// 30 * 97 points x 1441 565 -> 440 us, 190 such lengths 12% faster; short transforms without direct passes
+// are 10 to 30% faster with it). The other builds of whole transforms hold no direct pass.
+template <typename T, bool INV, int ROLE, bool MIXED, bool FL, bool FS, bool GEN>
+__global__ void __launch_bounds__(max_block_of(MIXED), (GEN ? 1 : mixed_waves<T, MIXED>)) k_fft(lds_geom G, const cx<T>* __restrict__ tw, long long batch,
                                               xload<T> ld, xstore<T> st, fourstep_args<T> fs)
 {
     constexpr bool PAD = !MIXED;
@@ -820,7 +825,7 @@ __global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) 
         }
         __syncthreads();
     }
-    fft_passes<T, INV, MIXED>(G, tw, c, FL ? 1 : 0, FS ? G.np - 1 : G.np);
+    fft_passes<T, INV, MIXED, (GEN || ROLE != role_direct)>(G, tw, c, FL ? 1 : 0, FS ? G.np - 1 : G.np);
     if constexpr (ROLE == role_direct)
     {
         if constexpr (FS)
@@ -932,12 +937,12 @@ inline void check_pass_radices(const stockham& s, bool mixed_build)
     }
 }
 
-template <typename T, bool INV, int ROLE, bool MIXED, bool FL, bool FS>
+template <typename T, bool INV, int ROLE, bool MIXED, bool FL, bool FS, bool GEN = false>
 void launch_fft_as(const lds_geom& G, const cx<T>* tw, long long batch, const xload<T>& ld, const xstore<T>& st,
                    const fourstep_args<T>& fs, unsigned grid, unsigned block, size_t sh, hipStream_t s)
 {
-    allow_lds(k_fft<T, INV, ROLE, MIXED, FL, FS>, sh);
-    hipLaunchKernelGGL((k_fft<T, INV, ROLE, MIXED, FL, FS>), dim3(grid), dim3(block), sh, s, G, tw, batch, ld, st, fs);
+    allow_lds(k_fft<T, INV, ROLE, MIXED, FL, FS, GEN>, sh);
+    hipLaunchKernelGGL((k_fft<T, INV, ROLE, MIXED, FL, FS, GEN>), dim3(grid), dim3(block), sh, s, G, tw, batch, ld, st, fs);
 }
 
 // launches the power-of-two or the mixed-radix build of a kernel role; mixed radices with the first
@@ -951,7 +956,10 @@ void launch_fft(bool mixed, const lds_geom& G, const cx<T>* tw, long long batch,
     // complex values in and out: batch items (columns or rows in the four-step roles) of G.n points
     timing::span ts([mixed] { return timing::kernel_name("k_fft", timing::type_name<T>(), INV, ROLE, mixed); },
                     2 * (long long)sizeof(cx<T>) * batch * G.n, s);
-    const bool wide = ROLE != role_direct || G.tpt >= 16;
+    bool gen = false; // whole transforms with a direct pass
+    for (int p = 0; p < G.np; ++p)
+        gen = gen || (ROLE == role_direct && G.pass[p].kind == pass_generic);
+    const bool wide = !gen && (ROLE != role_direct || G.tpt >= 16);
     const bool fl   = wide && G.pass[0].kind == pass_radix && (ROLE == role_row || plain(ld));
     const bool fl2  = fl && G.np >= 2;
     const bool fst  = wide && G.np >= 2 && G.pass[G.np - 1].kind == pass_radix && (ROLE == role_col || plain(st));
@@ -970,6 +978,8 @@ void launch_fft(bool mixed, const lds_geom& G, const cx<T>* tw, long long batch,
             launch_fft_as<T, INV, ROLE, true, true, true>(G, tw, batch, ld, st, fs, grid, block, sh, s);
         else if (fst)
             launch_fft_as<T, INV, ROLE, true, false, true>(G, tw, batch, ld, st, fs, grid, block, sh, s);
+        else if (gen)
+            launch_fft_as<T, INV, ROLE, true, false, false, ROLE == role_direct>(G, tw, batch, ld, st, fs, grid, block, sh, s);
         else
             launch_fft_as<T, INV, ROLE, true, false, false>(G, tw, batch, ld, st, fs, grid, block, sh, s);
     }
@@ -1016,6 +1026,30 @@ struct core_fft
         return t;
     }
 
+    // Threads of one workgroup's schedule with direct passes (large primes), which are the longest by far and take
+    // ceil(n / tpt) rounds in every wave: more than the least number where that saves a fifth of the rounds
+    // times waves. f64 1032 = 24 * 43 points take 172 threads, 6 rounds of 3 waves, instead of 129 and 8 rounds (x
+    // 4064: 200 -> 173 us); savings of an eighth, 1590 points in 228 threads instead of 199, measured slower.
+    static void widen_direct(stockham& s)
+    {
+        if (!has_direct(s))
+            return;
+        auto cost = [](const stockham& c)
+        {
+            const int per = pick_tpb(c);
+            return (double)((c.n + c.tpt - 1) / c.tpt) * ((c.tpt * per + 63) / 64) / per;
+        };
+        double best = 0.8 * cost(s);
+        int tpt     = s.tpt;
+        for (stockham c = s; c.tpt <= max_block_mixed; ++c.tpt)
+            if (cost(c) <= best)
+            {
+                best = std::nextafter(cost(c), 0.0); // fewer threads where two are level
+                tpt  = c.tpt;
+            }
+        s.tpt = tpt;
+    }
+
     core_fft(size_t len, hipStream_t s)
     {
         n = len;
@@ -1026,6 +1060,7 @@ struct core_fft
         if (fits_lds(n))
         {
             make_stockham((long long)n, S, pmax_of<T>);
+            widen_direct(S);
             check_pass_radices<T>(S, is_mixed(S));
             tpb = pick_tpb(S);
             tw.reset((size_t)std::max<long long>(1, S.tw_count) * sizeof(cx<T>));

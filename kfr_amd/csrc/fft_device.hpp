@@ -793,15 +793,15 @@ __device__ __forceinline__ void with_radix(int r, F&& f)
     }
 }
 
-// passes [first, last) of the transform held in LDS
-template <typename T, bool INV, bool MIXED, bool PAD>
+// passes [first, last) of the transform held in LDS; GEN: direct passes among them (MIXED builds)
+template <typename T, bool INV, bool MIXED, bool GEN, bool PAD>
 __device__ __forceinline__ void fft_passes(const lds_geom& G, const cx<T>* tw, const fft_ctx<T, PAD>& c, int first,
                                            int last)
 {
     for (int p = first; p < last; ++p)
     {
         const pass_desc& P = G.pass[p];
-        if constexpr (MIXED)
+        if constexpr (MIXED && GEN)
         {
             if (P.kind == pass_generic)
             {
@@ -818,7 +818,7 @@ __device__ __forceinline__ void fft_passes(const lds_geom& G, const cx<T>* tw, c
 template <typename T, bool INV, bool MIXED, bool PAD>
 __device__ __forceinline__ void fft_passes(const lds_geom& G, const cx<T>* tw, const fft_ctx<T, PAD>& c)
 {
-    fft_passes<T, INV, MIXED>(G, tw, c, 0, G.np);
+    fft_passes<T, INV, MIXED, true>(G, tw, c, 0, G.np);
 }
 // pass 0 from src to LDS
 template <typename T, bool INV, bool MIXED, bool PAD, typename Src>

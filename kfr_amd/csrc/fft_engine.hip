@@ -585,7 +585,7 @@ __global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) 
         block_load<!MIXED>(G, lds, first, batch, ld, ndiv);
         __syncthreads();
     }
-    fft_passes<T, false, MIXED>(G, tw, c, FL ? 1 : 0, G.np);
+    fft_passes<T, false, MIXED, true>(G, tw, c, FL ? 1 : 0, G.np);
     if (!c.valid)
         return;
     const long long csize = G.n;
@@ -659,7 +659,7 @@ __global__ void __launch_bounds__(max_block_of(MIXED), (mixed_waves<T, MIXED>)) 
         }
     }
     __syncthreads();
-    fft_passes<T, true, MIXED>(G, tw, c, 0, FS ? G.np - 1 : G.np);
+    fft_passes<T, true, MIXED, true>(G, tw, c, 0, FS ? G.np - 1 : G.np);
     if constexpr (FS)
         last_pass<T, true, MIXED>(
             G, tw, c,

@@ -151,6 +151,17 @@ def test_emulated_axes(t, shape, strided, tmp_path):
         assert oracle.rel_rms(run(ref.astype(dt), real, 1, True, rt).reshape(real) / v.size, v) <= 2 * bound
 
 
+# lengths with direct passes, the only ones that the build with them runs: one or two primes after
+# butterflies or alone, a schedule that takes more threads than the least (1032 = 24 * 43 in f64: 172)
+@pytest.mark.parametrize("t,n", [("f32", 1032), ("f64", 1032), ("f32", 11), ("f64", 286), ("f32", 2431)])
+def test_emulated_direct_passes(t, n, tmp_path):
+    r = subprocess.run([str(emu_build.build("asan")), "schedule", t, str(n)], capture_output=True, text=True, timeout=900)
+    if (t, n) == ("f64", 1032):
+        assert "threads/transform=172" in r.stdout, r.stdout
+    e = _dft("asan", tmp_path, np.complex64 if t == "f32" else np.complex128, n, 5, n % 2 == 0, 65)
+    assert e <= (1e-6 if t == "f32" else 1e-14)
+
+
 # the streaming filter's time-domain kernel: taps around a run of eight and a lane's share, calls shorter and
 # longer than a workgroup's outputs and the history. One non-finite sample reaches the outputs of its own taps
 # and no others, which keep every bit
