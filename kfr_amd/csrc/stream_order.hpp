@@ -24,7 +24,7 @@ namespace kfr_amd
 // by then, at once.
 struct stream_order
 {
-    stream_order()                    = default;
+    stream_order() { (void)hipGetDevice(&device); }
     stream_order(const stream_order&) = delete;
     ~stream_order()
     {
@@ -74,11 +74,10 @@ private:
     hipStream_t last = nullptr; // stream of the last call
     bool used        = false;
     bool pending     = false; // the last call is not recorded in ev
-    int device       = 0;     // the current device of that call
+    int device       = 0;     // the plan's: its calls run with it current
 
     void unrecorded(hipStream_t s)
     {
-        hip_check(hipGetDevice(&device), "hipGetDevice");
         last = s;
         used = pending = true;
     }
