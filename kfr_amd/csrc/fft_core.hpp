@@ -941,6 +941,9 @@ template <typename T, bool INV, int ROLE, bool MIXED, bool FL, bool FS, bool GEN
 void launch_fft_as(const lds_geom& G, const cx<T>* tw, long long batch, const xload<T>& ld, const xstore<T>& st,
                    const fourstep_args<T>& fs, unsigned grid, unsigned block, size_t sh, hipStream_t s)
 {
+    // complex values in and out: batch items (columns or rows in the four-step roles) of G.n points
+    timing::span ts([] { return timing::kernel_name("k_fft", timing::type_name<T>(), INV, ROLE, MIXED, FL, FS, GEN); },
+                    2 * (long long)sizeof(cx<T>) * batch * G.n, s);
     allow_lds(k_fft<T, INV, ROLE, MIXED, FL, FS, GEN>, sh);
     hipLaunchKernelGGL((k_fft<T, INV, ROLE, MIXED, FL, FS, GEN>), dim3(grid), dim3(block), sh, s, G, tw, batch, ld, st, fs);
 }
@@ -953,9 +956,6 @@ void launch_fft(bool mixed, const lds_geom& G, const cx<T>* tw, long long batch,
                 const xstore<T>& st, const fourstep_args<T>& fs, unsigned grid, unsigned block, size_t sh,
                 hipStream_t s)
 {
-    // complex values in and out: batch items (columns or rows in the four-step roles) of G.n points
-    timing::span ts([mixed] { return timing::kernel_name("k_fft", timing::type_name<T>(), INV, ROLE, mixed); },
-                    2 * (long long)sizeof(cx<T>) * batch * G.n, s);
     bool gen = false; // whole transforms with a direct pass
     for (int p = 0; p < G.np; ++p)
         gen = gen || (ROLE == role_direct && G.pass[p].kind == pass_generic);

@@ -723,7 +723,8 @@ struct gpu_dft_real<T>::impl
             const dim3 grid(nblocks(batch, f.tpb)), block(f.S.tpt * f.tpb);
             const fastdiv nd = make_fastdiv((uint32_t)csize);
             const bool mx    = is_mixed(f.S);
-            timing::span ts([mx] { return timing::kernel_name("k_real_fwd", timing::type_name<T>(), mx); },
+            const bool fl    = mx && plain(ld) && G.tpt >= 16 && G.pass[0].kind == pass_radix;
+            timing::span ts([=] { return timing::kernel_name("k_real_fwd", timing::type_name<T>(), mx, fl); },
                             2 * (long long)sizeof(cx<T>) * batch * (long long)csize, s);
             auto go = [&](auto kernel)
             {
@@ -733,7 +734,7 @@ struct gpu_dft_real<T>::impl
             };
             if (!mx)
                 go(k_real_fwd<T, false, false>);
-            else if (plain(ld) && G.tpt >= 16 && G.pass[0].kind == pass_radix)
+            else if (fl)
                 go(k_real_fwd<T, true, true>);
             else
                 go(k_real_fwd<T, true, false>);
@@ -793,11 +794,12 @@ struct gpu_dft_real<T>::impl
                 hipLaunchKernelGGL(kernel, dim3(nblocks(batch, f.tpb)), dim3(f.S.tpt * f.tpb), sh, s, G,
                                    f.tw.template as<cx<T>>(), batch, src, st, make_fastdiv((uint32_t)csize));
             };
-            timing::span ts([mx] { return timing::kernel_name("k_real_inv", timing::type_name<T>(), mx); },
+            const bool fs    = mx && plain(st) && G.tpt >= 16 && G.np >= 2 && G.pass[G.np - 1].kind == pass_radix;
+            timing::span ts([=] { return timing::kernel_name("k_real_inv", timing::type_name<T>(), mx, fs); },
                             2 * (long long)sizeof(cx<T>) * batch * (long long)csize, s);
             if (!mx)
                 go(k_real_inv<T, false, false>);
-            else if (plain(st) && G.tpt >= 16 && G.np >= 2 && G.pass[G.np - 1].kind == pass_radix)
+            else if (fs)
                 go(k_real_inv<T, true, true>);
             else
                 go(k_real_inv<T, true, false>);

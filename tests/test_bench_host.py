@@ -3,6 +3,7 @@ algorithmic-byte and flop counts, and the kernel-name and traffic-table parsing 
 from __future__ import annotations
 
 import json
+import re
 import subprocess
 import sys
 from pathlib import Path
@@ -40,9 +41,24 @@ def test_algorithmic_bytes_and_flops():
 def test_kernel_names_match_the_timing_records():
     assert rs.kernel_key("void kfr_amd::p2::k_pow2<float, 8, false, 3, 0>(kfr_amd::p2::args<float>)") == \
         "k_pow2<float, 8, false, 3, 0>"
-    assert rs.kernel_key("void kfr_amd::(anonymous namespace)::k_fft<double, true, 2, false>(kfr_amd::lds_geom)") == \
-        "k_fft<double, true, 2, false>"
+    assert rs.kernel_key("void kfr_amd::(anonymous namespace)::k_fft<double, true, 2, true, true, false, false>(kfr_amd::lds_geom)") == \
+        "k_fft<double, true, 2, true, true, false, false>"
     assert rs.kernel_key("__amd_rocclr_copyBuffer") == "__amd_rocclr_copyBuffer"
+
+
+def test_timing_names_give_every_template_argument():
+    """the name of a timing record is the profiler's key of the kernel launched, so each gives as many
+    arguments as the kernel's template has parameters"""
+    src = "\n".join(p.read_text() for p in sorted((ROOT / "kfr_amd" / "csrc").iterdir())
+                    if p.suffix in (".hip", ".hpp"))
+    kernels = {m[2]: len(m[1].split(",")) for m in
+               re.finditer(r"template <([^<>]*)>\s*__global__(?:[^;{](?!template))*?\b(k_\w+)\(", src)}
+    names = re.findall(r'kernel_name\(([^;]*?)\); \}', src)
+    assert len(kernels) >= 25 and len(names) >= 20
+    for args in names:
+        for k in re.findall(r'"(k_\w+)"', args):
+            given = args.replace("type_name<T>()", "T").count(",")
+            assert kernels[k] == given, (k, args)
 
 
 def test_traffic_table_is_read_for_the_named_kernel(tmp_path):
