@@ -378,6 +378,27 @@ __device__ __forceinline__ void run_pass(regs<T, L, ROLE, PREC>& v, cx<T>* lds, 
                   "mirrored last pass: two butterflies");
 }
 
+// v[k] times w * prod of pw[b] over the bits b of k (the conjugate with INV), for the values k that share the bits
+// below B with K. Depth first from the lowest bit: the same products as building all E factors from the
+// lowest bit up, but one per bit is held instead of all. With all of them columns of 2^11 and more points spill:
+// f32 2^11 52 (forward) and 148 (inverse) bytes per lane, now none, f64 2^11 inverse 92, now 36 (f32 2^22 x 8
+// inverse 302 -> 257 us and forward 273 -> 256, bf16 2^20 x 64 543 -> 470 and 498 -> 470, one bf16 2^20 inverse 39.7 -> 32.4, f64
+// 2^21 x 16 inverse 521 -> 493).
+template <typename T, bool INV, int LEE, int B, int K, int E, int NB>
+__device__ __forceinline__ void column_twiddles(cx<T> (&v)[E], cx<T> w, const cx<T> (&pw)[NB])
+{
+    if constexpr (B == LEE)
+    {
+        v[K] = ctw<INV>(v[K], w);
+        settle(v[K]);
+    }
+    else
+    {
+        column_twiddles<T, INV, LEE, B + 1, K>(v, w, pw);
+        column_twiddles<T, INV, LEE, B + 1, K + (1 << B)>(v, cmul(w, pw[B]), pw);
+    }
+}
+
 template <typename T, int L, bool INV, int ROLE, int PREC>
 __global__ void __launch_bounds__((geom<T, L, ROLE, PREC>::BS),
                                   (ROLE == role_direct || ROLE == role_row ? geom<T, L, ROLE, PREC>::lds_waves : 1))
@@ -591,17 +612,24 @@ __global__ void __launch_bounds__((geom<T, L, ROLE, PREC>::BS),
 #pragma unroll
             for (int b = 0; b < LEE; ++b)
                 pw[b] = table(((unsigned long long)col * (unsigned long long)(TP << b)) & nm);
-            cx<T> w[E];
-            w[0] = table((unsigned long long)col * (unsigned long long)t);
-#pragma unroll
-            for (int k = 1; k < E; ++k)
+            const cx<T> w0 = table((unsigned long long)col * (unsigned long long)t);
+            if constexpr (sizeof(T) == 4 || INV)
+                column_twiddles<T, INV, LEE, 0, 0>(v, w0, pw);
+            else
             {
-                const int hb = ilog2c(k + 1) - 1; // top bit of k
-                w[k]         = cmul(w[k - (1 << hb)], pw[hb]);
-            }
+                // f64 forward spills 20 bytes per lane this way, 36 the other (2^21 x 16 476 and 491 us)
+                cx<T> w[E];
+                w[0] = w0;
 #pragma unroll
-            for (int k = 0; k < E; ++k)
-                v[k] = ctw<INV>(v[k], w[k]);
+                for (int k = 1; k < E; ++k)
+                {
+                    const int hb = ilog2c(k + 1) - 1; // top bit of k
+                    w[k]         = cmul(w[k - (1 << hb)], pw[hb]);
+                }
+#pragma unroll
+                for (int k = 0; k < E; ++k)
+                    v[k] = ctw<INV>(v[k], w[k]);
+            }
         }
         if (valid)
         {
