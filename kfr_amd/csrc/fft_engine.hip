@@ -706,6 +706,17 @@ struct gpu_dft_real<T>::impl
                l.pdist == dist;
     }
 
+    // The packing and unpacking of a transform in one thread is one thread's work with 16-byte accesses a
+    // transform apart: f64 halves of 9 to 15 points, one butterfly since composite radices, take two threads
+    // (the second idle in the pass)
+    static stockham packing_threads(const stockham& s)
+    {
+        stockham r = s;
+        if (sizeof(T) == 8 && s.n >= 9 && is_mixed(s))
+            r.tpt = std::max(r.tpt, 2);
+        return r;
+    }
+
     void forward_op(const xload<T>& ld, cx<T>* out, long long odist, long long batch, hipStream_t s)
     {
         if (batch <= 0)
@@ -718,9 +729,10 @@ struct gpu_dft_real<T>::impl
         if (fused_forward())
         {
             core_fft<T>& f  = *c->core;
-            lds_geom G      = make_geom(f.S, f.tpb, 0, 1, (int)csize);
-            const size_t sh = lds_padded_elems((size_t)f.tpb * csize) * sizeof(cx<T>);
-            const dim3 grid(nblocks(batch, f.tpb)), block(f.S.tpt * f.tpb);
+            const stockham S = packing_threads(f.S);
+            lds_geom G       = make_geom(S, f.tpb, 0, 1, (int)csize);
+            const size_t sh  = lds_padded_elems((size_t)f.tpb * csize) * sizeof(cx<T>);
+            const dim3 grid(nblocks(batch, f.tpb)), block(S.tpt * f.tpb);
             const fastdiv nd = make_fastdiv((uint32_t)csize);
             const bool mx    = is_mixed(f.S);
             const bool fl    = mx && plain(ld) && G.tpt >= 16 && G.pass[0].kind == pass_radix;
@@ -785,13 +797,14 @@ struct gpu_dft_real<T>::impl
         {
             // one workgroup per transform: the unpacking runs in the load phase of the same kernel
             core_fft<T>& f   = *c->core;
-            lds_geom G       = make_geom(f.S, f.tpb, 0, 1, (int)csize);
+            const stockham S = packing_threads(f.S);
+            lds_geom G       = make_geom(S, f.tpb, 0, 1, (int)csize);
             const size_t sh  = lds_padded_elems((size_t)f.tpb * csize) * sizeof(cx<T>);
             const bool mx    = is_mixed(f.S);
             auto go          = [&](auto kernel)
             {
                 allow_lds(kernel, sh);
-                hipLaunchKernelGGL(kernel, dim3(nblocks(batch, f.tpb)), dim3(f.S.tpt * f.tpb), sh, s, G,
+                hipLaunchKernelGGL(kernel, dim3(nblocks(batch, f.tpb)), dim3(S.tpt * f.tpb), sh, s, G,
                                    f.tw.template as<cx<T>>(), batch, src, st, make_fastdiv((uint32_t)csize));
             };
             const bool fs    = mx && plain(st) && G.tpt >= 16 && G.np >= 2 && G.pass[G.np - 1].kind == pass_radix;
