@@ -2133,6 +2133,7 @@ os_conv<T>::os_conv(size_t nx, size_t nh, hipStream_t s) : p(new impl)
     p->tw.reset((size_t)std::max(1, cnt) * sizeof(cx<T>));
     p2::gen_pass_tables<T>(L, p->tw.template as<cx<T>>(), s);
     p->fft.reset(new pow2_fft<T>((size_t)1 << L, s));
+    p->fft->reserve(); // spectra of a few filters
 }
 
 template <typename T>
@@ -2235,6 +2236,8 @@ void os_conv<T>::backward(T* dx, T* dh, const T* g, const T* x, const T* h, long
         const long long bs   = std::max<long long>(64, N >> p2::log_e<T>);
         const long long want = std::min<long long>(a.nseg, std::max<long long>(1, (1ll << 20) / bs / batch));
         a.per                = (int)((a.nseg + want - 1) / want);
+        if (const char* e = std::getenv("KFR_AMD_CONV_SEGMENTS")) // per workgroup
+            a.per = std::max(1, std::atoi(e));
         a.groups             = (a.nseg + a.per - 1) / a.per;
         a.count              = a.groups * batch;
         a.scale = T(1) / T(N);

@@ -9,6 +9,8 @@
 //   emu_main filter f32|f64|c32|c64 taps n,n,... taps.bin in.bin out.bin   (streaming filter, calls of n samples)
 //   emu_main md f32|f64 d0,d1,.. real inverse in.bin out.bin   (axes; its schedule on standard output)
 //   emu_main schedule f32|f64 n
+//   emu_main conv f32|f64 nx nh batch shared in.bin out.bin   (overlap-save: signals, taps and output gradients to
+//                                   outputs, signal gradients and tap gradients, one after the other)
 //   emu_main order calls out.txt   (stream_order's launches, event records and waits for calls like 0-,5s,0-:
 //                                   stream handle, then s with or - without scratch)
 // The input is copied into a buffer of exactly its size and the output buffer holds exactly the
@@ -209,6 +211,47 @@ static int filter_main(bool complex, char** argv)
 }
 
 template <typename T>
+static int conv_main(char** argv)
+{
+    const size_t nx = std::strtoull(argv[3], nullptr, 10), nh = std::strtoull(argv[4], nullptr, 10);
+    const long long batch = std::atoll(argv[5]);
+    const bool shared     = std::atoi(argv[6]) != 0;
+    const size_t xn = batch * nx, hn = (shared ? 1 : batch) * nh, yn = batch * (nx + nh - 1);
+    const std::vector<char> in = read_file(argv[7]);
+    if (in.size() != (xn + hn + yn) * sizeof(T))
+        return 2;
+    size_t pos = 0;
+    auto take  = [&](size_t n)
+    {
+        T* p = static_cast<T*>(std::malloc(n * sizeof(T)));
+        std::memcpy(p, in.data() + pos * sizeof(T), n * sizeof(T));
+        pos += n;
+        return p;
+    };
+    T *x = take(xn), *h = take(hn), *g = take(yn);
+    T* out[3]         = {};
+    const size_t n[3] = { yn, xn, hn };
+    for (int k = 0; k < 3; ++k)
+    {
+        out[k] = static_cast<T*>(std::malloc(n[k] * sizeof(T)));
+        std::memset(out[k], 0x7f, n[k] * sizeof(T));
+    }
+    os_conv<T> c(nx, nh, nullptr);
+    c.forward(out[0], x, h, shared ? 0 : (long long)nh, batch, false, nullptr);
+    c.backward(out[1], out[2], g, x, h, shared ? 0 : (long long)nh, batch, false, nullptr);
+    FILE* f = std::fopen(argv[8], "wb");
+    for (int k = 0; f && k < 3; ++k)
+        if (std::fwrite(out[k], sizeof(T), n[k], f) != n[k])
+            return 4;
+    if (!f)
+        return 4;
+    std::fclose(f);
+    for (T* p : { x, h, g, out[0], out[1], out[2] })
+        std::free(p);
+    return 0;
+}
+
+template <typename T>
 static int md_main(char** argv)
 {
     std::vector<size_t> shape;
@@ -296,6 +339,8 @@ int main(int argc, char** argv)
         return t == "f32" || t == "c32" ? filter_main<float>(t == "c32", argv) : filter_main<double>(t == "c64", argv);
     if (kind == "md" && argc == 8)
         return t == "f64" ? md_main<double>(argv) : md_main<float>(argv);
+    if (kind == "conv" && argc == 9)
+        return t == "f64" ? conv_main<double>(argv) : conv_main<float>(argv);
     if (kind == "schedule" && argc == 4)
     {
         const size_t n = std::strtoull(argv[3], nullptr, 10);

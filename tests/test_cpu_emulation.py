@@ -330,9 +330,57 @@ def test_emulated_half_storage(storage, n, batch, multi, tmp_path):
         assert e <= (2e-3 if storage == "bf16" else 5e-4)
 
 
+def _conv(variant, tmp_path, t, nx, nh, batch, shared, seed, env=None):
+    """relative errors of the overlap-save output and its two gradients"""
+    dt = np.float32 if t == "f32" else np.float64
+    rng = np.random.default_rng(seed)
+    ny = nx + nh - 1
+    x, g = (rng.standard_normal((batch, n)).astype(dt) for n in (nx, ny))
+    h = rng.standard_normal((1 if shared else batch, nh)).astype(dt)
+    out = _run(variant, tmp_path, ["conv", t, nx, nh, batch, int(shared)], np.concatenate([x.ravel(), h.ravel(), g.ravel()]), dt, env)
+    m = 1 << (ny + nh).bit_length()
+    X, H, Gf = (np.fft.rfft(v.astype(np.float64), m) for v in (x, h, g))
+    dh = np.fft.irfft(Gf * X.conj(), m)[:, :nh]
+    ref = [np.fft.irfft(X * H, m)[:, :ny], np.fft.irfft(Gf * H.conj(), m)[:, :nx], dh.sum(0) if shared else dh]
+    parts = np.split(out, [batch * ny, batch * (ny + nx)])
+    return [oracle.rel_rms(a, r.ravel()) for a, r in zip(parts, ref)]
+
+
+# the overlap-save convolution and its gradients over blocks of 256 points: one segment and four, the last
+# ragged, a shared filter; workgroups of the filter gradient with one, three and one, and all of the segments
+@pytest.mark.parametrize("t,nx,nh,batch,shared,per", [("f32", 700, 30, 2, False, 0), ("f32", 700, 30, 3, False, 3),
+                                                      ("f64", 700, 30, 2, True, 3), ("f64", 300, 80, 3, True, 9),
+                                                      ("f32", 90, 40, 2, False, 0)])
+def test_emulated_convolution(t, nx, nh, batch, shared, per, tmp_path):
+    env = {"KFR_AMD_CONV_SEGMENTS": str(per)} if per else None
+    for e in _conv("asan", tmp_path, t, nx, nh, batch, shared, 92, env):
+        assert e <= (1e-6 if t == "f32" else 1e-14)
+
+
 @pytest.mark.skipif(os.environ.get("KFR_AMD_EMU_TSAN") != "1", reason="set KFR_AMD_EMU_TSAN=1")
 @pytest.mark.parametrize("dtype,n,batch", [(np.complex64, 30240, 3), (np.complex64, 1 << 15, 1),
                                            (np.complex128, 13440, 2)])
 def test_emulated_no_races(dtype, n, batch, tmp_path):
     e = _dft("tsan", tmp_path, dtype, n, batch, False, 60)
     assert e <= (1e-6 if dtype == np.complex64 else 1e-14)
+
+
+# the one-workgroup kernel with its two-round exchange, the time-domain filter, the convolution kernels, a
+# real transform unpacked in LDS and an axis along its stride
+@pytest.mark.skipif(os.environ.get("KFR_AMD_EMU_TSAN") != "1", reason="set KFR_AMD_EMU_TSAN=1")
+def test_emulated_no_races_in_shared_memory(tmp_path):
+    x = oracle.complex_uniform(66, (1, 1 << 15), np.complex64)
+    y = _run("tsan", tmp_path, ["dft", "f32", 1 << 15, 1, 0], x, np.complex64, {"EMU_CAPTURING": "1"})
+    assert oracle.rel_rms(y, np.fft.fft(x.astype(np.complex128))[0]) <= 1e-6
+    v = oracle.gaussian(67, 600, np.float32)
+    h = oracle.gaussian(68, 130, np.float32)
+    h.tofile(tmp_path / "h.bin")
+    y = _run("tsan", tmp_path, ["filter", "f32", 130, "400,200", tmp_path / "h.bin"], v, np.float32)
+    assert oracle.rel_rms(y, np.convolve(v.astype(np.float64), h.astype(np.float64))[:600]) <= 2e-6
+    assert max(_conv("tsan", tmp_path, "f32", 700, 30, 2, False, 93, {"KFR_AMD_CONV_SEGMENTS": "3"})) <= 1e-6
+    v = oracle.gaussian(69, 3 * 180, np.float32).reshape(3, 180)
+    X = np.fft.rfft(v.astype(np.float64)).astype(np.complex64)
+    assert oracle.rel_rms(_run("tsan", tmp_path, ["real", "f32", 180, 1, 3, 1], X, np.float32) / 180, v.ravel()) <= 1e-6
+    x = oracle.complex_uniform(70, (45, 20), np.complex64)
+    y = _run("tsan", tmp_path, ["md", "f32", "45,20", 0, 0], x, np.complex64)
+    assert oracle.rel_rms(y, np.fft.fft2(x.astype(np.complex128)).ravel()) <= 1e-6

@@ -387,6 +387,37 @@ def test_conv_shared_filter_gradient_many_items():
     assert ey < 1e-6 and ex < 1e-6 and eh < 1e-5
 
 
+# batches so large that a workgroup of the filter gradient takes several of a signal's segments, the last one
+# fewer: three segments in two and one (f32, f64), 45 in seven of 6 and one of 3 (f64, a shared filter)
+@pytest.mark.parametrize("nx,nh,batch,dt,shared", [(2000, 200, 8192, "f32", False), (650, 30, 6000, "f64", False),
+                                                   (10000, 30, 2000, "f64", True)])
+def test_conv_gradients_of_many_signals(nx, nh, batch, dt, shared):
+    torch = pytest.importorskip("torch")
+    from kfr_amd.autograd import fft_convolve
+    t = torch.float32 if dt == "f32" else torch.float64
+    block = 1 << max(8, (3 * (nh - 1) - 1).bit_length())
+    segments = -(-nx // (block - nh + 1))
+    want = min(segments, max(1, (1 << 20) // max(64, block >> (4 if dt == "f32" else 3)) // batch))
+    per = -(-segments // want)
+    assert per > 1 and segments % per != 0
+    gen = torch.Generator(device="cuda").manual_seed(94)
+    x = torch.randn(batch, nx, dtype=t, device="cuda", generator=gen).requires_grad_()
+    h = torch.randn(*(() if shared else (batch,)), nh, dtype=t, device="cuda", generator=gen).requires_grad_()
+    g = torch.randn(batch, nx + nh - 1, dtype=t, device="cuda", generator=gen)
+    y = fft_convolve(x, h)
+    dx, dh = torch.autograd.grad(y, (x, h), g)
+    x, h, g = (v.detach().double() for v in (x, h, g))
+    m = 1 << (nx + 2 * nh).bit_length()
+    X, H, G = (torch.fft.rfft(v, m) for v in (x, h, g))
+    rdh = torch.fft.irfft(G * X.conj(), m)[..., :nh]
+    ref = (torch.fft.irfft(X * H, m)[..., :nx + nh - 1], torch.fft.irfft(G * H.conj(), m)[..., :nx],
+           rdh.sum(0) if shared else rdh)
+    for got, want_, serial in zip((y, dx, dh), ref, (1, 1, batch if shared else 1)):
+        e = float((got.detach().double() - want_).norm() / want_.norm())
+        # a sum over the batch in the data's precision grows its error by the square root of its length
+        assert e <= (1e-6 if dt == "f32" else 1e-14) * serial ** 0.5
+
+
 def test_conv_empty_batch():
     """no signals: nothing is written by the forward call, the adjoint of a shared filter is zero"""
     torch = pytest.importorskip("torch")
