@@ -129,7 +129,8 @@ __device__ __forceinline__ void run_item(const len_desc& D, const cx<T>* __restr
 }
 
 // at most 128 VGPRs (4 waves per SIMD), so two workgroups share a CU: measured faster than the
-// unconstrained build (185 VGPRs, one workgroup per CU) despite a little spilling
+// unconstrained build (185 VGPRs, one workgroup per CU). f32 needs 123; f64 spills 36 bytes per lane with its
+// butterflies of 12 to 15 points, and 12,000 f64 transforms of up to 4096 points still gain by them (225 -> 189 us)
 template <typename T>
 __global__ void __launch_bounds__(block) __attribute__((amdgpu_waves_per_eu(4))) k_batch(const len_desc* __restrict__ lens, const work_item* __restrict__ items,
                                                  int nitems, const int* __restrict__ members,
@@ -201,12 +202,12 @@ struct host_len
 };
 
 // LDS paddings: one slot per 16 or per 32 values, or none (the tile is sized for one per 16). Untuned
-// lengths with odd factors run without (an odd first radix spreads its writes), powers of two with one
-// per 16
+// lengths with odd factors run without (see lds_pad; tuning changes 338 to 336 us over 20,000 lengths), powers
+// of two with one per 16
 constexpr int padshifts[] = { 4, 5, 30 };
 
-// Pass orders tried for one length: the planner's (powers of two, largest first, then 7, 5, 3 and the
-// direct primes), its reverse, and the odd factors ahead of the powers of two. Every order of one
+// Pass orders tried for one length: the planner's (powers of two largest first; mixed lengths with their largest
+// odd radix first, the others by size and direct primes last), its reverse, and all odd radices ahead of the even ones. Every order of one
 // radix multiset has the same threads per transform and table size; each pass reads its own stride
 // and twiddles from the length's descriptor, so any order computes the same transform.
 inline std::vector<std::vector<int>> radix_orders(const std::vector<int>& r)
@@ -516,7 +517,7 @@ gpu_batch<T>::gpu_batch(size_t count, const size_t* sizes, const int* inverse, b
                                         " does not fit one workgroup of the batch kernel");
         h.orders = radix_orders(h.S.radix);
         if (is_mixed(h.S))
-            h.padshift = 30; // an odd first radix: its LDS writes spread over the banks by themselves
+            h.padshift = 30; // unpadded, as the other kernels' mixed lengths
         h.tpb_max = std::max(1, block / h.S.tpt);
         while (h.tpb_max > 1 && lds_of<T>(h.m, h.tpb_max) > lds_cap)
             --h.tpb_max;

@@ -49,9 +49,8 @@ enum ld_mode : int
     ld_real_pad = 1, // real pairs p[2e], p[2e+1] of a zero-padded (optionally reversed) real signal
     ld_dct2     = 2, // (x[mirror(e)], 0)
     ld_dct3     = 3, // x[e] * W_{4n}^e (x[0] halved)
-    ld_c2r      = 4, // from_fmt: packed half-length sequence from a CCs/Perm half spectrum
-    ld_cpad     = 5, // zero-padded (optionally reversed) complex signal
-    ld_mul      = 6  // p[b*pdist + e] * q[e] (flag: conj(q[e]))
+    ld_cpad     = 4, // zero-padded (optionally reversed) complex signal
+    ld_mul      = 5  // p[b*pdist + e] * q[e] (flag: conj(q[e]))
 };
 
 enum st_mode : int
@@ -72,20 +71,21 @@ template <typename T>
 struct xload
 {
     int mode      = ld_plain;
-    int flag      = 0; // real_pad/cpad: reversed; c2r: pack format (1 CCs, 0 Perm); mul: conjugate q
-    int src       = 0; // c2r spectrum source: 0 p, 1 p*q*scale, 2 p*conj(q)*scale
+    int flag      = 0; // real_pad/cpad: reversed; half spectra: pack format (1 CCs, 0 Perm); mul: conjugate q
+    int src       = 0; // half spectra (spec): 0 p, 1 p*q*scale, 2 p*conj(q)*scale
     int mconj     = 0; // conjugate the post-multiplier
     const void* p = nullptr;
     long long pdist  = 0;
     const cx<T>* q   = nullptr;
     long long qdist  = 0;
-    const cx<T>* r   = nullptr; // c2r twiddles
+    const cx<T>* r   = nullptr; // half spectra: from_fmt twiddles
     long long n      = 0;
     T scale          = T(1);
     long long b0     = 0;
     const cx<T>* mtab = nullptr; // post-multiplier table (Bluestein chirp)
     long long lim    = LLONG_MAX; // elements at or beyond lim are zero
 
+    // value k of half spectrum b (k_real_inv, k_real_unpack)
     __device__ cx<T> spec(long long b, long long k) const
     {
         const cx<T> a = static_cast<const cx<T>*>(p)[b * pdist + k];
@@ -119,34 +119,6 @@ struct xload
         {
             const T v = static_cast<const T*>(p)[b * n + e] * (e == 0 ? T(0.5) : T(1));
             return { v * q[e].re, v * q[e].im };
-        }
-        case ld_c2r:
-        {
-            // from_fmt (src/dft/fft-impl.hpp:1853-1896); n = half length
-            const long long cs = n;
-            if (e == 0)
-            {
-                const cx<T> x0 = spec(b, 0);
-                if (flag == 1)
-                {
-                    const cx<T> xn = spec(b, cs);
-                    return { x0.re + xn.re, x0.re - xn.re };
-                }
-                return { x0.re + x0.im, x0.re - x0.im };
-            }
-            if (2 * e == cs)
-            {
-                const cx<T> xm = spec(b, e);
-                return { T(2) * xm.re, T(-2) * xm.im };
-            }
-            const bool lo     = 2 * e < cs;
-            const long long k = lo ? e : cs - e;
-            const cx<T> xk    = spec(b, k);
-            const cx<T> xnk   = spec(b, cs - k);
-            const cx<T> f1    = cadd(xk, cconj(xnk));
-            const cx<T> f2    = csub(xk, cconj(xnk));
-            const cx<T> t     = cmulc(f2, r[k]);
-            return lo ? cadd(f1, t) : cconj(csub(f1, t));
         }
         case ld_cpad:
         {
@@ -436,7 +408,7 @@ inline int workgroup_threads(long long nn, int pm, bool wide)
 // Schedule of a length with odd factors: the product of butterfly radices (2..10, 12, 14, 15, 16) with
 // the least modelled work per point. A pass costs its butterfly's arithmetic, its twiddles and one
 // exchange through LDS, times the lanes that its butterflies leave idle at the schedule's thread count,
-// so few passes of large radices with equal thread counts win: 960 points run as 15 x 16 x 4 on 64
+// so few passes of large radices with equal thread counts win: 960 points run as 15 x 8 x 8 on 64
 // threads. The largest odd radix goes first (its strided LDS writes meet no bank twice), direct passes
 // of larger primes last.
 inline bool plan_mixed(long long nn, stockham& S, int pm, int max_threads)
@@ -746,8 +718,8 @@ __device__ __forceinline__ void block_store(const lds_geom& G, const cx<T>* lds,
     } while (!PAD && e0 < total);
 }
 
-// Waves per SIMD that the mixed-radix kernels are compiled for: f32 in 128 VGPRs without spills (155
-// unbounded, a wave fewer); f64 as many as it comes to
+// Waves per SIMD that the mixed-radix kernels are compiled for: f32 four, in 128 VGPRs and without spills (up to
+// 165 unbounded, a wave fewer); f64 as many as it comes to
 template <typename T, bool MIXED>
 inline constexpr int mixed_waves = MIXED && sizeof(T) == 4 ? 4 : 1;
 

@@ -438,9 +438,9 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, const fastdiv& f)
 // writes straight to HBM, so a transform of np passes crosses LDS np - 1 times; a load or store
 // phase with element operations stages through LDS instead. What bounded these kernels was instructions
 // and LDS trips: staging both ends and radices of at most 7 for odd factors, 960 points made five trips
-// and took 172 us for 16384 f32 transforms; as 15 x 16 x 4 with two trips they take 57 us (4.4 TB/s, a
-// copy of the same bytes 49 us). f64 30240 x 256 (four-step, 168 x 180) 229 -> 111 us, the uneven batch of
-// 20,000 transforms 429 -> 338 us.
+// and took 173 us for 16384 f32 transforms; as 15 x 8 x 8 with two trips they take 54 us (a copy of the same
+// bytes 49 us). f64 30240 x 256 (four-step, 168 x 180) 228 -> 114 us, the uneven batch of 20,000 transforms
+// 429 -> 338 us.
 
 constexpr int max_passes = 20;
 // Complex values a thread holds per pass: about 16 complex f32 or 8 complex f64 (bflies). Kernels come
@@ -500,9 +500,10 @@ inline constexpr int bflies_of = bflies(R, pmax_of<T>);
 
 // Padded LDS layout (PAD): logical element x lives at x + (x >> padshift), one padding slot per 16
 // (or 32) elements, so that the power-of-two strides of the Stockham passes spread over the banks
-// instead of hitting one. Schedules with an odd factor start with an odd radix where they can, so the
-// strided writes of their first pass spread by themselves and the layout stays linear: one addition
-// per address instead of three operations.
+// instead of hitting one. Mixed schedules run unpadded, one addition per address instead of three
+// operations: most start with an odd radix, whose strided writes spread by themselves, and those of even radices
+// only (a quarter of the 7-smooth lengths, 192 = 16 * 12, 768 = 16 * 8 * 6) gain as much from the other changes of
+// these kernels (768 x 10922 f32 81 -> 31 us, f64 960 = 12 * 10 * 8 x 8738 76 -> 46); padded they were not measured.
 template <bool PAD>
 __device__ __forceinline__ int lds_pad(int x, int s)
 {

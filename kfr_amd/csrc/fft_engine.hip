@@ -789,13 +789,12 @@ struct gpu_dft_real<T>::impl
             h->real(true, static_cast<const cx<T>*>(src.p) + src.b0 * src.pdist, src.pdist,
                     static_cast<cx<T>*>(st.p) + st.b0 * (long long)csize, (long long)csize, rtw.ptr, fmt, batch, s))
             return;
-        src.mode = ld_c2r;
         src.r    = rtw.as<cx<T>>();
         src.n    = (long long)csize;
         src.flag = fmt;
         if (fused_forward())
         {
-            // one workgroup per transform: the unpacking runs in the load phase of the same kernel
+            // one workgroup per transform: the unpacking is the load phase of a kernel of its own
             core_fft<T>& f   = *c->core;
             const stockham S = packing_threads(f.S);
             lds_geom G       = make_geom(S, f.tpb, 0, 1, (int)csize);
@@ -929,7 +928,6 @@ void gpu_dft_real<T>::progressive_unit(int u, void* z, void* c, void* mid, bool 
     {
         // from_fmt unpacking (src/dft/fft-impl.hpp:1853-1896) into the half-length sequence
         xload<T> src = load_plain<T>(c, (long long)p->complex_size());
-        src.mode     = ld_c2r;
         src.r        = p->rtw.template as<cx<T>>();
         src.n        = cs;
         src.flag     = p->fmt;

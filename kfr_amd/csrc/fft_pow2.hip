@@ -1374,9 +1374,9 @@ bool rfft_any(int L, const cx<T>* in, long long idist, cx<T>* out, long long odi
 // sequence (f is real, so both convolutions come out separated), runs the forward transform, the
 // product with the filter spectrum, and the inverse transform in registers and LDS, and writes
 // the valid outputs: every signal value is read (N / lv) times and every output written once. Compiled for
-// the two workgroups per CU that its LDS allows (128 VGPRs; 240 without the bound), with 32-bit bounds and
-// the filter spectrum in groups, so that few values are held beside the transform: 2^20 x 128 with 4095 taps
-// 553 -> 500 us per call. The arithmetic of its two transforms alone is about 350 us.
+// the two workgroups per CU that its LDS allows (128 VGPRs, of which f32 2^13 and 2^14 spill 28 and 44 bytes per
+// lane and f64 from 2^10 20; 240 without the bound), with 32-bit bounds and the filter spectrum in groups, so
+// that few values are held beside the transform: 2^20 x 128 with 4095 taps 553 -> 500 us per call. The arithmetic of its two transforms alone is about 350 us.
 template <typename T>
 struct conv_os_args
 {

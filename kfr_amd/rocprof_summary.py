@@ -103,30 +103,6 @@ def read_traffic(path: str, key: str) -> float | None:
     return None
 
 
-def read_table(path: str) -> list[dict]:
-    """rows of the first table written by `table` in a markdown file (column name -> cell text, the
-    kernel key under 'kernel'), or [] when the file is absent"""
-    rows: list[dict] = []
-    head: list[str] | None = None
-    try:
-        with open(path) as fh:
-            for line in fh:
-                if not line.startswith("|"):
-                    if head is not None and rows:
-                        break
-                    continue
-                cells = [c.strip() for c in line.strip().strip("|").split("|")]
-                if head is None:
-                    head = cells
-                elif not set(cells[0]) <= set("-:"):
-                    row = dict(zip(head, cells))
-                    row["kernel"] = row.get("kernel", "").strip("`")
-                    rows.append(row)
-    except OSError:
-        return []
-    return rows
-
-
 def trace(db: str, top: int) -> str:
     c = sqlite3.connect(db)
     rows = c.execute("select name, total_calls, total_duration, average, percentage from top_kernels "

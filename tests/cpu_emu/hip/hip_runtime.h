@@ -6,10 +6,8 @@
 // threads that meet at __syncthreads (and at the LDS barrier builtin) on one std::barrier, and a
 // thread that returns drops out of the barrier, as an ended wave does on the GPU. The dynamic LDS of a
 // workgroup is one heap block of exactly the launch's byte count. Device memory is host memory.
-// Wave-level operations (__shfl_xor, v_permlane32_swap, the 32x32x16 bf16 MFMA) exchange operands
-// through a per-wave buffer between two wave barriers; the MFMA follows the lane layout of
-// v_mfma_f32_32x32x16_bf16 (lane l, slot s: A[l%32][8(l/32)+s], B[8(l/32)+s][l%32]; result slot v:
-// D[8(v/4)+4(l/32)+v%4][l%32]) with the products summed in FP32.
+// Wave-level operations (__shfl_xor) exchange operands through a per-wave buffer between two wave
+// barriers.
 #pragma once
 
 #include <algorithm>
@@ -83,9 +81,6 @@ EMU_SMEM_IN(kfr_amd::bt)
 #define __builtin_amdgcn_s_barrier() ::emu::sync()
 #define __builtin_amdgcn_fence(...) ((void)0)
 #define __builtin_amdgcn_sched_barrier(...) ((void)0)
-typedef unsigned emu_u32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 emu_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float emu_f32x16 __attribute__((ext_vector_type(16)));
 
 namespace emu
 {
@@ -111,81 +106,13 @@ V wave_read(const V& mine, int src)
     cur_wave->bar.arrive_and_wait();
     return r;
 }
-
-inline emu_u32x2 permlane32_swap(unsigned v0, unsigned v1)
-{
-    const int l = lane();
-    struct pair
-    {
-        unsigned a, b;
-    };
-    const pair other = wave_read(pair{ v0, v1 }, l ^ 32);
-    emu_u32x2 r;
-    r[0] = l >= 32 ? other.b : v0; // the upper half of v0 takes the lower half of v1
-    r[1] = l < 32 ? other.a : v1;  // the lower half of v1 takes the upper half of v0
-    return r;
-}
-
-inline emu_f32x16 mfma_32x32x16_bf16(emu_bf16x8 a, emu_bf16x8 b, emu_f32x16 c)
-{
-    struct ops
-    {
-        float a[8], b[8];
-    };
-    ops mine;
-    for (int s = 0; s < 8; ++s)
-    {
-        mine.a[s] = (float)a[s];
-        mine.b[s] = (float)b[s];
-    }
-    std::memcpy(cur_wave->slot[lane()], &mine, sizeof(ops));
-    cur_wave->bar.arrive_and_wait();
-    float A[32][16], B[16][32];
-    for (int l = 0; l < 64; ++l)
-    {
-        ops o;
-        std::memcpy(&o, cur_wave->slot[l], sizeof(ops));
-        for (int s = 0; s < 8; ++s)
-        {
-            A[l % 32][8 * (l / 32) + s] = o.a[s];
-            B[8 * (l / 32) + s][l % 32] = o.b[s];
-        }
-    }
-    cur_wave->bar.arrive_and_wait();
-    const int l = lane();
-    emu_f32x16 d;
-    for (int v = 0; v < 16; ++v)
-    {
-        const int i = 8 * (v / 4) + 4 * (l / 32) + v % 4, j = l % 32;
-        float acc   = c[v];
-        for (int k = 0; k < 16; ++k)
-            acc += A[i][k] * B[k][j];
-        d[v] = acc;
-    }
-    return d;
-}
 } // namespace emu
-
-#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B, C, ...) ::emu::mfma_32x32x16_bf16(A, B, C)
-#define __builtin_amdgcn_permlane32_swap(V0, V1, ...) ::emu::permlane32_swap(V0, V1)
 
 inline int __lane_id() { return emu::lane(); }
 template <typename V>
 inline V __shfl_xor(V v, int mask)
 {
     return emu::wave_read(v, emu::lane() ^ mask);
-}
-inline unsigned __float_as_uint(float f)
-{
-    unsigned u;
-    std::memcpy(&u, &f, 4);
-    return u;
-}
-inline float __uint_as_float(unsigned u)
-{
-    float f;
-    std::memcpy(&f, &u, 4);
-    return f;
 }
 inline uint32_t __umulhi(uint32_t a, uint32_t b) { return (uint32_t)(((uint64_t)a * b) >> 32); }
 inline void sincospi(double x, double* s, double* c)

@@ -5,7 +5,8 @@ global access outside its buffer aborts the run; the spectra are checked against
 
 Cases: the generic four-step over factors 3, 5, 7 with workgroups that straddle batch items
 (f32 at 16 points per thread), the power-of-two four-step, the mixed-radix menu lengths, Bluestein, a
-real transform, a DCT, the one-kernel DCT-II/III and R2C/C2R, the R2C repack pass; half-precision storage on emulated MFMA; and the f64
+real transform, a DCT, the one-kernel DCT-II/III and R2C/C2R, the R2C repack pass; half-precision storage; the
+streaming filter, the convolution and its gradients, axes of multidimensional arrays; and the f64
 generic kernels built at 16 points per thread (the geometry an earlier build ran on the GPU, where
 lengths with radix-5 passes came out wrong) on those lengths.
 Set KFR_AMD_EMU_TSAN=1 to also run a ThreadSanitizer build (a missing barrier shows as a race), and
@@ -305,9 +306,8 @@ def _from_half(h: np.ndarray, storage: str) -> np.ndarray:
     return f[..., 0] + 1j * f[..., 1]
 
 
-# half-precision storage with the radix-16 passes on (emulated) MFMA: one workgroup (2^10), the
-# four-step (2^15) and the multi-pass kernels with their scaled binary16 intermediates (2^15 and 2^16,
-# selected through KFR_AMD_HALF_MULTIPASS_MIN_LOG)
+# half-precision storage: one workgroup (2^10), the two-kernel form of few transforms (2^15) and the multi-pass
+# kernels with their f32 intermediates (2^15 and 2^16, selected through KFR_AMD_HALF_MULTIPASS_MIN_LOG)
 @pytest.mark.parametrize("storage,n,batch,multi", [("bf16", 1 << 10, 3, False), ("bf16", 1 << 15, 2, False),
                                                    ("bf16", 1 << 15, 2, True), ("f16", 1 << 16, 1, True)])
 def test_emulated_half_storage(storage, n, batch, multi, tmp_path):

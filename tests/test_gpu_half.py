@@ -1,5 +1,5 @@
-"""Half-precision storage (kfr_amd_dft_half_*): bfloat16 and binary16 complex data, FP32 arithmetic,
-radix-16 passes on MFMA. Errors are measured against the FP64 transform of the stored (already
+"""Half-precision storage (kfr_amd_dft_half_*): bfloat16 and binary16 complex data, FP32 arithmetic
+and intermediates. Errors are measured against the FP64 transform of the stored (already
 rounded) input, so they cover the computation and the rounding of the output (gpu)."""
 from __future__ import annotations
 
@@ -57,8 +57,7 @@ def test_half_config_2p20_batch64(storage):
 
 
 def test_half_intermediate_scaling_keeps_precision_across_ranges():
-    """bfloat16 data far outside binary16's range: the per-group scale of the binary16 intermediate
-    keeps the relative error unchanged"""
+    """bfloat16 data far outside binary16's range: the intermediate keeps the relative error unchanged"""
     for scale in (1e-30, 1e30):
         rel, mx, _, _ = _run("bf16", 1 << 16, 4, False, scale=scale, seed=5)
         print(f"scale={scale:g} rel_rms={rel:.3e}", flush=True)
