@@ -225,6 +225,14 @@ struct gpu_dft<T>::impl
         hip_check(hipStreamSynchronize(s), "plan initialisation");
     }
 
+    // the intermediate of a few power-of-two transforms (pow2_fft::reserve), for plans that run them plainly: complex
+    // plans, Bluestein lengths, convolutions and filters; real and DCT plans have one-kernel forms
+    void reserve()
+    {
+        if (core && core->pow2)
+            core->pow2->reserve();
+    }
+
     void init_bluestein(hipStream_t s)
     {
         M                = next_pow2(2 * n - 1);
@@ -257,6 +265,7 @@ struct gpu_dft<T>::impl
             if (const char* e = std::getenv("KFR_AMD_BLUESTEIN_CHUNK_MB"))
                 cap = (size_t)std::max(1, atoi(e)) << 20;
             bs_chunk = (long long)std::max<size_t>(1, cap / (M * sizeof(cx<T>)));
+            reserve();
         }
         hip_check(hipStreamSynchronize(s), "bluestein initialisation");
     }
@@ -382,8 +391,7 @@ struct gpu_dft<T>::impl
 template <typename T>
 gpu_dft<T>::gpu_dft(size_t n) : p(new impl(n))
 {
-    if (p->core && p->core->pow2)
-        p->core->pow2->reserve();
+    p->reserve();
 }
 template <typename T>
 gpu_dft<T>::~gpu_dft() = default;
@@ -1275,6 +1283,7 @@ struct gpu_conv<T>::impl
         }
         else
             r.reset(new typename gpu_dft_real<T>::impl(S, 1));
+            r->c->reserve();
     }
     long long cs() const { return (long long)(S / 2 + 1); }
 };
@@ -1699,6 +1708,7 @@ struct gpu_conv_filter<T>::impl
         S     = std::max<size_t>(next_pow2(std::max<size_t>(2 * block, 2 * nh1 + 2)), 2);
         L     = S - nh1;
         r.reset(new typename gpu_dft_real<T>::impl(S, 1));
+        r->c->reserve();
         hipStream_t s = library_stream();
         taps_dev.reset(nt * sizeof(T));
         hip_check(hipMemcpy(taps_dev.ptr, taps, nt * sizeof(T), hipMemcpyHostToDevice), "filter taps upload");
@@ -1781,6 +1791,7 @@ struct gpu_conv_filter_complex<T>::impl
         S     = std::max<size_t>(next_pow2(std::max<size_t>(2 * block, 2 * nh1 + 2)), 2);
         L     = S - nh1;
         f.reset(new typename gpu_dft<T>::impl(S));
+        f->reserve();
         hipStream_t s = library_stream();
         taps_dev.reset(nt * sizeof(cx<T>));
         hip_check(hipMemcpy(taps_dev.ptr, taps, nt * sizeof(cx<T>), hipMemcpyHostToDevice), "filter taps upload");
