@@ -1282,8 +1282,10 @@ struct gpu_conv<T>::impl
             hip_check(hipStreamSynchronize(s), "convolution plan initialisation");
         }
         else
+        {
             r.reset(new typename gpu_dft_real<T>::impl(S, 1));
             r->c->reserve();
+        }
     }
     long long cs() const { return (long long)(S / 2 + 1); }
 };

@@ -9,7 +9,7 @@
 //   emu_main filter f32|f64|c32|c64 taps n,n,... taps.bin in.bin out.bin   (streaming filter, calls of n samples)
 //   emu_main md f32|f64 d0,d1,.. real inverse in.bin out.bin   (axes; its schedule on standard output)
 //   emu_main schedule f32|f64 n
-//   emu_main conv f32|f64 nx nh batch shared in.bin out.bin   (overlap-save: signals, taps and output gradients to
+//   emu_main conv f32|f64 nx nh batch shared in.bin out.bin   (signals, taps and output gradients to
 //                                   outputs, signal gradients and tap gradients, one after the other)
 //   emu_main order calls out.txt   (stream_order's launches, event records and waits for calls like 0-,5s,0-:
 //                                   stream handle, then s with or - without scratch)
@@ -236,7 +236,7 @@ static int conv_main(char** argv)
         out[k] = static_cast<T*>(std::malloc(n[k] * sizeof(T)));
         std::memset(out[k], 0x7f, n[k] * sizeof(T));
     }
-    os_conv<T> c(nx, nh, nullptr);
+    gpu_conv<T> c(nx, nh);
     c.forward(out[0], x, h, shared ? 0 : (long long)nh, batch, false, nullptr);
     c.backward(out[1], out[2], g, x, h, shared ? 0 : (long long)nh, batch, false, nullptr);
     FILE* f = std::fopen(argv[8], "wb");

@@ -331,7 +331,7 @@ def test_emulated_half_storage(storage, n, batch, multi, tmp_path):
 
 
 def _conv(variant, tmp_path, t, nx, nh, batch, shared, seed, env=None):
-    """relative errors of the overlap-save output and its two gradients"""
+    """relative errors of a convolution plan's output and its two gradients"""
     dt = np.float32 if t == "f32" else np.float64
     rng = np.random.default_rng(seed)
     ny = nx + nh - 1
@@ -346,11 +346,12 @@ def _conv(variant, tmp_path, t, nx, nh, batch, shared, seed, env=None):
     return [oracle.rel_rms(a, r.ravel()) for a, r in zip(parts, ref)]
 
 
-# the overlap-save convolution and its gradients over blocks of 256 points: one segment and four, the last
-# ragged, a shared filter; workgroups of the filter gradient with one, three and one, and all of the segments
+# the convolution and its gradients, overlap-save over blocks of 256 points: one segment and four, the last
+# ragged, a shared filter; workgroups of the filter gradient with one, three and one, and all of the segments;
+# a filter as long as the signal, through full-length transforms
 @pytest.mark.parametrize("t,nx,nh,batch,shared,per", [("f32", 700, 30, 2, False, 0), ("f32", 700, 30, 3, False, 3),
                                                       ("f64", 700, 30, 2, True, 3), ("f64", 300, 80, 3, True, 9),
-                                                      ("f32", 90, 40, 2, False, 0)])
+                                                      ("f32", 90, 40, 2, False, 0), ("f32", 200, 200, 2, True, 0)])
 def test_emulated_convolution(t, nx, nh, batch, shared, per, tmp_path):
     env = {"KFR_AMD_CONV_SEGMENTS": str(per)} if per else None
     for e in _conv("asan", tmp_path, t, nx, nh, batch, shared, 92, env):
